@@ -107,6 +107,10 @@ template <typename T>
 struct TileTraits;
 template <>
 struct TileTraits<float> {
+    typedef float P __attribute__((ext_vector_type(2)));
+    // keeps x in an even-aligned register pair -- x.x in an even VGPR, x.y in
+    // the odd one above it (no instruction); see tile_sweep's cell
+    __device__ static __forceinline__ void pin(P& x) { asm("" : "+v"(x)); }
     using V = float4;  // one ds_read_b128 = 4 rows
     static constexpr int K = 4;
     __device__ static V pack(const float* v) { return make_float4(v[0], v[1], v[2], v[3]); }
@@ -121,6 +125,8 @@ struct TileTraits<float> {
 };
 template <>
 struct TileTraits<double> {
+    typedef double P __attribute__((ext_vector_type(2)));
+    __device__ static __forceinline__ void pin(P&) {}
     using V = double2;  // one ds_read_b128 = 2 rows
     static constexpr int K = 2;
     __device__ static V pack(const double* v) { return make_double2(v[0], v[1]); }
@@ -132,10 +138,12 @@ struct TileTraits<double> {
     __device__ static double shr(double x) { return shr1d(x); }
 };
 
-// Shape of a lane's emission table in LDS: per letter, NV vectors of K rows
-// (the last may hold fewer), tab[(letter*NV + q)*64 + lane] -- one ds_read
-// of 16 bytes per vector, conflict-free because consecutive lanes read
-// consecutive 16-byte words.  A last vector holding a single row would be
+// Shape of a lane's emission table in LDS: NV vectors of K rows (the last
+// may hold fewer), each for the 4 letters, tab[(q*4 + letter)*64 + lane] --
+// one ds_read of 16 bytes per vector, conflict-free because consecutive
+// lanes read consecutive 16-byte words; a letter's entry is 64 words on, so
+// its address is a shift of the letter whatever NV (a multiply by NV*64
+// never issues beside another wave's instruction).  A last vector holding a single row would be
 // read as one 4-byte word at a 16-byte lane stride, four lanes to a bank,
 // so such a row (kTail) sits in a table of scalars instead,
 // stab[letter*64 + lane], at a 4-byte lane stride.
@@ -158,7 +166,8 @@ struct TabShape {
 // SAFE: c4) instead of the lane's eps.
 template <typename T, int NR, bool ROWEPS>
 struct TileRead {
-    T c0[NR], c1[NR], c2[NR], c3[NR];  // FAST: b d e eps_r; SAFE: alpha w delta' e
+    typename TileTraits<T>::P c10[NR];  // (c1, c0)
+    typename TileTraits<T>::P c32[NR];  // (c3, c2); FAST: b d e eps_r are c0 .. c3, SAFE: alpha w delta' e
     T c4[ROWEPS ? NR : 1];             // SAFE with ROWEPS: eps_r
     T eps, beta;
     int L;
@@ -172,7 +181,7 @@ __device__ __forceinline__ T d_eps(const TileRead<T, NR, ROWEPS>& R, int j)
     if constexpr (!ROWEPS)
         return R.eps;
     else if constexpr (FAST)
-        return R.c3[j];
+        return R.c32[j].x;
     else
         return R.c4[j];
 }
@@ -264,21 +273,21 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
                 lx[j] = qdiv(pb, (T)3);
                 if (FAST) {
                     if (ri == 0) {
-                        R.c0[j] = 0;
-                        R.c1[j] = qdiv(br, alpha);
-                        R.c2[j] = 0;
+                        R.c10[j].y = 0;
+                        R.c10[j].x = qdiv(br, alpha);
+                        R.c32[j].y = 0;
                     } else {
-                        R.c0[j] = qdiv(br * pdelta, palpha * alpha);
-                        R.c1[j] = qdiv(br * psigma, alpha);
-                        R.c2[j] = qdiv(er * pdelta, delta * palpha);
+                        R.c10[j].y = qdiv(br * pdelta, palpha * alpha);
+                        R.c10[j].x = qdiv(br * psigma, alpha);
+                        R.c32[j].y = qdiv(er * pdelta, delta * palpha);
                     }
-                    R.c3[j] = ROWEPS ? er : (T)0;
+                    R.c32[j].x = ROWEPS ? er : (T)0;
                 } else {
-                    R.c0[j] = alpha;
-                    R.c1[j] = ri == 0 ? br : br * psigma;
-                    R.c2[j] = bn * delta;
+                    R.c10[j].y = alpha;
+                    R.c10[j].x = ri == 0 ? br : br * psigma;
+                    R.c32[j].y = bn * delta;
                     // equal betas keep eps exactly (no rounding of bn / br)
-                    R.c3[j] = bn == br ? er : qdiv(er * bn, br);
+                    R.c32[j].x = bn == br ? er : qdiv(er * bn, br);
                     if constexpr (ROWEPS)
                         R.c4[j] = er;
                 }
@@ -291,15 +300,15 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
                 lx[j] = 0;
                 const bool firstoob = (ri == L);
                 if (FAST) {
-                    R.c0[j] = 0;
-                    R.c1[j] = 0;
-                    R.c2[j] = firstoob ? qdiv(pdelta, palpha) : (T)1;
-                    R.c3[j] = 0;
+                    R.c10[j].y = 0;
+                    R.c10[j].x = 0;
+                    R.c32[j].y = firstoob ? qdiv(pdelta, palpha) : (T)1;
+                    R.c32[j].x = 0;
                 } else {
-                    R.c0[j] = 0;
-                    R.c1[j] = 0;
-                    R.c2[j] = firstoob ? beta : (T)0;
-                    R.c3[j] = 1;
+                    R.c10[j].y = 0;
+                    R.c10[j].x = 0;
+                    R.c32[j].y = firstoob ? beta : (T)0;
+                    R.c32[j].x = 1;
                     if constexpr (ROWEPS)
                         R.c4[j] = 0;
                 }
@@ -326,7 +335,7 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
                         v[k] = 0;  // past the lane's rows: never used
                     }
                 }
-                tab[(l * NV + q) * 64 + lane] = TT::pack(v);
+                tab[(q * 4 + l) * 64 + lane] = TT::pack(v);
             }
             if constexpr (Shape::kTail) {
                 constexpr int j = NR - 1;
@@ -334,8 +343,12 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
                 reinterpret_cast<T*>(tab + Shape::kVecs)[l * 64 + lane] = m ? lm[j] : lx[j];
             }
         }
+#pragma unroll
+        for (int j = 0; j < NR; ++j) {
+            TT::pin(R.c10[j]);
+            TT::pin(R.c32[j]);
+        }
     }
-
 }
 
 // One sweep of this group's read (R) against a hap of length HL at hoff;
@@ -394,12 +407,10 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
     };
 
     // ---- wavefront sweep -------------------------------------------------
-    T M[NR], D[NR];
+    typename TT::P MD[NR];
 #pragma unroll
-    for (int j = 0; j < NR; ++j) {
-        M[j] = 0;
-        D[j] = 0;
-    }
+    for (int j = 0; j < NR; ++j)
+        MD[j] = (T)0;
     T C0 = 0;
     if (active && HL > 0) {
         if (F32)
@@ -512,7 +523,9 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
     // M and D of the row above reach a lane two steps after they were
     // computed (diagonal dependency), I one step after: step u reads ring
     // entry u % 2 and refills it, so the unrolled steps need no copies
-    T Mr[2] = {(T)0, (T)0}, Dr[2] = {c0f, c0f};
+    typename TT::P MDr[2];
+    MDr[0].x = MDr[1].x = (T)0;
+    MDr[0].y = MDr[1].y = c0f;
     T Iin = 0;
     T acc = 0;
 
@@ -536,7 +549,7 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
     // unconditionally, the rest compare.
     const int acc_last = t + HL;
     const int n_free = wave_min(active ? HL : nsteps) + 1;  // steps s < n_free
-    const int lane_off = lane;  // tab index of this lane's letter-0 entry
+    const uint32_t lane_off = lane;  // tab index of this lane's letter-0 entry
 
     // emission values of step 0; each step loads the next step's values
     // before it computes
@@ -547,12 +560,12 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
     T lamS[2] = {(T)0, (T)0};  // the scalar-table row (Shape::kTail)
     uint32_t letters = __builtin_amdgcn_alignbyte(whi, wlo, shift);
     {
-        const V* trow = tab + __umul24(letters & 3u, NV * 64) + lane_off;
+        const V* trow = tab + (((letters & 3u) << 6) | lane_off);
 #pragma unroll
         for (int qq = 0; qq < NV; ++qq)
-            lam[0][qq] = trow[qq * 64];
+            lam[0][qq] = trow[qq * 256];
         if constexpr (Shape::kTail)
-            lamS[0] = stab[__umul24(letters & 3u, 64)];
+            lamS[0] = stab[(letters & 3u) << 6];
     }
 
     // GE: every lane's eps is kEpsGpu, held in a scalar register (opaque to
@@ -573,31 +586,47 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
             // reads as base 0 there, and padding columns are never accumulated
             const uint32_t nletter = u < 3 ? (letters >> (8 * (u + 1))) & 3u : next & 3u;
             {
-                const V* trow = tab + __umul24(nletter, NV * 64) + lane_off;
+                const V* trow = tab + ((nletter << 6) | lane_off);
 #pragma unroll
                 for (int qq = 0; qq < NV; ++qq)
-                    lam[nxt][qq] = trow[qq * 64];
+                    lam[nxt][qq] = trow[qq * 256];
                 if constexpr (Shape::kTail)
-                    lamS[nxt] = stab[__umul24(nletter, 64)];
+                    lamS[nxt] = stab[nletter << 6];
             }
-            T mp = Mr[cur], dp = Dr[cur], chain = Iin;
-            // the cell of row j with emission value lvk
+            typename TT::P up = MDr[cur];  // the row above's (M, D), one column back
+            T chain = Iin;
+            // the cell of row j with emission value lvk.  A SIMD issues a
+            // VALU instruction of one wave and, beside it, one of another
+            // wave -- but beside it only an instruction whose three vector
+            // sources do not all sit in registers of one parity (measured
+            // with two waves: 2.03 cycles per FMA with mixed parities, 4.2
+            // with one; a quarter of freely allocated FMAs has one).  So M
+            // and D of a row are a register pair, M even and D odd, and so
+            // are its coefficients (c1, c0) and (c3, c2): with chain in M's
+            // old register every FMA mixes parities.  150-base reads
+            // against 150-350-base haps: 2.69 -> 2.58 cycles per VALU
+            // instruction over the 19-row kernel, 1-2% of the call (the
+            // clock gives some of it back).  The last row's pair is only
+            // read by the transfer below, and pinning it cost a move.
             auto cell = [&](int j, T lvk) {
-                const T mo = M[j], dov = D[j];
+                const typename TT::P old = MD[j];
                 T t1;
                 if (FAST) {
-                    t1 = fma(R.c1[j], dp, mp);
-                    t1 = fma(R.c0[j], chain, t1);
-                    chain = fma(R.c2[j], chain, mp);
+                    t1 = fma(R.c10[j].x, up.y, up.x);
+                    t1 = fma(R.c10[j].y, chain, t1);
+                    chain = fma(R.c32[j].y, chain, up.x);
                 } else {
-                    t1 = fma(R.c1[j], dp, chain);
-                    t1 = fma(R.c0[j], mp, t1);
-                    chain = fma(R.c2[j], mp, R.c3[j] * chain);
+                    t1 = fma(R.c10[j].x, up.y, chain);
+                    t1 = fma(R.c10[j].y, up.x, t1);
+                    chain = fma(R.c32[j].y, up.x, R.c32[j].x * chain);
                 }
-                M[j] = lvk * t1;
-                D[j] = fma(GE ? eps_ge : d_eps<T, NR, FAST, ROWEPS>(R, j), dov, mo);
-                mp = mo;
-                dp = dov;
+                typename TT::P now;
+                now.x = lvk * t1;
+                now.y = fma(GE ? eps_ge : d_eps<T, NR, FAST, ROWEPS>(R, j), old.y, old.x);
+                if (j < NR - 1)
+                    TT::pin(now);
+                MD[j] = now;
+                up = old;
             };
 #pragma unroll
             for (int qq = 0; qq < NV; ++qq) {
@@ -617,6 +646,14 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
                 acc += (s4 + u <= acc_last) ? chain : (T)0;
             else
                 acc += chain;
+            // The lane transfers (DPP) never issue beside another wave's
+            // instruction, and the older wave of a SIMD goes first in every
+            // cycle, so a younger wave stood at each of its transfers until
+            // the older one waited for something.  With the priority raised
+            // over them they issue at once: 2.89 -> 2.69 cycles per VALU
+            // instruction over the 19-row kernel (3-5% of large calls, for
+            // two more instructions per step).
+            __builtin_amdgcn_s_setprio(3);
             if constexpr (RE) {
                 // a group's first lane must not see its neighbour's values:
                 // scaled by that alignment's lane factors they may overflow,
@@ -626,14 +663,16 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
                 // turns a select of a DPP result into an exec-masked DPP,
                 // which reads 0 from the masked-off source lanes.)
                 constexpr float kBig = 3.4028234663852886e38f;
-                Mr[cur] = fminf(TT::shr(M[NR - 1]), kBig) * nf;
-                Dr[cur] = fma(fminf(TT::shr(D[NR - 1]), kBig), nf, c0f);
+                MDr[cur].x = fminf(TT::shr(MD[NR - 1].x), kBig) * nf;
+                MDr[cur].y = fma(fminf(TT::shr(MD[NR - 1].y), kBig), nf, c0f);
                 Iin = fminf(TT::shr(chain), kBig) * nf;
             } else {
-                Mr[cur] = TT::shr(M[NR - 1]) * nf;
-                Dr[cur] = fma(TT::shr(D[NR - 1]), nf, c0f);
+                MDr[cur].x = TT::shr(MD[NR - 1].x) * nf;
+                MDr[cur].y = fma(TT::shr(MD[NR - 1].y), nf, c0f);
                 Iin = TT::shr(chain) * nf;
             }
+            TT::pin(MDr[cur]);
+            __builtin_amdgcn_s_setprio(0);
         }
         letters = next;
         wlo = whi;
@@ -647,7 +686,8 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
     // points; every lane of the wave takes part in the exchange.
     auto ds_check = [&]() {
         // values are never negative: no absolute values needed
-        const float m = fmaxf(fmaxf(fmaxf((float)Mr[0], (float)Mr[1]), fmaxf((float)Dr[0], (float)Dr[1])),
+        const float m = fmaxf(fmaxf(fmaxf((float)MDr[0].x, (float)MDr[1].x),
+                                    fmaxf((float)MDr[0].y, (float)MDr[1].y)),
                               (float)Iin);
         int x = ds_E;
         if (ds_E > 0 && m > kDsGuardF) {
@@ -669,13 +709,14 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
             const int S = x - ds_E;
 #pragma unroll
             for (int j = 0; j < NR; ++j) {
-                M[j] = ldexpf(M[j], S);
-                D[j] = ldexpf(D[j], S);
+                MD[j].x = ldexpf(MD[j].x, S);
+                MD[j].y = ldexpf(MD[j].y, S);
             }
-            Mr[0] = ldexpf(Mr[0], S);
-            Mr[1] = ldexpf(Mr[1], S);
-            Dr[0] = ldexpf(Dr[0], S);
-            Dr[1] = ldexpf(Dr[1], S);
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                MDr[k].x = ldexpf(MDr[k].x, S);
+                MDr[k].y = ldexpf(MDr[k].y, S);
+            }
             Iin = ldexpf(Iin, S);
             acc = ldexpf(acc, S);
             ds_E = x;
