@@ -44,12 +44,12 @@ __global__ void k_clear_list(ClearList cl)
 // encode 4 bytes per lane: dword loads of each input array.
 
 // One wave per hap: its code bytes (dwords over the padded length), whether
-// it holds a byte other than A/C/G/T within its length (the wildcard --
-// reference GPU semantics: any such byte; CPU semantics: 'N' -- or, under
-// CPU semantics, a byte that matches nothing but itself; alignments with
-// such haps go to the exact bin, so the tile kernels' emission tables need
-// only the four bases), and the longest hap (per-block maxima into
-// kHmaxParts counters, folded by k_scan_bins).
+// it holds, within its length, the wildcard (reference GPU semantics: any
+// byte other than A/C/G/T; CPU semantics: 'N') or, under CPU semantics, a
+// byte that matches nothing but itself -- alignments with such haps go to the
+// wildcard and exact bins, so the tile kernels' emission tables need only the
+// four bases -- and the longest hap (per-block maxima into kHmaxParts
+// counters, folded by k_scan_bins).
 __global__ __launch_bounds__(256) void k_hap_pass(BinParams bp)
 {
     const BatchDesc& b = *bp.bd;
@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256) void k_hap_pass(BinParams bp)
         }
         m = max(m, hl);
         const int nd = (max(hl, 0) >> 2) + 1;  // padded length: hl + 4 - hl % 4
-        bool other = false;
+        bool wild = false, exotic = false;
         for (int d = lane; d < nd; d += 64) {
             const uint32_t w = hd[d0 + d];
             uint32_t c = 0;
@@ -79,13 +79,15 @@ __global__ __launch_bounds__(256) void k_hap_pass(BinParams bp)
             for (int k = 0; k < 4; ++k) {
                 const uint32_t code = (uint32_t)base_code_sem((uint8_t)(w >> (8 * k)), bp.semantics);
                 c |= code << (8 * k);
-                other = other | ((4 * d + k < hl) & (code >= 4u));
+                wild = wild | ((4 * d + k < hl) & (code == 4u));
+                exotic = exotic | ((4 * d + k < hl) & (code > 4u));
             }
             out[d0 + d] = c;
         }
-        other = __any(other);
+        wild = __any(wild);
+        exotic = __any(exotic);
         if (lane == 0)
-            bp.hapflag[h] = other ? 1 : 0;
+            bp.hapflag[h] = exotic ? 2 : wild ? 1 : 0;
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1)
@@ -110,8 +112,8 @@ __global__ __launch_bounds__(256) void k_hap_pass(BinParams bp)
 // row whose max_read_len covers the read (its tile has room for one more
 // row); reads beyond the last row go to the multi-tile bin 2*ntiles.  Bin 2k
 // uses the rescaled (FAST) arithmetic when the read's coefficients keep it in
-// range, else bin 2k+1 (SAFE); under per-position gcp every row's eps
-// enters the check.  Reference CPU and per-position gcp semantics: a read
+// range, else bin 2k+1 (SAFE; a multi-tile read's form is the sign of its
+// nl); under per-position gcp every row's eps enters the check.  Reference CPU and per-position gcp semantics: a read
 // holding a byte other than A/C/G/T/N goes to the exact bin 2*ntiles+1.  The slot
 // combines its lanes' verdicts and the product of alpha with row-local
 // reductions.
@@ -153,11 +155,10 @@ __global__ __launch_bounds__(256) void k_read_meta(BinParams bp)
                 k = j;
                 break;
             }
-        const bool tiled = valid && L > 0 && k < bp.ntiles;
         const int off = (valid && L > 0) ? off_i : 0;
         const int nd = (valid && L > 0) ? (L >> 2) + 1 : 0;  // dwords of the padded read
         float eps = kEpsGpu;
-        if (tiled && bp.semantics == 1)
+        if (valid && L > 0 && bp.semantics == 1)
             eps = ph2pr[min((int)b.gcp[off], 127)];
         else if (row_gcp)
             eps = 0.f;  // the rows' own eps are checked below
@@ -184,8 +185,6 @@ __global__ __launch_bounds__(256) void k_read_meta(BinParams bp)
                 }
                 rows4[q] = make_uint4(w[0], w[1], w[2], w[3]);
             }
-            if (!tiled)  // uniform over the slot
-                continue;
             float dl[4], al[4], sg[4];
 #pragma unroll
             for (int x = 0; x < 4; ++x) {
@@ -241,16 +240,15 @@ __global__ __launch_bounds__(256) void k_read_meta(BinParams bp)
         m.nl = 1.0f;
         if (L <= 0) {
             m.bin = -1;
-        } else if (k == bp.ntiles) {
-            m.bin = 2 * bp.ntiles;
         } else if (bp.semantics != 0 && exv) {
             m.bin = 2 * bp.ntiles + 1;
         } else {
             bool fast = okv && bp.allow_fast != 0 && eps <= 0.5f;
             if (fast && !(nl >= 1e-30))  // the start constant must stay a normal float
                 fast = false;
-            m.nl = fast ? (float)nl : 1.0f;
-            m.bin = 2 * k + (fast ? 0 : 1);
+            const bool multi = k == bp.ntiles;
+            m.nl = fast ? (float)nl : multi ? -1.0f : 1.0f;
+            m.bin = multi ? 2 * k : 2 * k + (fast ? 0 : 1);
         }
         bp.meta[i] = m;
     }
@@ -396,48 +394,52 @@ __device__ __forceinline__ void group_bins_build(const BinParams& bp, const Batc
 }
 
 // Per-group hap summary, uniform across the block (every wave computes it
-// and writes the same values): haps with a sequence and
-// those of them that go to the exact bin (a byte other than A/C/G/T); the others are
+// and writes the same values): haps with a sequence, those of them that hold
+// the wildcard and those with other bytes (hapflag 1 and 2); the rest are
 // cut, in order, into segments of at most `budget` columns (at least one hap
 // each) -- the super-tasks' hap ranges and their work (sort key).
 constexpr int kMaxSegs = 128;
 struct GroupHaps {
-    int nonempty, other, nseg;
+    int nonempty, wild, exotic, nseg;
     int hs[kMaxSegs], he[kMaxSegs], work[kMaxSegs];
     int cols[64];         // staging: columns of 64 haps (0: not cut into segments)
-    int info[kMaxSegs];   // haps < kMaxSegs: length (0 if empty), top bit: flagged
+    int info[kMaxSegs];   // haps < kMaxSegs: length (0 if empty) | hapflag << 29
 };
 // Length (<= 0: empty) and flag of record hap h, from the LDS copy where
 // group_haps made one.
 __device__ __forceinline__ void hap_info(const BinParams& bp, const BatchDesc& b,
-                                         const GroupHaps& gh, int h0, int h, int& hl, bool& flag)
+                                         const GroupHaps& gh, int h0, int h, int& hl, int& flag)
 {
     if (h < kMaxSegs) {
         const int v = gh.info[h];
-        hl = v & 0x7fffffff;
-        flag = v < 0;
+        hl = v & 0x1fffffff;
+        flag = v >> 29;
     } else {
         hl = b.hap_len[h0 + h];
-        flag = bp.hapflag[h0 + h] != 0;
+        flag = bp.hapflag[h0 + h];
     }
 }
 __device__ __forceinline__ void group_haps(const BinParams& bp, const BatchDesc& b, int h0, int nh,
                                            GroupHaps& gh)
 {
-    int ne = 0, ex = 0, tot = 0;
+    int ne = 0, wi = 0, ex = 0, tot = 0;
     for (int h = (int)(threadIdx.x & 63); h < nh; h += 64) {
         const int hl = b.hap_len[h0 + h];
         if (hl > 0) {
             ++ne;
-            if (bp.hapflag[h0 + h] != 0)
-                ++ex;
-            else
+            const int flag = bp.hapflag[h0 + h];
+            if (flag == 0)
                 tot += hl;
+            else if (flag == 1)
+                ++wi;
+            else
+                ++ex;
         }
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         ne += __shfl_xor(ne, o, 64);
+        wi += __shfl_xor(wi, o, 64);
         ex += __shfl_xor(ex, o, 64);
         tot += __shfl_xor(tot, o, 64);
     }
@@ -452,10 +454,10 @@ __device__ __forceinline__ void group_haps(const BinParams& bp, const BatchDesc&
         int cols = 0;
         if (h < nh) {
             const int hl = b.hap_len[h0 + h];
-            const bool flag = hl > 0 && bp.hapflag[h0 + h] != 0;
-            cols = (hl > 0 && !flag) ? hl : 0;
+            const int flag = hl > 0 ? bp.hapflag[h0 + h] : 0;
+            cols = (hl > 0 && flag == 0) ? hl : 0;
             if (h < kMaxSegs)
-                gh.info[h] = (hl > 0 ? hl : 0) | (flag ? (int)0x80000000u : 0);
+                gh.info[h] = (hl > 0 ? hl : 0) | flag << 29;
         }
         gh.cols[threadIdx.x & 63] = cols;
         __syncthreads();
@@ -480,7 +482,8 @@ __device__ __forceinline__ void group_haps(const BinParams& bp, const BatchDesc&
     }
     if ((threadIdx.x & 63) == 0) {
         gh.nonempty = ne;
-        gh.other = ex;
+        gh.wild = wi;
+        gh.exotic = ex;
         if (cur > 0) {
             gh.hs[n] = start;
             gh.he[n] = nh;
@@ -508,8 +511,28 @@ __device__ __forceinline__ ChunkPlan chunk_plan(const BinParams& bp, int k, int 
     c.rem = reads - c.nfull * c.W;
     return c;
 }
-// The item bin of tile bin k (work-bin ids past the multi-tile and exact bins).
+// The item bin of tile bin k (work-bin ids past the bins of alignments).
 __device__ __forceinline__ int item_bin_of(const BinParams& bp, int k) { return bp.NB + k; }
+// The bin of one-alignment items of reads of bin k against haps of a flag (a
+// tile bin's with flag 0 are super-tasks and item-bin items instead).  The
+// strips of the multi-tile bin take the wildcard themselves, and with it the
+// reads of tiles (of callers' tables) that the wildcard tiles do not hold.
+__device__ __forceinline__ int run_bin_of(const BinParams& bp, int k, int flag)
+{
+    const int mb = 2 * bp.ntiles;
+    if (flag == 2)
+        return mb + 1;
+    return is_tile_bin(bp, k) ? (bp.tiles[k >> 1] < 64 * kWildRows ? mb + 2 : mb) : k;
+}
+// The sort key of such a run.
+__device__ __forceinline__ int run_key_of(const BinParams& bp, int k, int flag, int hl, int g)
+{
+    const int rb = run_bin_of(bp, k, flag);
+    if (rb != 2 * bp.ntiles + 2)
+        return key_of(rb, hl, g);
+    return rb * kKeysPerBin + (kHapBuckets - 1 - wild_bucket(k, hl)) * kKeyParts +
+           (g & (kKeyParts - 1));
+}
 
 // Records with many (hap, bin) runs -- haps x min(reads, 64) above
 // kBigGroupRuns -- are counted and scattered by a block of four waves
@@ -534,7 +557,7 @@ __device__ __forceinline__ void wave_sync()
 // waves, the large ones): its reads per bin (group_bins_build), the per-bin
 // alignment counts and the sort-key histogram.  A tile bin's full chunks get
 // one key (bin, segment columns) per hap segment, counted in super-tasks;
-// item bins, the multi-tile and the exact bins get one key (bin, hap length)
+// item bins, the multi-tile, exact and wildcard bins get one key (bin, hap length)
 // per (hap, bin) run, counted in alignments.
 template <int NW>
 __global__ __launch_bounds__(64 * NW) void k_count_keys_t(BinParams bp)
@@ -543,7 +566,6 @@ __global__ __launch_bounds__(64 * NW) void k_count_keys_t(BinParams bp)
     __shared__ GroupBins gb;
     __shared__ GroupHaps gh;
     __shared__ int cnt[kMaxBins + 1], pos[kMaxBins + 1];
-    const int eb = 2 * bp.ntiles + 1;
     for (int g = blockIdx.x; g < b.G; g += gridDim.x) {
         if (big_group(b, g) != (NW > 1))  // uniform over the block
             continue;
@@ -559,15 +581,18 @@ __global__ __launch_bounds__(64 * NW) void k_count_keys_t(BinParams bp)
             const int k = gb.k[e], c = gb.cnt[e];
             if (k == bp.NB)
                 continue;
+            auto add = [&](int bin, int haps) {
+                if (haps > 0)
+                    atomicAdd(&bp.align_part[bin * kAlignParts + part], c * haps);
+            };
+            const int plain = gh.nonempty - gh.wild - gh.exotic;
             if (is_tile_bin(bp, k)) {
-                const int tiled = gh.nonempty - gh.other;
-                if (tiled > 0)
-                    atomicAdd(&bp.align_part[k * kAlignParts + part], c * tiled);
-                if (gh.other > 0)
-                    atomicAdd(&bp.align_part[eb * kAlignParts + part], c * gh.other);
-            } else if (gh.nonempty > 0) {
-                atomicAdd(&bp.align_part[k * kAlignParts + part], c * gh.nonempty);
+                add(k, plain);
+                add(run_bin_of(bp, k, 1), gh.wild);
+            } else {
+                add(k, plain + gh.wild);
             }
+            add(run_bin_of(bp, k, 2), gh.exotic);
         }
         // per (tile bin entry, hap segment): its super-tasks' key
         for (int x = threadIdx.x; x < n * gh.nseg; x += 64 * NW) {
@@ -584,18 +609,17 @@ __global__ __launch_bounds__(64 * NW) void k_count_keys_t(BinParams bp)
         for (int x = threadIdx.x; x < nh * n; x += 64 * NW) {
             const int h = x / n, e = x - h * n;
             const int k = gb.k[e];
-            int hl;
-            bool other;
-            hap_info(bp, b, gh, h0, h, hl, other);
+            int hl, flag;
+            hap_info(bp, b, gh, h0, h, hl, flag);
             if (hl <= 0 || k == bp.NB)
                 continue;
-            if (is_tile_bin(bp, k) && !other) {
+            if (is_tile_bin(bp, k) && flag == 0) {
                 const ChunkPlan c = chunk_plan(bp, k, gb.cnt[e]);
                 if (c.rem > 0)
                     atomicAdd(&bp.key_count[key_of(item_bin_of(bp, k), hl, g)], c.rem);
                 continue;
             }
-            atomicAdd(&bp.key_count[key_of(is_tile_bin(bp, k) ? eb : k, hl, g)], gb.cnt[e]);
+            atomicAdd(&bp.key_count[run_key_of(bp, k, flag, hl, g)], gb.cnt[e]);
         }
         __syncthreads();
     }
@@ -758,7 +782,6 @@ __device__ __forceinline__ void scatter_hap_chunk(const BinParams& bp, const Bat
 {
     constexpr int kSkip = -2;  // run covered by a super-task
     const int lane = threadIdx.x & 63;
-    const int eb = 2 * bp.ntiles + 1;
     const int n = gb.n;
     auto sync = [] {
         if (kWaveSync)
@@ -773,12 +796,11 @@ __device__ __forceinline__ void scatter_hap_chunk(const BinParams& bp, const Bat
         if (x < hcn * n) {
             const int h = hc + x / n, e = x % n;
             const int k = gb.k[e];
-            int hl;
-            bool other;
-            hap_info(bp, b, gh, h0, h, hl, other);
+            int hl, flag;
+            hap_info(bp, b, gh, h0, h, hl, flag);
             base = -1;  // -inf
             if (hl > 0 && k != bp.NB) {
-                if (is_tile_bin(bp, k) && !other) {
+                if (is_tile_bin(bp, k) && flag == 0) {
                     // super-tasks cover the full chunks; left-over reads
                     // become items of the bin's item bin
                     const ChunkPlan cp = chunk_plan(bp, k, gb.cnt[e]);
@@ -787,8 +809,8 @@ __device__ __forceinline__ void scatter_hap_chunk(const BinParams& bp, const Bat
                                        : bp.bin_range[2 * kb] +
                                              atomicAdd(&bp.key_cursor[key_of(kb, hl, g)], cp.rem);
                 } else {
-                    const int kb = is_tile_bin(bp, k) ? eb : k;
-                    base = bp.bin_range[2 * kb] + atomicAdd(&bp.key_cursor[key_of(kb, hl, g)], gb.cnt[e]);
+                    base = bp.bin_range[2 * run_bin_of(bp, k, flag)] +
+                           atomicAdd(&bp.key_cursor[run_key_of(bp, k, flag, hl, g)], gb.cnt[e]);
                 }
             }
         }
@@ -816,10 +838,9 @@ __device__ __forceinline__ void scatter_hap_chunk(const BinParams& bp, const Bat
             cnt = gb.cnt[e];
             st = gb.st[e];
             if (base >= 0 && is_tile_bin(bp, gb.k[e])) {
-                int hl;
-                bool other;
-                hap_info(bp, b, gh, h0, h, hl, other);
-                if (!other) {  // an item-bin run: the left-over reads only
+                int hl, flag;
+                hap_info(bp, b, gh, h0, h, hl, flag);
+                if (flag == 0) {  // an item-bin run: the left-over reads only
                     const ChunkPlan cp = chunk_plan(bp, gb.k[e], cnt);
                     st += cp.nfull * cp.W;
                     cnt = cp.rem;

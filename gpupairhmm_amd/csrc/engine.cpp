@@ -194,7 +194,7 @@ void Engine::bins_for(const phmm_batch_view& v, int* NB, int* NW) const
     const bool small =
         roweps() || (opt.small_batch > 0 && v.num_alignments <= opt.small_batch);
     const int ntiles = (int)(small ? tiles_small : tiles).size();
-    *NB = 2 * ntiles + 2;
+    *NB = 2 * ntiles + 3;
     *NW = *NB + 2 * ntiles;
 }
 
@@ -335,7 +335,7 @@ int Engine::score_device(const phmm_batch_view& v, float* d_scores, hipStream_t 
     act = (roweps() || (opt.small_batch > 0 && table_n <= opt.small_batch)) ? &tiles_small : &tiles;
     const std::vector<phmm_tile_config>& tiles = *act;
     const int ntiles = (int)tiles.size();
-    const int NB = 2 * ntiles + 2;  // + multi-tile bin + exact bin
+    const int NB = 2 * ntiles + 3;  // + multi-tile, exact and wildcard bins
     const int NW = NB + 2 * ntiles; // + an item bin per tile bin
     const int G = v.num_groups;
     const int64_t nA = v.num_alignments;
@@ -578,8 +578,9 @@ int Engine::enqueue_prep(const BinParams& bp, const BatchDesc& hd, bool fixed, h
 }
 
 // Pass 1: FP32 tile kernels over the tile bins' super-tasks (results below
-// the rescue threshold go to the bin's rescue list) and the one-wave kernel
-// over the multi-tile and exact bins' items.  Batched: one persistent launch
+// the rescue threshold go to the bin's rescue list), then the strips and
+// packed waves of the multi-tile and wildcard bins and the one-wave kernel
+// over the exact bin's items (over all three where the pass does not scale).  Batched: one persistent launch
 // per kernel template covering all of its bins, larger tiles first.  Plain:
 // one launch per non-empty bin after the host has read the bin sizes back
 // (the reference's per-partition launches).
@@ -589,6 +590,7 @@ int Engine::enqueue_fwd(const FwdParams& fp, const BinParams& bp, bool plain, hi
     const int ntiles = (int)tiles.size();
     const int mb = 2 * ntiles;  // multi-tile bin
     const int eb = mb + 1;      // exact bin
+    const int wb = mb + 2;      // wildcard bin
     float* spill32 = static_cast<float*>(cur->call_spill);
     const int64_t n32 = (int64_t)(cur->call_spill_bytes / sizeof(float));
     const int32_t* h_bin_range = cur->h_bin_range;
@@ -669,26 +671,50 @@ int Engine::enqueue_fwd(const FwdParams& fp, const BinParams& bp, bool plain, hi
                 return rc;
         }
     }
-    // the multi-tile bin and the exact bin: one wave per alignment
-    if (plain) {
-        const int n = h_bin_range[2 * mb + 1] + h_bin_range[2 * eb + 1];
-        if (n <= 0)
-            return PHMM_OK;
-        stats.multitile_alignments += n;
-    }
+    // the multi-tile and wildcard bins: the scaled sweep, where the FP32 pass
+    // scales; the exact bin (and those two otherwise): one wave per alignment
+    const int n_special = plain ? h_bin_range[2 * mb + 1] + h_bin_range[2 * wb + 1] : 1;
+    const int n_exact = plain ? h_bin_range[2 * eb + 1] : 1;
+    if (plain)
+        stats.multitile_alignments += n_special + n_exact;
+    const int waves = num_cus * 8;
     BinSet ws;
-    ws.n = 2;
-    ws.bin[0] = mb;
-    ws.bin[1] = eb;
-    ws.lanes[0] = ws.lanes[1] = 64;
+    ws.bin[ws.n++] = eb;
+    if (scaled_pass()) {
+        SpecialSet ss;
+        ss.items = bp.items;
+        ss.range = bp.bin_range;
+        ss.strip_bin = mb;
+        ss.wild_bin = wb;
+        if (ctr >= kTaskCounters - kF64Sets - kReSets)
+            return set_error(PHMM_ERANGE, "too many set launches");
+        ss.next_task = bp.task_ctr + ctr++;
+        ss.hmax = bp.hmax;
+        ss.border = static_cast<float4*>(cur->call_spill);
+        ss.border_entries = (int64_t)(cur->call_spill_bytes / sizeof(float4));
+        ss.error_flag = bp.error_flag;
+        if (n_special > 0 &&
+            (rc = check(launch_fwd_special(fp, ss, plain ? std::min(waves, n_special) : waves, st),
+                        "multi-tile kernel")))
+            return rc;
+        // no byte is exact-only under the reference GPU semantics
+        if (n_exact <= 0 || opt.semantics == PHMM_SEM_GPU)
+            return PHMM_OK;
+    } else {
+        ws.bin[ws.n++] = mb;
+        ws.bin[ws.n++] = wb;
+        if (n_special + n_exact <= 0)
+            return PHMM_OK;
+    }
+    for (int i = 0; i < ws.n; ++i)
+        ws.lanes[i] = 64;
     ws.items = bp.items;
     ws.range = bp.bin_range;
     ws.counts = bp.bin_range + 1;
     ws.count_stride = 2;
-    const int blocks =
-        plain ? std::min(num_cus * 8, h_bin_range[2 * mb + 1] + h_bin_range[2 * eb + 1]) : num_cus * 8;
-    return check(launch_fwd_wave_f32(fp, ws, bp.hmax, spill32, n32, bp.error_flag, blocks, st),
-                 "multi-tile kernel");
+    return check(launch_fwd_wave_f32(fp, ws, bp.hmax, spill32, n32, bp.error_flag,
+                                     plain ? std::min(waves, n_special + n_exact) : waves, st),
+                 "exact kernel");
 }
 
 // Pass 2 (range_rescue): the rescue lists of tile bins whose rows per lane

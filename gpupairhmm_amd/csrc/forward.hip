@@ -14,8 +14,8 @@
 // wavefront).  Row-above values cross lanes with DPP wave_shr:1, a group's
 // first lane injects the row-0 boundary.  Emission probabilities for the
 // 4 bases x NR rows of each lane sit in LDS (one ds_read_b128 per 4 cells,
-// conflict-free by lane interleaving; haps holding any other byte go to the
-// one-wave kernel).  Its work comes in two units: super-tasks (up to 64/G
+// conflict-free by lane interleaving; haps holding the wildcard go to
+// k_fwd_special).  Its work comes in two units: super-tasks (up to 64/G
 // reads of one record against a segment of the record's haps: the wave sets
 // the reads up once and sweeps the haps one after another) and items (one
 // alignment per group: reads a record leaves over after full chunks, and the
@@ -42,6 +42,8 @@
 // (pairhmm_kernels.cuh:1325-1356): the first row past the read turns the
 // I-chain into (M+I) of the last row, later rows pass it through, and the
 // lane holding row R accumulates it one column behind.
+//
+// k_fwd_special -- reads of several tiles and haps with the wildcard.
 //
 // k_fwd_wave -- one alignment per wave, any read length, FP32 or FP64, with
 // the plain (unscaled) recurrence.  Reads longer than the largest tile are
@@ -139,7 +141,8 @@ struct TileTraits<double> {
 };
 
 // Shape of a lane's emission table in LDS: NV vectors of K rows (the last
-// may hold fewer), each for the 4 letters, tab[(q*4 + letter)*64 + lane] --
+// may hold fewer), each for the NL letters (4: the bases; 5: the wildcard of
+// the hap too), tab[(q*NL + letter)*64 + lane] --
 // one ds_read of 16 bytes per vector, conflict-free because consecutive
 // lanes read consecutive 16-byte words; a letter's entry is 64 words on, so
 // its address is a shift of the letter whatever NV (a multiply by NV*64
@@ -147,14 +150,14 @@ struct TileTraits<double> {
 // read as one 4-byte word at a 16-byte lane stride, four lanes to a bank,
 // so such a row (kTail) sits in a table of scalars instead,
 // stab[letter*64 + lane], at a 4-byte lane stride.
-template <typename T, int NR>
+template <typename T, int NR, int NL = 4>
 struct TabShape {
     static constexpr int K = TileTraits<T>::K;
     static constexpr bool kTail = K > 1 && NR % K == 1;
     static constexpr int NV = kTail ? NR / K : (NR + K - 1) / K;
-    static constexpr int kVecs = 4 * NV * 64;
+    static constexpr int kVecs = NL * NV * 64;
     static constexpr int kWords =  // table size in units of the vector type
-        kVecs + (kTail ? (4 * 64 * (int)sizeof(T) + (int)sizeof(typename TileTraits<T>::V) - 1) /
+        kVecs + (kTail ? (NL * 64 * (int)sizeof(T) + (int)sizeof(typename TileTraits<T>::V) - 1) /
                              (int)sizeof(typename TileTraits<T>::V)
                        : 0);
 };
@@ -208,10 +211,12 @@ __device__ __forceinline__ T beta_of(T e)
 // beta, so row r+1's M adds it with weight 1): c2 = beta_{r+1} delta_r,
 // c3 = eps_r beta_{r+1} / beta_r, and D chain Dh = M< + eps_r Dh<; the last
 // row's beta_{L+1} is taken as beta_L, which the epilogue divides out.
-template <typename T, int NR, bool FAST, bool ROWEPS>
+//
+// row0: the first row of the tile (reads of several tiles).
+template <typename T, int NR, bool FAST, bool ROWEPS, int NL = 4>
 __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTraits<T>::V* tab,
                                            bool active, int read, int t,
-                                           TileRead<T, NR, ROWEPS>& R)
+                                           TileRead<T, NR, ROWEPS>& R, int row0 = 0)
 {
     const BatchDesc& bd = *p.bd;
     using TT = TileTraits<T>;
@@ -241,7 +246,7 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
     auto row_eps = [&](int ri) -> T { return (T)ph2pr_of(p.ph2pr, bd.gcp[roff + ri]); };
 
     // ---- per-row coefficients and the emission table -------------------
-    const int r0 = t * NR;
+    const int r0 = row0 + t * NR;
     {
         T pdelta = 0, psigma = 0, palpha = 1;
         if (r0 >= 1 && r0 - 1 < L) {
@@ -314,14 +319,14 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
                 }
             }
         }
-        // emission table: tab[(letter*NV + q)*64 + lane] = rows K*q .. K*q+K-1
-        // for the four bases (haps with any other byte go to the one-wave
-        // kernel; a read's 'N' matches every base), a single last row in the
-        // scalar table
-        using Shape = TabShape<T, NR>;
+        // emission table: tab[(q*NL + letter)*64 + lane] = rows K*q .. K*q+K-1
+        // for the four bases and, with NL 5, a hap's wildcard, which every
+        // row matches (a read's 'N' matches every base), a single last row in
+        // the scalar table
+        using Shape = TabShape<T, NR, NL>;
         constexpr int NV = Shape::NV;
 #pragma unroll
-        for (int l = 0; l < 4; ++l) {
+        for (int l = 0; l < NL; ++l) {
 #pragma unroll
             for (int q = 0; q < NV; ++q) {
                 T v[K];
@@ -329,17 +334,17 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
                 for (int k = 0; k < K; ++k) {
                     const int j = K * q + k;
                     if (j < NR) {
-                        const bool m = (l == code[j]) || (code[j] == 4);
+                        const bool m = l == 4 || (l == code[j]) || (code[j] == 4);
                         v[k] = m ? lm[j] : lx[j];
                     } else {
                         v[k] = 0;  // past the lane's rows: never used
                     }
                 }
-                tab[(q * 4 + l) * 64 + lane] = TT::pack(v);
+                tab[(q * NL + l) * 64 + lane] = TT::pack(v);
             }
             if constexpr (Shape::kTail) {
                 constexpr int j = NR - 1;
-                const bool m = (l == code[j]) || (code[j] == 4);
+                const bool m = l == 4 || (l == code[j]) || (code[j] == 4);
                 reinterpret_cast<T*>(tab + Shape::kVecs)[l * 64 + lane] = m ? lm[j] : lx[j];
             }
         }
@@ -349,6 +354,151 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
             TT::pin(R.c32[j]);
         }
     }
+}
+
+// One cell: row j of the lane's tile at the lane's column, with emission value
+// lam.  `up` holds the row above's (M, D) one column back, `chain` its I at
+// this column; both move on to this row's.
+//
+// A SIMD issues a VALU instruction of one wave and, beside it, one of another
+// wave -- but beside it only an instruction whose three vector sources do not
+// all sit in registers of one parity (measured with two waves: 2.03 cycles
+// per FMA with mixed parities, 4.2 with one; a quarter of freely allocated
+// FMAs has one).  So M and D of a row are a register pair, M even and D odd,
+// and so are its coefficients (c1, c0) and (c3, c2): with chain in M's old
+// register every FMA mixes parities.  150-base reads against 150-350-base
+// haps: 2.69 -> 2.58 cycles per VALU instruction over the 19-row kernel, 1-2%
+// of the call (the clock gives some of it back).  The last row's pair is only
+// read by the lane transfer, and pinning it cost a move.
+template <typename T, int NR, bool FAST, bool ROWEPS>
+__device__ __forceinline__ void tile_cell(const TileRead<T, NR, ROWEPS>& R, int j, T lam, T eps,
+                                          typename TileTraits<T>::P& md,
+                                          typename TileTraits<T>::P& up, T& chain)
+{
+    const typename TileTraits<T>::P old = md;
+    T t1;
+    if (FAST) {
+        t1 = fma(R.c10[j].x, up.y, up.x);
+        t1 = fma(R.c10[j].y, chain, t1);
+        chain = fma(R.c32[j].y, chain, up.x);
+    } else {
+        t1 = fma(R.c10[j].x, up.y, chain);
+        t1 = fma(R.c10[j].y, up.x, t1);
+        chain = fma(R.c32[j].y, up.x, R.c32[j].x * chain);
+    }
+    typename TileTraits<T>::P now;
+    now.x = lam * t1;
+    now.y = fma(eps, old.y, old.x);
+    if (j < NR - 1)
+        TileTraits<T>::pin(now);
+    md = now;
+    up = old;
+}
+
+// In-pass scaling: the lane above's value of an exponent.  The shifted value
+// is kept opaque to the compiler: fused into the subtraction that uses it
+// (v_subrev_u32_dpp), it measured as E_{t-1} - E_t on gfx950.
+__device__ __forceinline__ int ds_above(int v)
+{
+    int u = shr1i(v);
+    asm volatile("" : "+v"(u));
+    return u;
+}
+// x capped at kDsSpan per lane above the group's lanes over it (x_t <= x_k +
+// kDsSpan * (t - k) for k < t: a prefix minimum of x - kDsSpan * t); t: the
+// lane's index in its group.
+__device__ __forceinline__ int ds_span_cap(int x, int t)
+{
+    int z = x - kDsSpan * t;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(z, o, 64);
+        if (t >= o)
+            z = y < z ? y : z;
+    }
+    return z + kDsSpan * t;
+}
+// The exponent a lane starts with, from the insertion floor at row index
+// `last` of a read whose packed rows start at rw: the product of the rows'
+// chain coefficients down to that row, which telescopes -- FAST: eps^R *
+// delta_0 / delta_R / prod(alpha_0 .. alpha_{R-1}); SAFE: eps per row.  The
+// alpha factors (each <= 1) are left out, which can only put the estimate
+// below the true floor.  No lane exchange needed.
+template <bool FAST>
+__device__ __forceinline__ int ds_start(const FwdParams& p, float C0, float eps, int last,
+                                        const uint32_t* rw)
+{
+    float fl = __log2f(C0) + (float)last * __log2f(eps);
+    if (FAST && last > 0)
+        fl += __log2f(ph2pr_of(p.ph2pr, row_iq(rw[0]))) -
+              __log2f(ph2pr_of(p.ph2pr, row_iq(rw[last])));
+    // the floor of the row at 2^kDsFloor
+    const int e0 = (int)floorf((float)kDsFloor - fl);
+    return e0 < 0 ? 0 : e0;
+}
+// The exponent of a lane with exponent E that holds or took in values up to
+// m (never negative): lowered to put m at 2^kDsGuardTo once it passed
+// `guard`, never below 0.
+__device__ __forceinline__ int ds_lowered(int E, float m, float guard)
+{
+    if (!(E > 0 && m > guard))
+        return E;
+    // v_frexp_exp reads inf as 0: an overflowed lane keeps its exponent and
+    // fails acceptance
+    const int g = E + kDsGuardTo - (__builtin_amdgcn_frexp_expf(m) - 1);
+    return g < 0 ? 0 : g;
+}
+// The score of a scaled result: the sum a * 2^-E (ok: the sweep's acceptance),
+// or, refused, -inf and an entry in `list`.  Returns whether the sum fell
+// below the rescue threshold and is finished.
+template <bool FAST>
+__device__ __forceinline__ bool ds_finish(const FwdParams& p, const WorkItem& it, float a, int E,
+                                          bool ok, float nl, float beta, WorkItem* list,
+                                          int32_t* count)
+{
+    if (!ok || !(a >= 0x1p-100f && a <= 3.4028234663852886e38f)) {
+        p.bd->scores[it.out] = -INFINITY;
+        list[atomicAdd(count, 1)] = it;
+        return false;
+    }
+    // the unscaled sum, where it is a normal float: the score and threshold
+    // test of the unscaled instance, bit for bit
+    const float at = ldexpf(a, -E);
+    float raw;
+    if (at >= 0x1p-126f) {
+        p.bd->scores[it.out] = FAST ? log10f(at) - (kLog10Scale - kLog10FastKappa)
+                                    : log10f(at) - (kLog10Scale + log10f(beta));
+        raw = FAST ? at * nl : at / beta;
+    } else {
+        // a * 2^-E = m * 2^K exactly: the score does not depend on how the
+        // rows were split into lanes
+        int e2 = 0;
+        const float m = frexpf(a, &e2);
+        const int K = e2 - E;
+        const double off = FAST ? (double)kLog10Scale - (double)kLog10FastKappa
+                                : (double)kLog10Scale + log10((double)beta);
+        p.bd->scores[it.out] =
+            (float)(log10((double)m) + (double)K * 0.30102999566398119521 - off);
+        raw = ldexpf(FAST ? a * nl : a / beta, -E);
+    }
+    return !(raw >= p.rescue_min);
+}
+// The score of an unscaled FP32 sum; returns whether the sum reached the
+// rescue threshold.
+template <bool FAST>
+__device__ __forceinline__ bool f32_finish(const FwdParams& p, const WorkItem& it, float a, float nl,
+                                           float beta)
+{
+    float score, raw;
+    if (FAST) {
+        score = log10f(a) - (kLog10Scale - kLog10FastKappa);
+        raw = a * nl;
+    } else {
+        score = log10f(a) - (kLog10Scale + log10f(beta));
+        raw = a / beta;
+    }
+    p.bd->scores[it.out] = score;
+    return raw >= p.rescue_min;
 }
 
 // One sweep of this group's read (R) against a hap of length HL at hoff;
@@ -466,27 +616,6 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
     }
     int ds_E = 0;  // DS: this lane's exponent (held = true * 2^ds_E)
     bool ds_any = false;  // DS: some lane of the wave is scaled (uniform)
-    // DS: x capped at kDsSpan per lane above the group's lanes over it
-    // (x_t <= x_k + kDsSpan * (t - k) for k < t: a prefix minimum of
-    // x - kDsSpan * t)
-    auto ds_span_cap = [&](int x) {
-        int z = x - kDsSpan * t;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const int y = __shfl_up(z, o, 64);
-            if (t >= o)
-                z = y < z ? y : z;
-        }
-        return z + kDsSpan * t;
-    };
-    // DS: the lane above's value of an exponent.  The shifted value is
-    // kept opaque to the compiler: fused into the subtraction that uses it
-    // (v_subrev_u32_dpp), it measured as E_{t-1} - E_t on gfx950.
-    auto ds_above = [&](int v) {
-        int u = shr1i(v);
-        asm volatile("" : "+v"(u));
-        return u;
-    };
     // DS: the transfer factor 2^(E_t - E_{t-1}), exact as long as the
     // exponents stay within kDsSpan
     auto ds_factor = [&]() -> T {
@@ -494,27 +623,14 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
         return first ? (T)0 : (T)ldexpf(1.0f, d);
     };
     if constexpr (DS) {
-        // The insertion floor at the lane's last row R (the read's last
-        // row for the lanes past it): the product of the rows' chain
-        // coefficients from row 1 to R, which telescopes -- FAST: eps^R *
-        // delta_0 / delta_R / prod(alpha_0 .. alpha_{R-1}); SAFE: eps per
-        // row.  The alpha factors (each <= 1) are left out, which can only
-        // put the estimate below the true floor.  No lane exchange needed.
-        float fl = 0.0f;
-        if (active && C0 > 0 && L > 0) {
-            const int last = min((t + 1) * NR, L) - 1;
-            fl = __log2f((float)C0) + (float)last * __log2f((float)R.eps);
-            if (FAST && last > 0) {
-                const uint32_t* rw = p.rows + bd.read_off[it.read];
-                fl += __log2f(ph2pr_of(p.ph2pr, row_iq(rw[0]))) -
-                      __log2f(ph2pr_of(p.ph2pr, row_iq(rw[last])));
-            }
-        }
-        // the floor of the lane's last row at 2^kDsFloor
-        const int e0 = (int)floorf((float)kDsFloor - fl);
-        int x = first || e0 < 0 ? 0 : e0;
+        // from the floor of the lane's last row (the read's last row for the
+        // lanes past it); a group's first lane is not scaled
+        int x = 0;
+        if (active && C0 > 0 && L > 0 && !first)
+            x = ds_start<FAST>(p, (float)C0, (float)R.eps, min((t + 1) * NR, L) - 1,
+                               p.rows + bd.read_off[it.read]);
         if (__ballot(!first && x - ds_above(x) > kDsSpan))  // steep gap scores only
-            x = ds_span_cap(x);
+            x = ds_span_cap(x, t);
         ds_E = x;
         nf = ds_factor();
         ds_any = __ballot(ds_E > 0) != 0;
@@ -595,38 +711,9 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
             }
             typename TT::P up = MDr[cur];  // the row above's (M, D), one column back
             T chain = Iin;
-            // the cell of row j with emission value lvk.  A SIMD issues a
-            // VALU instruction of one wave and, beside it, one of another
-            // wave -- but beside it only an instruction whose three vector
-            // sources do not all sit in registers of one parity (measured
-            // with two waves: 2.03 cycles per FMA with mixed parities, 4.2
-            // with one; a quarter of freely allocated FMAs has one).  So M
-            // and D of a row are a register pair, M even and D odd, and so
-            // are its coefficients (c1, c0) and (c3, c2): with chain in M's
-            // old register every FMA mixes parities.  150-base reads
-            // against 150-350-base haps: 2.69 -> 2.58 cycles per VALU
-            // instruction over the 19-row kernel, 1-2% of the call (the
-            // clock gives some of it back).  The last row's pair is only
-            // read by the transfer below, and pinning it cost a move.
             auto cell = [&](int j, T lvk) {
-                const typename TT::P old = MD[j];
-                T t1;
-                if (FAST) {
-                    t1 = fma(R.c10[j].x, up.y, up.x);
-                    t1 = fma(R.c10[j].y, chain, t1);
-                    chain = fma(R.c32[j].y, chain, up.x);
-                } else {
-                    t1 = fma(R.c10[j].x, up.y, chain);
-                    t1 = fma(R.c10[j].y, up.x, t1);
-                    chain = fma(R.c32[j].y, up.x, R.c32[j].x * chain);
-                }
-                typename TT::P now;
-                now.x = lvk * t1;
-                now.y = fma(GE ? eps_ge : d_eps<T, NR, FAST, ROWEPS>(R, j), old.y, old.x);
-                if (j < NR - 1)
-                    TT::pin(now);
-                MD[j] = now;
-                up = old;
+                tile_cell<T, NR, FAST, ROWEPS>(
+                    R, j, lvk, GE ? eps_ge : d_eps<T, NR, FAST, ROWEPS>(R, j), MD[j], up, chain);
             };
 #pragma unroll
             for (int qq = 0; qq < NV; ++qq) {
@@ -689,13 +776,7 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
         const float m = fmaxf(fmaxf(fmaxf((float)MDr[0].x, (float)MDr[1].x),
                                     fmaxf((float)MDr[0].y, (float)MDr[1].y)),
                               (float)Iin);
-        int x = ds_E;
-        if (ds_E > 0 && m > kDsGuardF) {
-            // v_frexp_exp reads inf as 0: an overflowed lane keeps its
-            // exponent and fails acceptance
-            const int g = ds_E + kDsGuardTo - (__builtin_amdgcn_frexp_expf(m) - 1);
-            x = g < 0 ? 0 : g;
-        }
+        int x = ds_lowered(ds_E, m, kDsGuardF);
         // any distance in one step: v_ldexp is exact wherever the result
         // stays normal
         if (__ballot(x != ds_E)) {
@@ -705,7 +786,7 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
             // the lane below sees, does); the scan only where a gap opened
             const int xu = ds_above(x);
             if (__ballot(!first && x - xu > kDsSpan))
-                x = ds_span_cap(x);
+                x = ds_span_cap(x, t);
             const int S = x - ds_E;
 #pragma unroll
             for (int j = 0; j < NR; ++j) {
@@ -808,46 +889,10 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
     int slot = -1;  // REC: the rescued alignment's rescue-list slot
     if (active && t == L / NR) {
         if (DS && (ds_fb || ds_E > 0 || !((float)acc <= 3.4028234663852886e38f))) {
-            const float a = (float)acc;
-            if (!ds_fb && a >= 0x1p-100f && a <= 3.4028234663852886e38f) {
-                // the unscaled sum, where it is a normal float: the score and
-                // threshold test of the unscaled instance, bit for bit
-                const float at = ldexpf(a, -ds_E);
-                float raw;
-                if (at >= 0x1p-126f) {
-                    bd.scores[it.out] = FAST ? log10f(at) - (kLog10Scale - kLog10FastKappa)
-                                             : log10f(at) - (kLog10Scale + log10f((float)beta));
-                    raw = FAST ? at * nl : at / (float)beta;
-                } else {
-                    // a * 2^-E = m * 2^K exactly: the score does not depend
-                    // on how the rows were split into lanes
-                    int e2 = 0;
-                    const float m = frexpf(a, &e2);
-                    const int K = e2 - ds_E;
-                    const double off = FAST ? (double)kLog10Scale - (double)kLog10FastKappa
-                                            : (double)kLog10Scale + log10((double)(float)beta);
-                    bd.scores[it.out] =
-                        (float)(log10((double)m) + (double)K * 0.30102999566398119521 - off);
-                    raw = ldexpf(FAST ? a * nl : a / (float)beta, -ds_E);
-                }
-                ds_done = !(raw >= p.rescue_min);
-            } else {
-                bd.scores[it.out] = -INFINITY;
-                const int n = atomicAdd(p.rescue_counts + bin, 1);
-                p.rescue_items[rescue_base + n] = it;
-            }
+            ds_done = ds_finish<FAST>(p, it, (float)acc, ds_E, !ds_fb, nl, (float)beta,
+                                      p.rescue_items + rescue_base, p.rescue_counts + bin);
         } else if (F32) {
-            const float a = (float)acc;
-            float score, raw;
-            if (FAST) {
-                score = log10f(a) - (kLog10Scale - kLog10FastKappa);
-                raw = a * nl;
-            } else {
-                score = log10f(a) - (kLog10Scale + log10f((float)beta));
-                raw = a / (float)beta;
-            }
-            bd.scores[it.out] = score;
-            if (p.rescue_on && !(raw >= p.rescue_min)) {
+            if (!f32_finish<FAST>(p, it, (float)acc, nl, (float)beta) && p.rescue_on) {
                 const int n = atomicAdd(p.rescue_counts + bin, 1);
                 p.rescue_items[rescue_base + n] = it;
                 if (REC && p.re_on)
@@ -919,7 +964,7 @@ __device__ __forceinline__ int tile_items_task(const FwdParams& p, typename Tile
 // A super-task: the groups set up their reads once and sweep the segment's
 // haps in turn (all groups share each hap, so every sweep is uniform across
 // the wave).  Empty haps were scored -inf by the scatter; haps holding a
-// byte other than A/C/G/T belong to the exact bin.
+// byte other than A/C/G/T have bins of their own.
 template <typename T, int NR, bool FAST, bool ROWEPS, bool DS = false, bool GE = false>
 __device__ __forceinline__ int tile_super_task(const FwdParams& p, typename TileTraits<T>::V* tab,
                                                const SuperTask& st, int G, int rescue_base, int bin)
@@ -1088,13 +1133,208 @@ struct WaveScalar<float> {
     __device__ static float shr(float v) { return shr1f(v); }
     __device__ static float ldexp(float v, int k) { return ldexpf(v, k); }
     __device__ static int ilogb(float v) { return ilogbf(v); }
+    // ilogb of a positive finite value in one instruction
+    __device__ static int expo(float v) { return __builtin_amdgcn_frexp_expf(v) - 1; }
 };
 template <>
 struct WaveScalar<double> {
     __device__ static double shr(double v) { return shr1d(v); }
     __device__ static double ldexp(double v, int k) { return ::ldexp(v, k); }
     __device__ static int ilogb(double v) { return ::ilogb(v); }
+    __device__ static int expo(double v) { return __builtin_amdgcn_frexp_exp(v) - 1; }
 };
+
+// k_fwd_wave's arithmetic for reads of one tile, `take` items (reads below 64 *
+// NR bases, no byte that matches nothing but itself, one gap continuation per
+// read) side by side on the wave, G lanes each.  What differs is how the
+// emission values are found: in an LDS table of five letters (as
+// tile_setup's), with the letters loaded four columns ahead, where k_fwd_wave
+// compares codes.  It runs k_fwd_wave's 64 steps past the hap as well: the
+// lanes rescale over them, and with them the sum.
+template <typename T, int NR>
+__device__ __forceinline__ void pack_task(const FwdParams& p, typename TileTraits<T>::V* tab,
+                                          const WorkItem* items, int take, int G)
+{
+    using S = WaveScalar<T>;
+    using V = typename TileTraits<T>::V;
+    constexpr int K = TileTraits<T>::K, NV = NR / K, NL = 5;
+    static_assert(NR % K == 0, "whole vectors");
+    constexpr int kNone = -(1 << 28);
+    const BatchDesc& bd = *p.bd;
+    const int lane = threadIdx.x, grp = lane / G, t = lane - grp * G;
+    const bool active = grp < take;
+    WorkItem it;
+    it.read = 0;
+    it.hap = 0;
+    it.out = -1;
+    it.pad = 0;
+    if (active)
+        it = items[grp];
+    const int L = active ? bd.read_len[it.read] : 0, HL = active ? bd.hap_len[it.hap] : 0;
+    const int roff = active ? bd.read_off[it.read] : 0;
+    T eps = (T)kEpsGpu, beta = (T)kBetaGpu;
+    if (p.semantics == 1 && active) {
+        const float e = ph2pr_of(p.ph2pr, bd.gcp[roff]);
+        eps = (T)e;
+        beta = (T)1 - (T)e;
+    }
+    const T C0 = active ? S::ldexp((T)1, 64) / (T)HL : (T)0;
+    T ca[NR], cb[NR], cdl[NR], cs[NR], ce[NR];
+#pragma unroll
+    for (int q = 0; q < NV; ++q) {
+        T lm[K], lx[K];
+        int code[K];
+#pragma unroll
+        for (int x = 0; x < K; ++x) {
+            const int j = K * q + x, ri = t * NR + j;
+            if (ri < L) {
+                const uint32_t w = p.rows[roff + ri];
+                const T pb = (T)ph2pr_of(p.ph2pr, row_bq(w));
+                const T de = (T)ph2pr_of(p.ph2pr, row_iq(w));
+                const T si = (T)ph2pr_of(p.ph2pr, row_dq(w));
+                ca[j] = (T)1 - (de + si);
+                cb[j] = beta;
+                cdl[j] = de;
+                cs[j] = si;
+                ce[j] = eps;
+                lm[x] = (T)1 - pb;
+                code[x] = row_code(w);
+                lx[x] = code[x] == 4 ? lm[x] : pb / (T)3;
+            } else {
+                ca[j] = 0;
+                cb[j] = 0;
+                cdl[j] = ri == L ? (T)1 : (T)0;
+                cs[j] = 0;
+                ce[j] = 1;
+                lm[x] = 0;
+                lx[x] = 0;
+                code[x] = 4;
+            }
+        }
+#pragma unroll
+        for (int l = 0; l < NL; ++l) {
+            T v[K];
+#pragma unroll
+            for (int x = 0; x < K; ++x)
+                v[x] = l == 4 || l == code[x] ? lm[x] : lx[x];
+            tab[(q * NL + l) * 64 + lane] = TileTraits<T>::pack(v);
+        }
+    }
+    T M[NR], D[NR];
+#pragma unroll
+    for (int j = 0; j < NR; ++j) {
+        M[j] = 0;
+        D[j] = 0;
+    }
+    int sc = 0, sc_end = 0;
+    T acc = 0, acc_end = 0, C0s = C0;
+    T Ml = 0, Dl = t == 0 ? C0 : (T)0, Mul = 0, Dul = Dl, Iin = 0;
+    const int tr = L / NR;
+    auto rescale = [&](int kk) {
+#pragma unroll
+        for (int j = 0; j < NR; ++j) {
+            M[j] = S::ldexp(M[j], kk);
+            D[j] = S::ldexp(D[j], kk);
+        }
+        Ml = S::ldexp(Ml, kk);
+        Dl = S::ldexp(Dl, kk);
+        Mul = S::ldexp(Mul, kk);
+        Dul = S::ldexp(Dul, kk);
+        Iin = S::ldexp(Iin, kk);
+        acc = S::ldexp(acc, kk);
+        C0s = S::ldexp(C0s, kk);
+        sc -= kk;
+    };
+    auto fit = [&](int e_in) {
+        T my = fmax(fmax(fmax(Ml, Dl), fmax(Mul, Dul)), fmax(Iin, acc));
+#pragma unroll
+        for (int j = 0; j < NR; ++j)
+            my = fmax(my, fmax(M[j], D[j]));
+        const int e_my = my > (T)0 ? S::expo(my) : kNone;
+        const int e = e_in > e_my ? e_in : e_my;
+        if (e > kNone && (e > 96 || e < -32))
+            rescale(64 - e);
+    };
+    auto expo = [&](T v, int e) { return v > (T)0 ? S::expo(v) + e : kNone; };
+    // the letters of four columns at a time, the next four loaded ahead;
+    // columns outside the hap read as the wildcard
+    const uint32_t* hdw = reinterpret_cast<const uint32_t*>(p.hapc + (active ? bd.hap_off[it.hap] : 0));
+    const int hdw_last = HL >> 2;
+    const uint32_t shift = (uint32_t)(-t) & 3u;
+    auto hap_dword = [&](int q) { return hdw[min(max(q, 0), hdw_last)]; };
+    const int q0 = (0 - t) >> 2;
+    uint32_t wlo = hap_dword(q0), whi = hap_dword(q0 + 1), wnx = hap_dword(q0 + 2);
+    auto emission = [&](int c, uint32_t code, V (&lam)[NV]) {
+        const uint32_t letter = (uint32_t)c < (uint32_t)HL ? code & 7u : 4u;
+        const V* trow = tab + ((letter << 6) | lane);
+#pragma unroll
+        for (int q = 0; q < NV; ++q)
+            lam[q] = trow[q * (NL * 64)];
+    };
+    const int nsteps = wave_max(active ? HL + 64 : 0);
+    const int s_end = HL + 63;  // the last step of this alignment
+    V lam[2][NV];
+    uint32_t letters = __builtin_amdgcn_alignbyte(whi, wlo, shift);
+    emission(-t, letters, lam[0]);
+    for (int s4 = 0; s4 < nsteps; s4 += 4) {
+        const uint32_t next = __builtin_amdgcn_alignbyte(wnx, whi, shift);
+        wlo = whi;
+        whi = wnx;
+        wnx = hap_dword(((s4 - t) >> 2) + 3);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int s = s4 + u, c = s - t;
+            emission(c + 1, u < 3 ? letters >> (8 * (u + 1)) : next, lam[(u + 1) & 1]);
+            T mp = Mul, dp = Dul, chain = Iin;
+#pragma unroll
+            for (int q = 0; q < NV; ++q) {
+                T lv[K];
+                TileTraits<T>::unpack(lam[u & 1][q], lv);
+#pragma unroll
+                for (int x = 0; x < K; ++x) {
+                    const int j = K * q + x;
+                    const T mo = M[j], dov = D[j];
+                    M[j] = lv[x] * (ca[j] * mp + cb[j] * (chain + dp));
+                    chain = cdl[j] * mp + ce[j] * chain;
+                    D[j] = cs[j] * mo + ce[j] * dov;
+                    mp = mo;
+                    dp = dov;
+                }
+            }
+            if (t == tr && c >= 1 && c <= HL)
+                acc += chain;
+            const T sM = S::shr(M[NR - 1]), sD = S::shr(D[NR - 1]), sI = S::shr(chain);
+            const int ssc = shr1i(sc);
+            int e_in = kNone;
+            if (t != 0) {
+                e_in = expo(sM, ssc - sc);
+                const int e2 = expo(sD, ssc - sc), e3 = expo(sI, ssc - sc);
+                e_in = e2 > e_in ? e2 : e_in;
+                e_in = e3 > e_in ? e3 : e_in;
+            }
+            fit(e_in);
+            const int d = ssc - sc;
+            Mul = Ml;
+            Dul = Dl;
+            Ml = t == 0 ? (T)0 : S::ldexp(sM, d);
+            Dl = t == 0 ? C0s : S::ldexp(sD, d);
+            Iin = t == 0 ? (T)0 : S::ldexp(sI, d);
+            if (s == s_end) {
+                acc_end = acc;
+                sc_end = sc;
+            }
+        }
+        letters = next;
+    }
+    if (active && t == tr) {
+        const double lg = log10((double)acc_end) + (double)sc_end * 0.30102999566398119521 -
+                          log10((double)C0 * (double)HL);
+        bd.scores[it.out] = (float)lg;
+        const double lmin = log10((double)p.rescue_min) - (double)kLog10Scale;
+        if (sizeof(T) == 4 && p.rescue_on && !(acc_end > (T)0 && lg >= lmin && lg < 1e30))
+            p.final_items[atomicAdd(p.final_count, 1)] = it;
+    }
+}
 
 // The items are those of the BinSet, one wave each (blocks take every
 // gridDim-th item of the bins' concatenated item sequence).  `spill` holds
@@ -1110,7 +1350,8 @@ struct WaveScalar<double> {
 // T = float (multi-tile first pass) appends results below the rescue
 // threshold (as the tile kernels define it) to the final list, which the
 // T = double instance recomputes.
-template <typename T, int NR>
+// PACK (one bin): runs of items that pack_task takes go to it instead.
+template <typename T, int NR, bool PACK = false>
 __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const int32_t* hmax_ptr,
                                                  T* spill, int64_t spill_elems,
                                                  int32_t* error_flag)
@@ -1141,7 +1382,30 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
     // row; ex[2c] / ex[2c+1] the exponents M/D and I were stored with
     int32_t* ex = reinterpret_cast<int32_t*>(sp + 3 * (int64_t)(hmax + 1));
 
-    for (int w = blockIdx.x; w < n; w += nblk) {
+    // PACK: runs of three items (as many as fit side by side for reads of up
+    // to 167 bases at 8 rows per lane), shorter where the blocks outnumber them
+    const int run = PACK ? max(1, min(3, (n + nblk - 1) / nblk)) : 1;
+    for (int v = blockIdx.x * run; v < n; v += nblk * run)
+    for (int w = v; w < min(n, v + run); ++w) {
+        if constexpr (PACK) {
+            __shared__ typename TileTraits<T>::V tab[5 * (NR / TileTraits<T>::K) * 64];
+            const WorkItem* q = bs.items + __shfl(sl.begin, 0, 64) + w;
+            const int rem = min(n, v + run) - w;
+            int L = 0;
+            bool ok = true;
+            if (lane < rem) {
+                const int hl = bd.hap_len[q[lane].hap];
+                L = bd.read_len[q[lane].read];
+                ok = p.semantics == 0 && L > 0 && L < TR && hl > 0 && hl <= hmax;
+            }
+            if (!__ballot(!ok)) {
+                const int G = (wave_max(L) + NR) / NR;  // ceil((L + 1) / NR)
+                const int take = min(rem, 64 / G);
+                pack_task<T, NR>(p, tab, q, take, G);
+                w += take - 1;
+                continue;
+            }
+        }
         const int kb = set_find(sl, w);
         const int begin = __shfl(sl.begin, kb, 64);
         const int w0 = __shfl(sl.incl - sl.ntask, kb, 64);
@@ -1349,6 +1613,308 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
 }
 
 // ---------------------------------------------------------------------------
+// k_fwd_special
+// ---------------------------------------------------------------------------
+// What the tile bins cannot take: reads of several tiles (strips, on the
+// scaled tile sweep) and haps holding the wildcard.
+//
+// Strips: one wave per alignment, the read cut into tiles of 64 lanes x
+// kStripRows rows swept one after another.  A tile's last lane writes its
+// last row's (M, D, I) and its exponent per column to a border row in global
+// memory; the next tile's first lane takes them in instead of row 0.  It
+// scales like every other lane, so the values are put on its exponent as they
+// are read, 16 columns at a time between two checks (v_ldexp: exact unless a
+// value leaves the normal range, which the checks keep it from as they do
+// from lane to lane), through an LDS window that the other lanes read zeros
+// beside.  The border row is written 64 columns behind where it is read, so
+// the tiles of a read share one.  The emission table holds the wildcard as a
+// fifth letter.  Bound by the VALU like the tile kernels.  The one-wave
+// kernel, with 1024-row tiles, an exponent check of every row per column and
+// FP64 for what falls below the FP32 range, took 23.5 ms for 2,560 alignments
+// of 1100-1500-base reads with 1500-2000-base haps; the strips take 1.5 ms
+// (whole calls).  12 rows per lane waste less of the last tile than 16
+// (768-row steps instead of 1024).
+//
+// Wildcard haps: the one-wave kernel's arithmetic (its 64 steps past the hap
+// included; 177 of 908k scores differ, by at most 8e-6) with as many alignments side by side on the wave as
+// its lanes hold, the emission values from an LDS table of five letters
+// instead of compares, and the letters loaded four columns ahead.  The items
+// are sorted by (read class, hap length) and a wave takes a run of them.  908k
+// mixed alignments of which 5% have such a hap: 20.0 -> 7.2 ms per call.
+constexpr int kStripRows = 12;
+constexpr int kStripPad = 256;  // border entries beyond the longest hap
+// Long reads meet more of the steepest growths between two checks than the
+// tiles' reads do: the strips scale down from 2^40 (at 2^kDsGuard, 2 of 2,560
+// alignments overflowed and cost an FP64 pass of 3 ms).
+constexpr float kStripGuard = 0x1p40f;
+
+// One alignment on the whole wave.  win: 32 entries of LDS; border: the
+// block's border row.  Returns 1 when the sum fell below the rescue threshold
+// and was finished by the scaling.
+template <bool FAST>
+__device__ __forceinline__ int strip_task(const FwdParams& p, float4* tab, float4* win,
+                                          float4* border, const WorkItem& it)
+{
+    using TT = TileTraits<float>;
+    constexpr int NR = kStripRows, NL = 5, TR = 64 * NR;
+    using Shape = TabShape<float, NR, NL>;
+    constexpr int NV = Shape::NV;
+    static_assert(!Shape::kTail && NR % 4 == 0, "whole vectors");
+    const BatchDesc& bd = *p.bd;
+    const int t = threadIdx.x;
+    const bool first = t == 0;
+    const int L = bd.read_len[it.read], HL = bd.hap_len[it.hap];
+    const int ntiles = (L + TR) / TR;  // tiles of the read's rows and one more
+    const uint32_t* rw = p.rows + bd.read_off[it.read];
+    const uint32_t* hdw = reinterpret_cast<const uint32_t*>(p.hapc + bd.hap_off[it.hap]);
+    const int hdw_last = HL >> 2;
+    const uint32_t shift = (uint32_t)(-t) & 3u;
+    // letters past the hap read as base 0 (the wildcard, which every row
+    // matches, would let values grow there and scale the lanes down)
+    auto hap_dword = [&](int q) { return q > hdw_last ? 0u : hdw[max(q, 0)]; };
+    // this lane's view of the window: the first lane's columns, zeros for
+    // the others (in entries 16 ..)
+    if (t >= 16 && t < 32)
+        win[t] = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4* seen = win + (first ? 0 : 16);
+
+    TileRead<float, NR, false> R;
+    float acc = 0.f, C0 = 0.f;
+    int E = 0;
+    bool bad = false;
+    for (int k = 0; k < ntiles; ++k) {
+        const int row0 = k * TR;
+        const bool top = k == 0, last = k == ntiles - 1;
+        tile_setup<float, NR, FAST, false, NL>(p, tab, true, it.read, t, R, row0);
+        C0 = FAST ? (kScale / (float)HL) * (R.nl * (1.0f / kFastKappa)) : kScale / (float)HL;
+        // exponents: the insertion floor of the lane's last row, none for the
+        // read's first lane
+        int x = 0;
+        if (!(top && first))
+            x = ds_start<FAST>(p, C0, R.eps, min(row0 + (t + 1) * NR, L) - 1, rw);
+        if (__ballot(!first && x - ds_above(x) > kDsSpan))
+            x = ds_span_cap(x, t);
+        E = x;
+        auto factor = [&]() {
+            const int d = E - ds_above(E);
+            return first ? 0.f : ldexpf(1.0f, d);
+        };
+        float nf = factor();
+        bool any = __ballot(E > 0) != 0;
+
+        // border columns c0 .. c0+15 (lanes 0-15), raw and on the first
+        // lane's exponent; row 0 has D = C0 in every column
+        auto fetch = [&](int c0) {
+            return top || t >= 16 ? make_float4(0.f, C0, 0.f, 0.f) : border[64 + c0 + t];
+        };
+        auto scaled = [&](const float4& r, int c) {
+            if (top)
+                return r;
+            const int sh = __builtin_amdgcn_readfirstlane(E) - __float_as_int(r.w);
+            // column HL still carries the chain of the last one (a row's chain
+            // runs one column behind); past it nothing was written
+            const bool in = c <= HL;
+            return make_float4(in ? ldexpf(r.x, sh) : 0.f, in ? ldexpf(r.y, sh) : 0.f,
+                               in ? ldexpf(r.z, sh) : 0.f, 0.f);
+        };
+        TT::P MD[NR], MDr[2];
+#pragma unroll
+        for (int j = 0; j < NR; ++j)
+            MD[j] = 0.f;
+        // before step 0 the first lane holds the row above at columns -1 (row
+        // 0 only) and 0
+        const float4 raw0 = fetch(0);
+        const float4 b0 = scaled(raw0, t);
+        MDr[0].x = 0.f;
+        MDr[0].y = first && top ? C0 : 0.f;
+        MDr[1].x = first ? b0.x : 0.f;
+        MDr[1].y = first ? b0.y : 0.f;
+        float Iin = first ? b0.z : 0.f;
+        float4 raw = fetch(1);
+        acc = 0.f;
+        const int res_t = last ? (L - row0) / NR : 63;
+        const int nsteps = HL + res_t + 1;
+        const int acc_last = t + HL;
+
+        const int q0 = (0 - t) >> 2;
+        uint32_t wlo = hap_dword(q0), whi = hap_dword(q0 + 1), wnx = hap_dword(q0 + 2);
+        uint32_t letters = __builtin_amdgcn_alignbyte(whi, wlo, shift);
+        float4 lam[2][NV];
+#pragma unroll
+        for (int q = 0; q < NV; ++q)
+            lam[0][q] = (tab + (((letters & 7u) << 6) | t))[q * (NL * 64)];
+        auto sweep4 = [&](int s4, int w4, bool bounded) {
+            const uint32_t next = __builtin_amdgcn_alignbyte(wnx, whi, shift);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int cur = u & 1, nxt = cur ^ 1;
+                const uint32_t nletter = u < 3 ? (letters >> (8 * (u + 1))) & 7u : next & 7u;
+                const float4* trow = tab + ((nletter << 6) | t);
+#pragma unroll
+                for (int q = 0; q < NV; ++q)
+                    lam[nxt][q] = trow[q * (NL * 64)];
+                const float4 in = seen[w4 + u];  // the row above at column s + 1
+                TT::P up = MDr[cur];
+                float chain = Iin;
+#pragma unroll
+                for (int q = 0; q < NV; ++q) {
+                    float lv[4];
+                    TT::unpack(lam[cur][q], lv);
+#pragma unroll
+                    for (int x4 = 0; x4 < 4; ++x4)
+                        tile_cell<float, NR, FAST, false>(R, 4 * q + x4, lv[x4], R.eps,
+                                                          MD[4 * q + x4], up, chain);
+                }
+                if (bounded)
+                    acc += (s4 + u <= acc_last) ? chain : 0.f;
+                else
+                    acc += chain;
+                if (!last && t == 63)  // column s - 63
+                    border[s4 + u + 1] =
+                        make_float4(MD[NR - 1].x, MD[NR - 1].y, chain, __int_as_float(E));
+                __builtin_amdgcn_s_setprio(3);  // as in tile_sweep
+                MDr[cur].x = fmaf(shr1f(MD[NR - 1].x), nf, in.x);
+                MDr[cur].y = fmaf(shr1f(MD[NR - 1].y), nf, in.y);
+                Iin = fmaf(shr1f(chain), nf, in.z);
+                TT::pin(MDr[cur]);
+                __builtin_amdgcn_s_setprio(0);
+            }
+            letters = next;
+            wlo = whi;
+            whi = wnx;
+            wnx = hap_dword(((s4 - t) >> 2) + 3);
+        };
+        for (int s0 = 0; s0 < nsteps; s0 += 16) {
+            // columns s0+1 .. s0+16 for the steps below; the next 16 are
+            // fetched over them
+            const float4 v = scaled(raw, s0 + 1 + t);
+            if (t < 16)
+                win[t] = v;
+            __builtin_amdgcn_wave_barrier();
+            raw = fetch(s0 + 17);
+            if (s0 + 16 <= HL + 1) {
+                for (int w4 = 0; w4 < 16; w4 += 4)
+                    sweep4(s0 + w4, w4, false);
+            } else {
+                for (int w4 = 0; w4 < 16; w4 += 4)
+                    sweep4(s0 + w4, w4, true);
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (any) {
+                const float m = fmaxf(fmaxf(fmaxf(MDr[0].x, MDr[1].x), fmaxf(MDr[0].y, MDr[1].y)), Iin);
+                x = ds_lowered(E, m, kStripGuard);
+                if (__ballot(x != E)) {
+                    if (__ballot(!first && x - ds_above(x) > kDsSpan))
+                        x = ds_span_cap(x, t);
+                    const int S = x - E;
+#pragma unroll
+                    for (int j = 0; j < NR; ++j) {
+                        MD[j].x = ldexpf(MD[j].x, S);
+                        MD[j].y = ldexpf(MD[j].y, S);
+                    }
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        MDr[u].x = ldexpf(MDr[u].x, S);
+                        MDr[u].y = ldexpf(MDr[u].y, S);
+                    }
+                    Iin = ldexpf(Iin, S);
+                    acc = ldexpf(acc, S);
+                    E = x;
+                    nf = factor();
+                    any = __ballot(E > 0) != 0;
+                }
+            }
+        }
+        const int dl = E - ds_above(E);
+        if (t <= res_t)
+            bad = bad || (E > 0 && !(acc <= 3.4028234663852886e38f)) ||
+                  (t >= 1 && (dl > 127 || dl < -126));
+        __syncthreads();  // the border row is visible to the next tile
+    }
+    const bool ok = __ballot(bad) == 0;
+    bool done = false;
+    if (t == (L - (ntiles - 1) * TR) / NR) {
+        if (ok && acc >= 0x1p-100f && acc <= 3.4028234663852886e38f) {
+            // acc * 2^-E in the start constant's units
+            int e2 = 0;
+            const double m = (double)frexpf(acc, &e2);
+            bd.scores[it.out] = (float)(log10(FAST ? m * (double)kFastKappa : m / (double)R.beta) +
+                                        (double)(e2 - E) * 0.30102999566398119521 - kLog10ScaleD);
+            done = !(ldexpf(FAST ? acc * R.nl : acc / R.beta, -E) >= p.rescue_min);
+        } else {
+            bd.scores[it.out] = -INFINITY;
+            p.final_items[atomicAdd(p.final_count, 1)] = it;
+        }
+    }
+    return __ballot(done) ? 1 : 0;
+}
+
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_fwd_special(
+    FwdParams p, SpecialSet ss)
+{
+    constexpr int kTab = TabShape<float, kWildRows, 5>::kWords;
+    static_assert(TabShape<float, kStripRows, 5>::kWords + 32 <= kTab, "the window beside the table");
+    __shared__ float4 tab[kTab];
+    const BatchDesc& bd = *p.bd;
+    const int nm = ss.range[2 * ss.strip_bin + 1], nw = ss.range[2 * ss.wild_bin + 1];
+    if (nm + nw == 0)
+        return;
+    const WorkItem* strips = ss.items + ss.range[2 * ss.strip_bin];
+    const WorkItem* wilds = ss.items + ss.range[2 * ss.wild_bin];
+    float4* border = ss.border;
+    if (nm > 0) {  // a border row per block, for as many blocks as the arena holds
+        const int64_t stride = (int64_t)*ss.hmax + kStripPad;
+        const int64_t cap = ss.border_entries / stride;
+        if ((int64_t)blockIdx.x >= cap) {
+            if (blockIdx.x == 0 && threadIdx.x == 0)
+                atomicOr(ss.error_flag, 1);
+            return;
+        }
+        border += blockIdx.x * stride;
+    }
+    // a run of items per task: 12 or 24 fill whole waves for most reads (4, 6
+    // or 12 side by side); the longer run where every wave gets several, the
+    // shorter (or, for few items, 4) to spread them over the device
+    const int per_wave = nw / (int)gridDim.x;
+    const int run = per_wave >= 72 ? 24 : per_wave >= 4 ? 12 : 4;
+    const int total = nm + (nw + run - 1) / run;
+    int done = 0;
+    for (int task = next_task(ss.next_task); task < total; task = next_task(ss.next_task)) {
+        task = __builtin_amdgcn_readfirstlane(task);
+        if (task < nm) {
+            const WorkItem it = strips[task];
+            float4* win = tab + TabShape<float, kStripRows, 5>::kWords;
+            const ReadMeta m = p.meta[it.read];
+            const bool fast = m.bin == ss.strip_bin ? m.nl > 0.f : (m.bin & 1) == 0;
+            done += fast ? strip_task<true>(p, tab, win, border, it)
+                         : strip_task<false>(p, tab, win, border, it);
+            continue;
+        }
+        int i = (task - nm) * run;
+        const int end = min(i + run, nw);
+        while (i < end) {  // as many of the next items as fit side by side
+            const int n = end - i;  // at most 24: one lane each
+            const int L = (int)threadIdx.x < n ? bd.read_len[wilds[i + threadIdx.x].read] : 0;
+            const int G = (wave_max(L) + kWildRows) / kWildRows;  // ceil((L + 1) / rows)
+            const int take = min(n, 64 / G);
+            pack_task<float, kWildRows>(p, tab, wilds + i, take, G);
+            i += take;
+        }
+    }
+    if (done > 0 && threadIdx.x == 0)
+        atomicAdd(p.scaled_total, (unsigned long long)done);
+}
+
+hipError_t launch_fwd_special(const FwdParams& p, const SpecialSet& ss, int grid, hipStream_t st)
+{
+    if (!p.scaled_total || !p.rescue_on || !ss.items || !ss.range || !ss.next_task || !ss.hmax ||
+        !ss.border || !ss.error_flag || grid <= 0)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_fwd_special, dim3(grid), dim3(64), 0, st, p, ss);
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------
 // launchers
 // ---------------------------------------------------------------------------
 template <typename K>
@@ -1543,8 +2109,12 @@ hipError_t launch_fwd_wave_f64(const FwdParams& p, const BinSet& bs, const int32
 {
     if (bs.n < 1 || bs.n > 64 || !bs.counts || !bs.items || blocks <= 0)
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_fwd_wave<double, 8>), dim3(blocks), dim3(64), 0, st, p, bs, hmax_ptr,
-                       spill, spill_elems, error_flag);
+    if (bs.n == 1)
+        hipLaunchKernelGGL((k_fwd_wave<double, 8, true>), dim3(blocks), dim3(64), 0, st, p, bs,
+                           hmax_ptr, spill, spill_elems, error_flag);
+    else
+        hipLaunchKernelGGL((k_fwd_wave<double, 8>), dim3(blocks), dim3(64), 0, st, p, bs, hmax_ptr,
+                           spill, spill_elems, error_flag);
     return hipGetLastError();
 }
 

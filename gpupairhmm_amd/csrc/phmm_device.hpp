@@ -36,6 +36,7 @@ struct __attribute__((aligned(16))) SuperTask {
 constexpr float kScale = 2.1267646664908054e37f;  // FLT_MAX / 16 (exact)
 constexpr float kLog10Scale = 37.3277194f;      // log10(FLT_MAX / 16)
 constexpr double kScaleD = 2.1267646664908054e37;
+constexpr double kLog10ScaleD = 37.327719436447699;  // the same in double
 
 // Headroom divisor of the rescaled kernel's start constant (see
 // k_fwd_tile_set): every rescaled cell stays below FLT_MAX/16.
@@ -48,10 +49,11 @@ constexpr double kStartF64 = 0x1p1000;
 constexpr double kLog10StartF64 = 301.02999566398120;  // 1000 * log10(2)
 
 constexpr int kMaxTiles = 32;
-// Bins: 2 per tile class (FAST, SAFE), the multi-tile bin, and the exact
-// bin (haps with a byte other than A/C/G/T; under reference CPU semantics
-// also reads with a byte other than A/C/G/T/N).
-constexpr int kMaxBins = 2 * kMaxTiles + 2;
+// Bins: 2 per tile class (FAST, SAFE), the multi-tile bin (reads longer than
+// the largest tile), the exact bin (reads and haps with a byte that matches
+// nothing but itself: reference CPU semantics only) and the wildcard bin
+// (tile reads against haps holding the wildcard).
+constexpr int kMaxBins = 2 * kMaxTiles + 3;
 // Work bins: the bins above, then one item bin per tile bin (the alignments
 // of a record's reads left over after full chunks of 64/lanes reads).
 constexpr int kMaxWorkBins = kMaxBins + 2 * kMaxTiles;
@@ -79,6 +81,15 @@ __host__ __device__ inline int hap_bucket(int h)
         return h < 0 ? 0 : h;
     int b = 2048 + ((h - 2048) >> 4);
     return b < kHapBuckets - 1 ? b : kHapBuckets - 1;
+}
+
+// The wildcard bin's sort key, which takes the hap length's place: the read's
+// tile bin k (class and form), then the hap length in steps of 32.
+constexpr int kWildLens = kHapBuckets / (2 * kMaxTiles);
+__host__ __device__ inline int wild_bucket(int k, int h)
+{
+    const int q = h >> 5;
+    return k * kWildLens + (q < kWildLens - 1 ? q : kWildLens - 1);
 }
 
 // Gap-continuation constants of the reference GPU kernel
@@ -113,7 +124,8 @@ __host__ __device__ inline int base_code_sem(uint8_t b, int semantics)
 // Per-read metadata from the read pass.
 struct __attribute__((aligned(8))) ReadMeta {
     int32_t bin;     // work-list bin; -1: empty read
-    float nl;        // product of alpha over the read (rescaled kernel)
+    float nl;        // product of alpha over the read (rescaled form); -1: a
+                     // read of several tiles that the rescaled form does not admit
 };
 
 // The per-call part of a batch: device pointers of a self-contained batch
@@ -148,7 +160,7 @@ struct FwdParams {
     const uint8_t* hapc;         // hap base codes, indexed like hap bytes
     const ReadMeta* meta;
     const int32_t* read_perm;    // reads of each record ordered by bin
-    const uint8_t* hapflag;      // 1: the hap holds a byte other than A/C/G/T (exact bin)
+    const uint8_t* hapflag;      // per hap: 0 A/C/G/T only, 1 the wildcard too, 2 other bytes
     const float* ph2pr;          // 128 entries
     WorkItem* rescue_items;      // per tile bin: alignments to recompute in FP64
     int32_t* rescue_counts;      // per bin
@@ -242,7 +254,7 @@ constexpr int kDsGuardTo = 0;
 // Everything the binning kernels read and write (binning.hip).
 struct BinParams {
     const BatchDesc* bd;
-    int32_t NB;                // bins of reads: 2*ntiles + 2
+    int32_t NB;                // bins of alignments: 2*ntiles + 3
     int32_t NW;                // work bins: NB + 2*ntiles (item bin of tile bin k: NB + k)
     // scratch
     uint32_t* rows;
@@ -265,7 +277,7 @@ struct BinParams {
     SuperTask* st;             // tile bins' work, in bin_range units
     int32_t* align_range;      // [2*NB]: per bin, begin / count in alignments
     int32_t* align_part;       // [NB*kAlignParts]: partial alignment counts per bin (k_scan_keys sums each bin's into its first)
-    uint8_t* hapflag;          // [nH]: 1 = hap holds a byte other than A/C/G/T
+    uint8_t* hapflag;          // [nH]: 0 A/C/G/T only, 1 the wildcard too, 2 other bytes
     WorkItem* items;
     const float* ph2pr;
     // tiles
@@ -343,6 +355,20 @@ hipError_t launch_fwd_tile_set_re(int NR, bool fast, const FwdParams& p, const B
 // tile_re_supported; not under per-position gcp).
 hipError_t launch_fwd_tile_set_scaled(int NR, bool fast, const FwdParams& p, const BinSet& bs,
                                       int grid, hipStream_t st);
+// Rows per lane of the wildcard tiles.
+constexpr int kWildRows = 16;
+// The multi-tile and wildcard bins on the scaled sweep (k_fwd_special).
+struct SpecialSet {
+    const WorkItem* items = nullptr;
+    const int32_t* range = nullptr;  // bin_range
+    int32_t strip_bin = 0, wild_bin = 0;
+    int32_t* next_task = nullptr;
+    const int32_t* hmax = nullptr;
+    float4* border = nullptr;        // border rows of the strips, one per block
+    int64_t border_entries = 0;
+    int32_t* error_flag = nullptr;
+};
+hipError_t launch_fwd_special(const FwdParams& p, const SpecialSet& ss, int grid, hipStream_t st);
 hipError_t launch_fwd_wave_f32(const FwdParams& p, const BinSet& bs, const int32_t* hmax_ptr,
                                float* spill, int64_t spill_elems, int32_t* error_flag, int blocks,
                                hipStream_t st);
