@@ -175,6 +175,13 @@ struct TileRead {
     T eps, beta;
     int L;
     float nl;
+    // log2 of the insertion floor at the lane's last row (the read's last row
+    // for the lanes past it), less the start constant's: the product of the
+    // rows' chain coefficients, which telescopes -- FAST: eps^R * delta_0 /
+    // delta_R / prod(alpha_0 .. alpha_{R-1}); SAFE: eps per row.  The alpha
+    // factors (each <= 1) are left out, which can only put the estimate below
+    // the true floor.  (In-pass scaling; one gap continuation per read.)
+    float floor2;
 };
 
 // Gap continuation of the D chain of row j.
@@ -242,81 +249,89 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
     R.beta = beta;
     R.L = L;
     R.nl = nl;
-    // per-position gcp: eps and beta of row index ri (0-based, < L)
-    auto row_eps = [&](int ri) -> T { return (T)ph2pr_of(p.ph2pr, bd.gcp[roff + ri]); };
 
     // ---- per-row coefficients and the emission table -------------------
+    // No branch per row: all of a lane's rows are loaded at once (rows past
+    // the read repeat its last one and are selected away), then all their
+    // table entries, so that a setup waits twice for memory and not twice per
+    // row: 4.56 -> 4.47 ms per call of 10,000 records x 25 reads of 150 bases x
+    // 4 haps, with the next hap's loads ahead of a super-task's sweep and the
+    // descriptor's pointers in registers.
     const int r0 = row0 + t * NR;
     {
-        T pdelta = 0, psigma = 0, palpha = 1;
-        if (r0 >= 1 && r0 - 1 < L) {
-            const uint32_t w = p.rows[roff + r0 - 1];
-            pdelta = (T)ph2pr_of(p.ph2pr, row_iq(w));
-            psigma = (T)ph2pr_of(p.ph2pr, row_dq(w));
-            palpha = (T)1 - (pdelta + psigma);
+        const int rlast = L > 0 ? L - 1 : 0;
+        uint32_t w[NR], wp;
+        uint8_t g[ROWEPS ? NR + 1 : 1];
+        wp = p.rows[roff + min(max(r0 - 1, 0), rlast)];
+#pragma unroll
+        for (int j = 0; j < NR; ++j)
+            w[j] = p.rows[roff + min(r0 + j, rlast)];
+        if constexpr (ROWEPS) {
+#pragma unroll
+            for (int j = 0; j <= NR; ++j)
+                g[j] = bd.gcp[roff + min(r0 + j, rlast)];
         }
+        T pb[NR], de[NR], si[NR], er[ROWEPS ? NR + 1 : 1];
+#pragma unroll
+        for (int j = 0; j < NR; ++j) {  // (the packed rows' qualities are at most 127)
+            pb[j] = (T)p.ph2pr[row_bq(w[j])];
+            de[j] = (T)p.ph2pr[row_iq(w[j])];
+            si[j] = (T)p.ph2pr[row_dq(w[j])];
+        }
+        // the row above the lane's first one
+        const bool above = r0 >= 1 && r0 - 1 < L;
+        T pdelta = above ? (T)p.ph2pr[row_iq(wp)] : (T)0;
+        T psigma = above ? (T)p.ph2pr[row_dq(wp)] : (T)0;
+        T palpha = above ? (T)1 - (pdelta + psigma) : (T)1;
+        if constexpr (ROWEPS) {
+#pragma unroll
+            for (int j = 0; j <= NR; ++j)
+                er[j] = (T)ph2pr_of(p.ph2pr, g[j]);
+        }
+        // (the clamped loads leave row min(r0 + NR, L) - 1 in w[NR - 1])
+        const int lrow = min(r0 + NR, L) - 1;
+        R.floor2 = (float)lrow * __log2f((float)eps);
+        if (FAST && lrow > 0)
+            R.floor2 += __log2f(p.ph2pr[row_iq(p.rows[roff])]) - __log2f((float)de[NR - 1]);
         T lm[NR], lx[NR];
         int code[NR];
 #pragma unroll
         for (int j = 0; j < NR; ++j) {
             const int ri = r0 + j;  // 0-based row; 1-based row ri+1
-            if (ri < L) {
-                const uint32_t w = p.rows[roff + ri];
-                const T pb = (T)ph2pr_of(p.ph2pr, row_bq(w));
-                const T delta = (T)ph2pr_of(p.ph2pr, row_iq(w));
-                const T sigma = (T)ph2pr_of(p.ph2pr, row_dq(w));
-                const T alpha = (T)1 - (delta + sigma);
-                // gap continuation of this row, and (SAFE) the next row's beta
-                T er = eps, br = beta, bn = beta;
-                if constexpr (ROWEPS) {
-                    er = row_eps(ri);
-                    br = beta_of(er);
-                    bn = ri + 1 < L ? beta_of(row_eps(ri + 1)) : beta;
-                }
-                code[j] = row_code(w);
-                lm[j] = (T)1 - pb;
-                lx[j] = qdiv(pb, (T)3);
-                if (FAST) {
-                    if (ri == 0) {
-                        R.c10[j].y = 0;
-                        R.c10[j].x = qdiv(br, alpha);
-                        R.c32[j].y = 0;
-                    } else {
-                        R.c10[j].y = qdiv(br * pdelta, palpha * alpha);
-                        R.c10[j].x = qdiv(br * psigma, alpha);
-                        R.c32[j].y = qdiv(er * pdelta, delta * palpha);
-                    }
-                    R.c32[j].x = ROWEPS ? er : (T)0;
-                } else {
-                    R.c10[j].y = alpha;
-                    R.c10[j].x = ri == 0 ? br : br * psigma;
-                    R.c32[j].y = bn * delta;
-                    // equal betas keep eps exactly (no rounding of bn / br)
-                    R.c32[j].x = bn == br ? er : qdiv(er * bn, br);
-                    if constexpr (ROWEPS)
-                        R.c4[j] = er;
-                }
+            const bool in = ri < L, top = ri == 0, firstoob = ri == L;
+            const T delta = de[j], sigma = si[j];
+            const T alpha = (T)1 - (delta + sigma);
+            // gap continuation of this row, and (SAFE) the next row's beta
+            T e = eps, br = beta, bn = beta;
+            if constexpr (ROWEPS) {
+                e = er[j];
+                br = beta_of(e);
+                bn = ri + 1 < L ? beta_of(er[j + 1]) : beta;
+            }
+            code[j] = in ? row_code(w[j]) : 4;
+            lm[j] = in ? (T)1 - pb[j] : (T)0;
+            lx[j] = in ? qdiv(pb[j], (T)3) : (T)0;
+            if (FAST) {
+                const T c0 = qdiv(br * pdelta, palpha * alpha);
+                const T c1 = qdiv(top ? br : br * psigma, alpha);
+                const T c2 = qdiv(in ? e * pdelta : pdelta, in ? delta * palpha : palpha);
+                R.c10[j].y = in && !top ? c0 : (T)0;
+                R.c10[j].x = in ? c1 : (T)0;
+                R.c32[j].y = in ? (top ? (T)0 : c2) : firstoob ? c2 : (T)1;
+                R.c32[j].x = ROWEPS && in ? e : (T)0;
+            } else {
+                R.c10[j].y = in ? alpha : (T)0;
+                R.c10[j].x = in ? (top ? br : br * psigma) : (T)0;
+                R.c32[j].y = in ? bn * delta : firstoob ? beta : (T)0;
+                // equal betas keep eps exactly (no rounding of bn / br)
+                R.c32[j].x = in ? (bn == br ? e : qdiv(e * bn, br)) : (T)1;
+                if constexpr (ROWEPS)
+                    R.c4[j] = in ? e : (T)0;
+            }
+            if (in) {  // rows past the read keep the last row's values
                 pdelta = delta;
                 psigma = sigma;
                 palpha = alpha;
-            } else {
-                code[j] = 4;
-                lm[j] = 0;
-                lx[j] = 0;
-                const bool firstoob = (ri == L);
-                if (FAST) {
-                    R.c10[j].y = 0;
-                    R.c10[j].x = 0;
-                    R.c32[j].y = firstoob ? qdiv(pdelta, palpha) : (T)1;
-                    R.c32[j].x = 0;
-                } else {
-                    R.c10[j].y = 0;
-                    R.c10[j].x = 0;
-                    R.c32[j].y = firstoob ? beta : (T)0;
-                    R.c32[j].x = 1;
-                    if constexpr (ROWEPS)
-                        R.c4[j] = 0;
-                }
             }
         }
         // emission table: tab[(q*NL + letter)*64 + lane] = rows K*q .. K*q+K-1
@@ -418,22 +433,11 @@ __device__ __forceinline__ int ds_span_cap(int x, int t)
     }
     return z + kDsSpan * t;
 }
-// The exponent a lane starts with, from the insertion floor at row index
-// `last` of a read whose packed rows start at rw: the product of the rows'
-// chain coefficients down to that row, which telescopes -- FAST: eps^R *
-// delta_0 / delta_R / prod(alpha_0 .. alpha_{R-1}); SAFE: eps per row.  The
-// alpha factors (each <= 1) are left out, which can only put the estimate
-// below the true floor.  No lane exchange needed.
-template <bool FAST>
-__device__ __forceinline__ int ds_start(const FwdParams& p, float C0, float eps, int last,
-                                        const uint32_t* rw)
+// The exponent a lane starts with: its insertion floor (R.floor2) at
+// 2^kDsFloor.
+__device__ __forceinline__ int ds_start(float C0, float floor2)
 {
-    float fl = __log2f(C0) + (float)last * __log2f(eps);
-    if (FAST && last > 0)
-        fl += __log2f(ph2pr_of(p.ph2pr, row_iq(rw[0]))) -
-              __log2f(ph2pr_of(p.ph2pr, row_iq(rw[last])));
-    // the floor of the row at 2^kDsFloor
-    const int e0 = (int)floorf((float)kDsFloor - fl);
+    const int e0 = (int)floorf((float)kDsFloor - (__log2f(C0) + floor2));
     return e0 < 0 ? 0 : e0;
 }
 // The exponent of a lane with exponent E that holds or took in values up to
@@ -527,8 +531,10 @@ __device__ __forceinline__ bool f32_finish(const FwdParams& p, const WorkItem& i
 // kEpsGpu for every read: the D chain's multiplier is then wave-uniform and
 // sits in a scalar register, so those FMAs read two vector operands, not
 // three (about 1.4% of the sweep's time on gfx950).
+// ONE: every group sweeps the same hap (a super-task), so its length needs no
+// reduction over the wave.
 template <typename T, int NR, bool FAST, bool ROWEPS, bool RE = false, bool DS = false,
-          bool GE = false>
+          bool GE = false, bool ONE = false>
 __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename TileTraits<T>::V* tab,
                                           const TileRead<T, NR, ROWEPS>& R, bool active, int G,
                                           int t, int HL, int hoff, const WorkItem& it,
@@ -627,8 +633,7 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
         // lanes past it); a group's first lane is not scaled
         int x = 0;
         if (active && C0 > 0 && L > 0 && !first)
-            x = ds_start<FAST>(p, (float)C0, (float)R.eps, min((t + 1) * NR, L) - 1,
-                               p.rows + bd.read_off[it.read]);
+            x = ds_start((float)C0, R.floor2);
         if (__ballot(!first && x - ds_above(x) > kDsSpan))  // steep gap scores only
             x = ds_span_cap(x, t);
         ds_E = x;
@@ -645,7 +650,7 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
     T Iin = 0;
     T acc = 0;
 
-    const int Hmax = wave_max(HL);
+    const int Hmax = ONE ? __builtin_amdgcn_readfirstlane(HL) : wave_max(HL);
     const int nsteps = Hmax + G;
     // Hap letters: lane t consumes column c = s - t at step s.  Each lane
     // keeps a window of two dwords of its hap codes and shifts it by
@@ -664,7 +669,7 @@ __device__ __forceinline__ int tile_sweep(const FwdParams& p, const typename Til
     // s <= t + HL, needs a bound: steps below the wave's smallest HL add
     // unconditionally, the rest compare.
     const int acc_last = t + HL;
-    const int n_free = wave_min(active ? HL : nsteps) + 1;  // steps s < n_free
+    const int n_free = (ONE ? Hmax : wave_min(active ? HL : nsteps)) + 1;  // steps s < n_free
     const uint32_t lane_off = lane;  // tab index of this lane's letter-0 entry
 
     // emission values of step 0; each step loads the next step's values
@@ -979,19 +984,26 @@ __device__ __forceinline__ int tile_super_task(const FwdParams& p, typename Tile
     TileRead<T, NR, ROWEPS> R;
     tile_setup<T, NR, FAST, ROWEPS>(p, tab, active, rd, t, R);
     int done = 0;
+    // the next hap's length, offset and flag are loaded before a sweep
+    int hl_next = bd.hap_len[st.h0 + st.hs], off_next = bd.hap_off[st.h0 + st.hs];
+    int flag_next = p.hapflag[st.h0 + st.hs];
     for (int h = st.hs; h < st.he; ++h) {
         const int hap = st.h0 + h;
-        const int HL = bd.hap_len[hap];
-        if (HL <= 0 || p.hapflag[hap] != 0)
+        const int HL = hl_next, hoff = off_next, flag = flag_next;
+        if (h + 1 < st.he) {
+            hl_next = bd.hap_len[hap + 1];
+            off_next = bd.hap_off[hap + 1];
+            flag_next = p.hapflag[hap + 1];
+        }
+        if (HL <= 0 || flag != 0)
             continue;
         WorkItem it;
         it.read = rd;
         it.hap = hap;
         it.out = st.aoff + (rd - st.r0) * st.nh + h;
         it.pad = 0;
-        done += tile_sweep<T, NR, FAST, ROWEPS, false, DS, GE>(p, tab, R, active, G, t, HL,
-                                                              bd.hap_off[hap], it, rescue_base,
-                                                              bin);
+        done += tile_sweep<T, NR, FAST, ROWEPS, false, DS, GE, true>(p, tab, R, active, G, t, HL, hoff, it,
+                                                              rescue_base, bin);
     }
     return done;
 }
@@ -1110,6 +1122,10 @@ __attribute__((amdgpu_waves_per_eu(tile_waves_per_simd<T, NR, FAST, RE, DS>(), 8
     const int total = set_lanes(bs, 0, sl);
     if (total == 0)  // empty bins (common in a persistent launch): no atomic traffic
         return;
+    // the descriptor's pointers in registers: behind p.bd every use of one in
+    // a task would wait for the pointer first
+    const BatchDesc bd = *p.bd;
+    p.bd = &bd;
     // DS: alignments finished by the scaling below the threshold.  The
     // scaled instances (the default FP32 pass) carry a copy of the sweep
     // for the reference GPU semantics, whose eps is one constant.
@@ -1665,7 +1681,6 @@ __device__ __forceinline__ int strip_task(const FwdParams& p, float4* tab, float
     const bool first = t == 0;
     const int L = bd.read_len[it.read], HL = bd.hap_len[it.hap];
     const int ntiles = (L + TR) / TR;  // tiles of the read's rows and one more
-    const uint32_t* rw = p.rows + bd.read_off[it.read];
     const uint32_t* hdw = reinterpret_cast<const uint32_t*>(p.hapc + bd.hap_off[it.hap]);
     const int hdw_last = HL >> 2;
     const uint32_t shift = (uint32_t)(-t) & 3u;
@@ -1691,7 +1706,7 @@ __device__ __forceinline__ int strip_task(const FwdParams& p, float4* tab, float
         // read's first lane
         int x = 0;
         if (!(top && first))
-            x = ds_start<FAST>(p, C0, R.eps, min(row0 + (t + 1) * NR, L) - 1, rw);
+            x = ds_start(C0, R.floor2);
         if (__ballot(!first && x - ds_above(x) > kDsSpan))
             x = ds_span_cap(x, t);
         E = x;
@@ -1793,6 +1808,7 @@ __device__ __forceinline__ int strip_task(const FwdParams& p, float4* tab, float
             __builtin_amdgcn_wave_barrier();
             raw = fetch(s0 + 17);
             if (s0 + 16 <= HL + 1) {
+#pragma unroll
                 for (int w4 = 0; w4 < 16; w4 += 4)
                     sweep4(s0 + w4, w4, false);
             } else {
