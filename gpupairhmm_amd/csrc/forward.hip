@@ -1052,13 +1052,34 @@ __device__ __forceinline__ int set_find(const SetLane& s, int task)
     return __ffsll((long long)m) - 1;
 }
 
-// Next task of a wave from the launch's counter (one atomic per task).
-__device__ __forceinline__ int next_task(int32_t* ctr)
+// Tasks of a persistent launch.  2048 waves that all take their first task
+// from the launch's counter stand in line for it: the last one starts 20 us
+// after the first.  So with few tasks per block, block b starts on task b and
+// only later tasks come from the counter, and a launch of no more tasks than
+// blocks touches none: 250 reads against 32 haps 244.9 -> 226.4 us, 1000
+// records of 8 x 4 316.6 -> 299.6 us.  With many, the blocks start on the last
+// tasks instead and then take the others from the first on: tasks come largest
+// first, and a block that becomes resident late, behind another launch's
+// blocks, then holds back a small one (1000 records of up to 500 reads of 30 to
+// 250 bases: 42970 us all from the counter, 43814 from the front, 42357 from
+// the end).  In between neither holds: from the end, large tasks start too late
+// (400 records of 16 x 8 with 2-5 kb haps: 5417 us, 5312 from the counter), and
+// from the front they are held back (300 records of the mixed batch: 13290 us,
+// 13100 from the counter).
+constexpr int kFrontRounds = 4, kTailRounds = 8;  // tasks per block
+__device__ __forceinline__ int next_task(int32_t* ctr, int total, bool first)
 {
+    const int blocks = gridDim.x;
+    const bool front = total < kFrontRounds * blocks, tail = total >= kTailRounds * blocks;
+    if (first && (front || tail))
+        return tail ? total - 1 - (int)blockIdx.x : (int)blockIdx.x;
+    if (total <= blocks)
+        return total;
     int t = 0;
     if (threadIdx.x == 0)
         t = atomicAdd(ctr, 1);
-    return __shfl(t, 0, 64);
+    t = __shfl(t, 0, 64) + (front ? blocks : 0);
+    return tail && t >= total - blocks ? total : t;
 }
 
 // Bins of one template in one persistent launch.  Waves take tasks in order
@@ -1086,7 +1107,8 @@ __device__ __forceinline__ int tile_set_tasks(const FwdParams& p, const BinSet& 
                                               int total)
 {
     int done = 0;
-    for (int task = next_task(bs.next_task); task < total; task = next_task(bs.next_task)) {
+    for (int task = next_task(bs.next_task, total, true); task < total;
+         task = next_task(bs.next_task, total, false)) {
         // the task's bin, in scalar registers (uniform across the wave)
         const int k = set_find(sl, task);
         const int bin = __builtin_amdgcn_readfirstlane(__shfl(sl.bin, k, 64));
@@ -1895,7 +1917,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
     const int run = per_wave >= 72 ? 24 : per_wave >= 4 ? 12 : 4;
     const int total = nm + (nw + run - 1) / run;
     int done = 0;
-    for (int task = next_task(ss.next_task); task < total; task = next_task(ss.next_task)) {
+    for (int task = next_task(ss.next_task, total, true); task < total;
+         task = next_task(ss.next_task, total, false)) {
         task = __builtin_amdgcn_readfirstlane(task);
         if (task < nm) {
             const WorkItem it = strips[task];
