@@ -50,16 +50,17 @@ __global__ void k_clear_list(ClearList cl)
 // wildcard and exact bins, so the tile kernels' emission tables need only the
 // four bases -- and the longest hap (per-block maxima into kHmaxParts
 // counters, folded by k_scan_bins).
-__global__ __launch_bounds__(256) void k_hap_pass(BinParams bp)
+// Block `block` of `nblocks` (256 threads); returns its longest hap (thread 0).
+__device__ __forceinline__ int hap_pass(const BinParams& bp, const BatchDesc& b, int block,
+                                        int nblocks)
 {
-    const BatchDesc& b = *bp.bd;
     __shared__ int wmax[4];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int nwaves = gridDim.x * (blockDim.x >> 6);
+    const int nwaves = nblocks * (blockDim.x >> 6);
     const uint32_t* hd = reinterpret_cast<const uint32_t*>(b.hap_data);
     uint32_t* out = reinterpret_cast<uint32_t*>(bp.hapc);
     int m = 0;
-    const int h0 = blockIdx.x * (blockDim.x >> 6) + wv;
+    const int h0 = block * (blockDim.x >> 6) + wv;
     // the next hap's length and offset are loaded one hap ahead
     int hl_next = h0 < b.nH ? b.hap_len[h0] : 0;
     int off_next = h0 < b.nH ? b.hap_off[h0] : 0;
@@ -95,13 +96,16 @@ __global__ __launch_bounds__(256) void k_hap_pass(BinParams bp)
     if (lane == 0)
         wmax[wv] = m;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int bm = 0;
-        for (int k = 0; k < (int)(blockDim.x >> 6); ++k)
-            bm = max(bm, wmax[k]);
-        if (bm > 0)  // the parts start at 0: blocks without haps skip the atomic
-            atomicMax(&bp.hmax_part[blockIdx.x & (kHmaxParts - 1)], bm);
-    }
+    int bm = 0;
+    for (int k = 0; k < (int)(blockDim.x >> 6); ++k)
+        bm = max(bm, wmax[k]);
+    return bm;
+}
+__global__ __launch_bounds__(256) void k_hap_pass(BinParams bp)
+{
+    const int bm = hap_pass(bp, *bp.bd, blockIdx.x, gridDim.x);
+    if (threadIdx.x == 0 && bm > 0)  // the parts start at 0: blocks without haps skip the atomic
+        atomicMax(&bp.hmax_part[blockIdx.x & (kHmaxParts - 1)], bm);
 }
 
 // Per read (16 lanes each, four reads per wave): its packed rows and its
@@ -117,9 +121,10 @@ __global__ __launch_bounds__(256) void k_hap_pass(BinParams bp)
 // holding a byte other than A/C/G/T/N goes to the exact bin 2*ntiles+1.  The slot
 // combines its lanes' verdicts and the product of alpha with row-local
 // reductions.
-__global__ __launch_bounds__(256) void k_read_meta(BinParams bp)
+// Block `block` of `nblocks` (256 threads).
+__device__ __forceinline__ void read_meta(const BinParams& bp, const BatchDesc& b, int block,
+                                          int nblocks)
 {
-    const BatchDesc& b = *bp.bd;
     __shared__ float ph2pr[128];
     for (int q = threadIdx.x; q < 128; q += blockDim.x)
         ph2pr[q] = bp.ph2pr[q];
@@ -132,11 +137,11 @@ __global__ __launch_bounds__(256) void k_read_meta(BinParams bp)
     const bool row_gcp = bp.semantics == 2;  // per-position gcp: eps of every row
     uint4* rows4 = reinterpret_cast<uint4*>(bp.rows);
     const int sl = threadIdx.x & 15;
-    const int nslots = gridDim.x * (blockDim.x >> 4);
+    const int nslots = nblocks * (blockDim.x >> 4);
     // every 16-lane slot runs the same number of iterations, so the row-local
     // reductions below never have a slot missing
     const int iters = (b.nR + nslots - 1) / nslots;
-    const int i0 = blockIdx.x * (blockDim.x >> 4) + (threadIdx.x >> 4);
+    const int i0 = block * (blockDim.x >> 4) + (threadIdx.x >> 4);
     // the next read's length and offset are loaded one read ahead
     int L_next = i0 < b.nR ? b.read_len[i0] : 0;
     int off_next = i0 < b.nR ? b.read_off[i0] : 0;
@@ -253,21 +258,24 @@ __global__ __launch_bounds__(256) void k_read_meta(BinParams bp)
         bp.meta[i] = m;
     }
 }
+__global__ __launch_bounds__(256) void k_read_meta(BinParams bp)
+{
+    read_meta(bp, *bp.bd, blockIdx.x, gridDim.x);
+}
 
 // Exclusive prefix of R_g*H_g (the reference's resultOffsetsPerBatch,
-// gpuworker.cuh:802-815), one block of 1024 threads, four consecutive
+// gpuworker.cuh:802-815), one block of up to 1024 threads, four consecutive
 // groups per thread and pass.
-__global__ __launch_bounds__(1024) void k_align_offsets(BinParams bp)
+__device__ __forceinline__ void align_offsets(const BinParams& bp, const BatchDesc& b)
 {
-    const BatchDesc& b = *bp.bd;
-    const int G = b.G;
+    const int G = b.G, nt = blockDim.x, nwv = nt >> 6;
     __shared__ int64_t wsum[16];
     __shared__ int64_t carry;
     if (threadIdx.x == 0)
         carry = 0;
     __syncthreads();
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int base = 0; base < G; base += 4096) {
+    for (int base = 0; base < G; base += 4 * nt) {
         const int g0 = base + 4 * (int)threadIdx.x;
         int64_t p[4];
 #pragma unroll
@@ -285,7 +293,7 @@ __global__ __launch_bounds__(1024) void k_align_offsets(BinParams bp)
         __syncthreads();
         if (threadIdx.x == 0) {
             int64_t s = 0;
-            for (int k = 0; k < 16; ++k) {
+            for (int k = 0; k < nwv; ++k) {
                 const int64_t t = wsum[k];
                 wsum[k] = s;
                 s += t;
@@ -301,12 +309,16 @@ __global__ __launch_bounds__(1024) void k_align_offsets(BinParams bp)
             run += p[u];
         }
         __syncthreads();
-        if (threadIdx.x == 1023)
+        if ((int)threadIdx.x == nt - 1)
             carry = incl;
         __syncthreads();
     }
     if (threadIdx.x == 0)
         bp.align_off[G] = carry;
+}
+__global__ __launch_bounds__(1024) void k_align_offsets(BinParams bp)
+{
+    align_offsets(bp, *bp.bd);
 }
 
 // Sort key of a unit of group g: bin, then descending hap length (or
@@ -951,6 +963,325 @@ __global__ __launch_bounds__(64 * NW) void k_scatter_t(BinParams bp)
                                                w_off[wv], w_st[wv], w_h[wv], w_base[wv]);
         __syncthreads();  // the next group rebuilds gb and gh
     }
+}
+
+// ---------------------------------------------------------------------------
+// Small calls: the whole preparation in three launches
+// ---------------------------------------------------------------------------
+// A small call's time is its launches: each of the sequence's kernels costs
+// 4.5 us by itself, the descriptor's copy with the gaps around it 23 us, and
+// the counting sort's passes are latency (a record's runs in turn, atomics of
+// many records on one hap length).  Its tasks need no order -- they are fewer
+// than the device's waves or not many more -- so three kernels write them:
+// k_tiny_desc takes the descriptor from host memory, k_tiny_prep encodes haps
+// and reads side by side, k_tiny_plan cuts one record per block into tasks.
+// Before -> after, us per call: 250 reads x 32 haps 226 -> 153, 1000 records of
+// 8 x 4 300 -> 128, 50 records of 8 x 4 133 -> 68.
+// late_begin: where tl.late starts, counted from the final list.
+__global__ __launch_bounds__(256) void k_tiny_desc(BinParams bp, TinyLists tl, const BatchDesc* src,
+                                                   int late_begin)
+{
+    static_assert(sizeof(BatchDesc) % 4 == 0 && sizeof(BatchDesc) / 4 <= 256, "one word per thread");
+    const int i = threadIdx.x;
+    if (i < (int)(sizeof(BatchDesc) / 4))
+        reinterpret_cast<uint32_t*>(const_cast<BatchDesc*>(bp.bd))[i] =
+            reinterpret_cast<const volatile uint32_t*>(src)[i];
+    if (i < kTinyCounts)
+        tl.counts[i] = 0;
+    if (i < 4)
+        tl.counts[kTinyFinalRange + i] = i == 2 ? late_begin : 0;
+    if (i == 0)
+        *bp.task_ctr = 0;
+}
+
+__global__ __launch_bounds__(256) void k_tiny_prep(BinParams bp)
+{
+    const BatchDesc b = *bp.bd;
+    int block = blockIdx.x;
+    if (block == 0) {
+        align_offsets(bp, b);
+        return;
+    }
+    block -= 1;
+    if (block < kTinyHapBlocks) {
+        const int bm = hap_pass(bp, b, block, kTinyHapBlocks);
+        if (threadIdx.x == 0)
+            bp.hmax_part[block] = bm;
+        return;
+    }
+    read_meta(bp, b, block - kTinyHapBlocks, kTinyReadBlocks);
+}
+
+// A record's hap segments for k_tiny_plan (one wave): n = columns / budget of
+// about equal columns, each hap in the segment that holds its middle, or one
+// hap each.
+__device__ __forceinline__ void tiny_haps(const BinParams& bp, const BatchDesc& b, int h0, int nh,
+                                          GroupHaps& gh)
+{
+    const int lane = threadIdx.x & 63;
+    int ne = 0, wi = 0, ex = 0, tot = 0, normal = 0;
+    for (int h = lane; h < nh; h += 64) {
+        const int hl = max(b.hap_len[h0 + h], 0), flag = bp.hapflag[h0 + h];
+        if (h < kMaxSegs)
+            gh.info[h] = hl | (hl > 0 ? flag : 0) << 29;
+        ne += hl > 0;
+        wi += (hl > 0) & (flag == 1);
+        ex += (hl > 0) & (flag == 2);
+        normal += (hl > 0) & (flag == 0);
+        tot += flag == 0 ? hl : 0;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        ne += __shfl_xor(ne, o, 64);
+        wi += __shfl_xor(wi, o, 64);
+        ex += __shfl_xor(ex, o, 64);
+        normal += __shfl_xor(normal, o, 64);
+        tot += __shfl_xor(tot, o, 64);
+    }
+    const int want = (int)((float)tot / (float)b.col_budget + 0.5f);
+    const int n = max(1, min(want, min(normal, kMaxSegs - 1)));
+    // (64 bits: exact columns, so a later hap's segment is never a lower one)
+    const double scale = (double)n / (double)max(tot, 1);
+    const bool each = n == normal;
+    int before = 0, haps = 0, segs = 0, last = -1;  // columns, haps, segments and segment so far
+    for (int c0 = 0; c0 < nh; c0 += 64) {
+        const int h = c0 + lane;
+        int cols = 0;
+        if (h < nh) {
+            const int hl = b.hap_len[h0 + h];
+            cols = hl > 0 && bp.hapflag[h0 + h] == 0 ? hl : 0;
+        }
+        int x = cols;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(x, o, 64);
+            x += lane >= o ? y : 0;
+        }
+        const int at = before + x - cols;  // columns before this hap
+        const unsigned long long m = __ballot(cols > 0);
+        const unsigned long long below = m & ((1ull << lane) - 1);
+        const int sg = each ? haps + __popcll(below)
+                            : min((int)(((double)at + 0.5 * (double)cols) * scale), n - 1);
+        const int prev = __shfl(sg, below ? 63 - __clzll((long long)below) : 0, 64);
+        const bool first = cols > 0 && sg != (below ? prev : last);
+        const unsigned long long f = __ballot(first);
+        if (first) {
+            const int q = segs + __popcll(f & ((1ull << lane) - 1));
+            gh.hs[q] = h;
+            if (q > 0)
+                gh.he[q - 1] = h;
+        }
+        segs += __popcll(f);
+        before += __shfl(x, 63, 64);
+        haps += __popcll(m);
+        if (m)
+            last = __shfl(sg, 63 - __clzll((long long)m), 64);
+    }
+    if (lane == 0) {
+        gh.nonempty = ne;
+        gh.wild = wi;
+        gh.exotic = ex;
+        gh.nseg = segs;
+        if (segs > 0)
+            gh.he[segs - 1] = nh;
+    }
+}
+
+// Per record: its reads ordered by (form, tile class), longest first, cut into
+// chunks of as many of a class as fit side by side (the last may hold fewer;
+// a chunk does not go on into the next class, whose reads would sweep more
+// columns past the hap than they do elsewhere, and with them the scaling's
+// verdict could differ), each against the record's hap segments; and the
+// items of the other bins.  A record is one block's chain of dependent steps:
+// classes, haps and tasks each in parallel over lanes (28.6 us for 250 reads
+// against 32 haps where one lane went over them, 8.0 now).
+__global__ __launch_bounds__(256) void k_tiny_plan(BinParams bp, TinyLists tl)
+{
+    const BatchDesc b = *bp.bd;
+    __shared__ GroupHaps gh;
+    __shared__ int cnt[kMaxBins + 1], pos[kMaxBins + 1];
+    // a class's chunks: reads at .. end-1, the first chunk's number, reads per
+    // chunk, lanes per read
+    struct Run {
+        int at, end, first, W, G;
+    };
+    __shared__ Run runs[2][kMaxTiles];
+    __shared__ int nruns[2], nchunks[2], base[2], item_base[3], item_n[3];
+    static_assert(kMaxTiles <= 64, "one class per lane");
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int mb = 2 * bp.ntiles, NB1 = bp.NB + 1;
+    if (blockIdx.x == 0 && tid < 64) {  // the longest hap
+        int m = 0;
+        for (int q = tid; q < kTinyHapBlocks; q += 64)
+            m = max(m, bp.hmax_part[q]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+            m = max(m, __shfl_xor(m, o, 64));
+        if (tid == 0)
+            *bp.hmax = m;
+    }
+    for (int g = blockIdx.x; g < b.G; g += gridDim.x) {
+        const int r0 = b.rprefix[g], nr = b.nreads[g], h0 = b.hprefix[g], nh = b.nhaps[g];
+        const int64_t A = bp.align_off[g];
+        for (int k = tid; k < NB1; k += 256)
+            cnt[k] = 0;
+        __syncthreads();
+        for (int r = tid; r < nr; r += 256) {
+            const int k = bp.meta[r0 + r].bin;
+            atomicAdd(&cnt[k < 0 ? bp.NB : k], 1);
+        }
+        if (wv == 3)
+            tiny_haps(bp, b, h0, nh, gh);
+        __syncthreads();
+        if (wv < 2) {
+            // this form's classes (form = wave), the longest first: lane l has
+            // class ntiles-1-l
+            const int c = bp.ntiles - 1 - lane, k = 2 * c + wv;
+            const int reads = c >= 0 ? cnt[k] : 0;
+            const int G = c >= 0 ? bp.lanes[c] : 64, W = 64 / G;
+            const int chunks = (reads + W - 1) / W;
+            int at = reads, nc = chunks;  // inclusive sums
+            int fast = c >= 0 && wv == 1 ? cnt[2 * c] : 0;
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(at, o, 64), z = __shfl_up(nc, o, 64);
+                at += lane >= o ? y : 0;
+                nc += lane >= o ? z : 0;
+                fast += __shfl_xor(fast, o, 64);  // SAFE after FAST
+            }
+            const unsigned long long m = __ballot(reads > 0);
+            if (c >= 0)
+                pos[k] = fast + at - reads;
+            if (reads > 0) {
+                Run& r = runs[wv][__popcll(m & ((1ull << lane) - 1))];
+                r.at = fast + at - reads;
+                r.end = fast + at;
+                r.first = nc - chunks;
+                r.W = W;
+                r.G = G;
+            }
+            if (lane == 63) {
+                const int tasks = nc * gh.nseg;
+                nruns[wv] = __popcll(m);
+                nchunks[wv] = nc;
+                base[wv] = tasks > 0 ? atomicAdd(&tl.counts[kTinyFast + wv], tasks) : 0;
+            }
+        } else if (wv == 2) {  // the other bins' reads, after both forms
+            int at = 0;
+            for (int k = lane; k < mb; k += 64)
+                at += cnt[k];
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1)
+                at += __shfl_xor(at, o, 64);
+            if (lane == 0)
+                for (int k = mb; k < NB1; ++k) {
+                    pos[k] = at;
+                    at += cnt[k];
+                }
+        }
+        __syncthreads();
+        for (int r = tid; r < nr; r += 256) {
+            const int k = bp.meta[r0 + r].bin;
+            bp.read_perm[r0 + atomicAdd(&pos[k < 0 ? bp.NB : k], 1)] = r0 + r;
+        }
+        // super-tasks: a class per wave, a hap segment per lane; tasks of one
+        // segment lie together, the longest class first
+        for (int form = 0; form < 2; ++form) {
+            const int n = nruns[form], nc = nchunks[form];
+            for (int q = wv; q < n; q += 4) {
+                const Run r = runs[form][q];
+                const int chunks = (r.end - r.at + r.W - 1) / r.W;
+                // one chunk's segments, or with few segments several chunks' at once
+                const int side = max(1, min(64 / max(gh.nseg, 1), chunks));
+                for (int ch0 = 0; ch0 < chunks; ch0 += side)
+                    for (int y = lane; y < gh.nseg * side; y += 64) {
+                        const int sg = y / side, ch = ch0 + y - sg * side;
+                        if (ch >= chunks)
+                            continue;
+                        const int at = r.at + ch * r.W;
+                        SuperTask t;
+                        t.perm = r0 + at;
+                        t.nc = min(r.W, r.end - at) | r.G << 8;
+                        t.h0 = h0;
+                        t.nh = nh;
+                        t.hs = gh.hs[sg];
+                        t.he = gh.he[sg];
+                        t.r0 = r0;
+                        t.aoff = (int32_t)A;
+                        tl.st[form][base[form] + sg * nc + r.first + ch] = t;
+                    }
+            }
+        }
+        // one-alignment items (strips, wildcard, exact) and empty alignments
+        const int odd = cnt[mb] + cnt[mb + 1] + cnt[mb + 2] + cnt[bp.NB];
+        if (odd > 0 || gh.nonempty < nh || gh.wild + gh.exotic > 0) {  // uniform
+            if (tid < 3)
+                item_n[tid] = 0;
+            const bool plain_haps = gh.nonempty == nh && gh.wild + gh.exotic == 0;
+            // two passes over the pairs, a read per wave: count, then write
+            for (int pass = 0; pass < 2; ++pass) {
+                __syncthreads();
+                if (pass == 1 && tid < 3) {
+                    item_base[tid] = item_n[tid] > 0 ? atomicAdd(&tl.counts[kTinyStrips + tid], item_n[tid]) : 0;
+                    item_n[tid] = 0;
+                }
+                __syncthreads();
+                for (int r = wv; r < nr; r += 4) {
+                    const int k = bp.meta[r0 + r].bin;
+                    const bool tile = k >= 0 && is_tile_bin(bp, k);
+                    if (tile && plain_haps)
+                        continue;
+                    const int64_t row = A + (int64_t)r * nh;
+                    for (int h1 = 0; h1 < nh; h1 += 64) {
+                        const int h = h1 + lane;
+                        int hl = 0, flag = 0;
+                        if (h < nh)
+                            hap_info(bp, b, gh, h0, h, hl, flag);
+                        const bool empty = h < nh && (k < 0 || hl <= 0);
+                        if (empty && pass == 0)
+                            b.scores[row + h] = -INFINITY;
+                        const bool item = h < nh && !empty && !(tile && flag == 0);
+                        const int rb = item ? run_bin_of(bp, k, flag) : -1;
+                        const int list = !item ? -1 : rb == mb ? 0 : rb == mb + 2 ? 1 : 2;
+                        for (int l = 0; l < 3; ++l) {
+                            const unsigned long long m = __ballot(list == l);
+                            if (!m)
+                                continue;
+                            int at = 0;
+                            if (lane == 0)
+                                at = atomicAdd(&item_n[l], __popcll(m));
+                            at = __shfl(at, 0, 64);
+                            if (pass == 0 || list != l)
+                                continue;
+                            WorkItem it;
+                            it.read = r0 + r;
+                            it.hap = h0 + h;
+                            it.out = (int32_t)(row + h);
+                            it.pad = 0;
+                            WorkItem* out = l == 0 ? tl.strips : l == 1 ? tl.wilds : tl.exact;
+                            out[item_base[l] + at + __popcll(m & ((1ull << lane) - 1))] = it;
+                        }
+                    }
+                }
+            }
+        }
+        __syncthreads();  // the next record rebuilds the tables
+    }
+}
+
+hipError_t launch_tiny_prep(const BinParams& bp, const TinyLists& tl, const BatchDesc* src,
+                            int late_begin, hipStream_t st)
+{
+    static_assert(kTinyHapBlocks <= kHmaxParts, "one maximum per block");
+    hipLaunchKernelGGL(k_tiny_desc, dim3(1), dim3(256), 0, st, bp, tl, src, late_begin);
+    hipLaunchKernelGGL(k_tiny_prep, dim3(1 + kTinyHapBlocks + kTinyReadBlocks), dim3(256), 0, st, bp);
+    return hipGetLastError();
+}
+
+hipError_t launch_tiny_plan(const BinParams& bp, const TinyLists& tl, int grid, hipStream_t st)
+{
+    hipLaunchKernelGGL(k_tiny_plan, dim3(grid), dim3(256), 0, st, bp, tl);
+    return hipGetLastError();
 }
 
 __global__ void k_add_counts(CountSums c)

@@ -120,7 +120,12 @@ void Engine::free_ctx(CallCtx& c)
         hipHostFree(c.h_desc);
     if (c.h_bin_range)
         hipHostFree(c.h_bin_range);
+    if (c.h_tiny)
+        hipHostFree(c.h_tiny);
     for (auto& ev : c.desc_ev)
+        if (ev)
+            hipEventDestroy(ev);
+    for (auto& ev : c.tiny_ev)
         if (ev)
             hipEventDestroy(ev);
     if (c.call_done)
@@ -174,6 +179,9 @@ int Engine::init_ctx(int k)
         (rc = check(hipHostMalloc(reinterpret_cast<void**>(&c.h_desc),
                                   sizeof(BatchDesc) * kDescRing, hipHostMallocDefault),
                     "pinned descriptors")) ||
+        (rc = check(hipHostMalloc(reinterpret_cast<void**>(&c.h_tiny), sizeof(BatchDesc) * 2,
+                                  hipHostMallocDefault),
+                    "pinned descriptors")) ||
         (rc = check(hipHostMalloc(reinterpret_cast<void**>(&c.h_bin_range),
                                   2 * sizeof(int32_t) * (kMaxWorkBins + kMaxBins),
                                   hipHostMallocDefault),
@@ -181,6 +189,9 @@ int Engine::init_ctx(int k)
         return rc;
     for (int i = 0; i < kDescRing; ++i)
         if ((rc = check(hipEventCreateWithFlags(&c.desc_ev[i], hipEventDisableTiming), "event")))
+            return rc;
+    for (hipEvent_t& ev : c.tiny_ev)
+        if ((rc = check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "event")))
             return rc;
     if ((rc = check(hipEventCreateWithFlags(&c.call_done, hipEventDisableTiming), "event")))
         return rc;
@@ -246,6 +257,13 @@ void Engine::scratch_sizes(const phmm_batch_view& v, int NB, int NW, size_t out[
     out[kHapFlag] = (size_t)std::max(v.num_haps, 1);
     // per-lane magnitudes of rescued alignments: 16 bytes per rescue-list slot
     out[kRescueExps] = (size_t)kReKnownLanes * nA;
+    // small calls: the SAFE super-tasks, strips, exact-bin items, SAFE rescue
+    // list, final and late lists (their other lists are in the arrays above),
+    // at offsets that follow from the buffer's size
+    size_t cap = 1 << 16;
+    while (nA <= (size_t)kTinyAlignments && cap < nA)
+        cap *= 2;
+    out[kTinyScratch] = kTinyBytes * cap;
 }
 
 int Engine::ensure_pin(PinBuf& b, size_t bytes, const char* what)
@@ -347,18 +365,28 @@ int Engine::score_device(const phmm_batch_view& v, float* d_scores, hipStream_t 
     static const char* const kScratchName[kNumScratch] = {
         "rows", "hap codes", "read meta", "group bins", "group bins", "read perm",
         "align offsets", "keys", "keys", "bin ranges", "work items", "alignment ranges",
-        "super-tasks", "rescue list", "final list", "hap flags", "rescue maxima"};
+        "super-tasks", "rescue list", "final list", "hap flags", "rescue maxima", "small-call lists"};
     size_t need[kNumScratch];
     scratch_sizes(v, NB, NW, need);
+    bool tiny = tiny_call(v);
     void* sp[kNumScratch];
     if (arena) {
         // the allocation-free form: every buffer at a 256-byte boundary of
-        // the arena, the spill arena takes the rest
-        size_t o = 0;
-        for (int i = 0; i < kNumScratch; ++i) {
-            sp[i] = arena + o;
-            o = align256(o + need[i]);
-        }
+        // the arena, the spill arena takes the rest; the small-call lists
+        // only where they fit as well
+        auto carve = [&]() {
+            size_t o = 0;
+            for (int i = 0; i < kNumScratch; ++i) {
+                sp[i] = arena + o;
+                o = align256(o + need[i]);
+            }
+            return o;
+        };
+        need[kTinyScratch] = kTinyBytes * (size_t)std::max<int64_t>(nA, 1);
+        tiny = tiny && carve() + kMinArenaSpill <= arena_bytes;
+        if (!tiny)
+            need[kTinyScratch] = 0;
+        const size_t o = carve();
         if (o + kMinArenaSpill > arena_bytes)
             return set_error(PHMM_ERANGE,
                              "score_device: the batch needs " + std::to_string(o + kMinArenaSpill) +
@@ -406,22 +434,34 @@ int Engine::score_device(const phmm_batch_view& v, float* d_scores, hipStream_t 
         const double mean_hl = v.num_haps > 0 ? (double)v.hap_bytes / v.num_haps : 0.0;
         const double cols = (double)nA * mean_hl;
         hd.col_budget = (int32_t)std::min(8192.0, std::max(256.0, cols / (8.0 * 32768.0)));
+        if (tiny) {
+            // a task per resident wave, or several where a wave has many
+            // columns: no order evens their lengths out
+            const double w = tiny_columns(v);
+            hd.col_budget = (int32_t)std::max(1.0, w <= 512.0 ? w : std::max(256.0, w / 8));
+        }
     }
     hd.read_bytes = v.read_bytes;
     hd.hap_bytes = v.hap_bytes;
     hd.num_alignments = nA;
-    {
-        const int k = c.desc_next;
+    const bool plain = opt.mode == PHMM_MODE_PLAIN;
+    const bool eager = plain || !opt.graphs || arena || eager_hint;
+    const int dk = c.desc_next;
+    if (!tiny || eager) {
+        const int k = dk;
         c.desc_next = (c.desc_next + 1) % kDescRing;
         if (c.desc_used[k] && (rc = check(hipEventSynchronize(c.desc_ev[k]), "descriptor slot")))
             return rc;
         c.h_desc[k] = hd;
+        c.desc_used[k] = true;
+    }
+    if (!tiny) {
+        const int k = dk;
         if ((rc = check(hipMemcpyAsync(c.desc.p, &c.h_desc[k], sizeof(BatchDesc),
                                        hipMemcpyHostToDevice, st),
                         "descriptor copy")) ||
             (rc = check(hipEventRecord(c.desc_ev[k], st), "event")))
             return rc;
-        c.desc_used[k] = true;
     }
 
     // counters: [0] max hap length, [1] final-list count, [2] error flag,
@@ -505,8 +545,75 @@ int Engine::score_device(const phmm_batch_view& v, float* d_scores, hipStream_t 
             ev_free.pop_back();
         }
     }
-    const bool plain = opt.mode == PHMM_MODE_PLAIN;
-    if (plain || !opt.graphs || arena || eager_hint) {
+    // `eager` puts the stages on the stream one by one; else each is launched
+    // as a captured graph of `g` -- one for the whole call, or one per stage
+    // when the forward kernels are timed
+    auto stages = [&](auto enqueue) -> int {
+        static const int kStages[] = {kStagePrep, kStageFwd, kStageRescue};
+        int r2;
+        for (int i = 0; i < 3; ++i) {
+            if ((r2 = enqueue(kStages[i])))
+                return r2;
+            if (timed)
+                hipEventRecord(evp.e[i], st);
+        }
+        return PHMM_OK;
+    };
+    auto graph_of = [&](Graphs& g, auto enqueue) -> int {
+        auto launch = [&](int which, hipGraphExec_t* ex) -> int {
+            int r2;
+            if (!*ex && (r2 = capture([&](hipStream_t cs) { return enqueue(which, cs); }, ex)))
+                return r2;
+            ++graph_launches;
+            return check(hipGraphLaunch(*ex, st), "graph launch");
+        };
+        if (!timed)
+            return launch(kStagePrep | kStageFwd | kStageRescue, &g.all);
+        return stages([&](int which) {
+            return launch(which, which == kStagePrep ? &g.prep : which == kStageFwd ? &g.fwd : &g.rescue);
+        });
+    };
+    if (!eager && c.graphs[0].gen != c.generation) {
+        drop_graphs(c);
+        for (Graphs* g : {&c.graphs[0], &c.graphs[1], &c.tiny[0], &c.tiny[1]})
+            g->gen = c.generation;
+    }
+    if (tiny) {
+        TinyLists tl{};
+        tl.st[0] = static_cast<SuperTask*>(sp[kSuperTasks]);
+        tl.st[1] = static_cast<SuperTask*>(sp[kTinyScratch]);
+        const size_t cap = (arena ? need[kTinyScratch] : c.sbuf[kTinyScratch].cap) / kTinyBytes;
+        WorkItem* list = reinterpret_cast<WorkItem*>(tl.st[1] + cap);
+        tl.strips = list;
+        tl.exact = list + cap;
+        tl.rescue[1] = list + 2 * cap;
+        fp.final_items = list + 3 * cap;
+        tl.late = list + 4 * cap;
+        tl.wilds = bp.items;
+        tl.rescue[0] = fp.rescue_items;
+        tl.counts = bp.task_ctr + 1;
+        static_assert(1 + kTinyWords <= kTaskCounters, "counters");
+        fp.final_count = tl.counts + kTinyFinal;
+        if (eager) {
+            if ((rc = stages([&](int which) {
+                     return enqueue_tiny(which, bp, fp, tl, &c.h_desc[dk], st);
+                 })) ||
+                (rc = check(hipEventRecord(c.desc_ev[dk], st), "event")))
+                return rc;
+        } else {
+            const int k = c.tiny_next;
+            c.tiny_next ^= 1;
+            if (c.tiny_used[k] && (rc = check(hipEventSynchronize(c.tiny_ev[k]), "descriptor slot")))
+                return rc;
+            c.h_tiny[k] = hd;
+            if ((rc = graph_of(c.tiny[k], [&](int which, hipStream_t cs) {
+                     return enqueue_tiny(which, bp, fp, tl, &c.h_tiny[k], cs);
+                 })) ||
+                (rc = check(hipEventRecord(c.tiny_ev[k], st), "event")))
+                return rc;
+            c.tiny_used[k] = true;
+        }
+    } else if (eager) {
         if ((rc = enqueue_prep(bp, hd, false, st)))
             return rc;
         if (plain) {
@@ -533,34 +640,18 @@ int Engine::score_device(const phmm_batch_view& v, float* d_scores, hipStream_t 
         if (timed)
             hipEventRecord(evp.e[2], st);
     } else {
-        // batched: replay captured graphs -- one for the whole call, or one
-        // per stage when the forward kernels are timed
-        Graphs& graphs = c.graphs[act == &tiles_small ? 1 : 0];
-        if (graphs.gen != c.generation) {
-            drop_graphs(c);
-            c.graphs[0].gen = c.graphs[1].gen = c.generation;
-        }
-        auto launch = [&](int stages, hipGraphExec_t* ex) -> int {
-            int r2;
-            if (!*ex && (r2 = capture(stages, bp, fp, hd, ex)))
-                return r2;
-            ++graph_launches;
-            return check(hipGraphLaunch(*ex, st), "graph launch");
-        };
-        if (!timed) {
-            if ((rc = launch(kStagePrep | kStageFwd | kStageRescue, &graphs.all)))
-                return rc;
-        } else {
-            if ((rc = launch(kStagePrep, &graphs.prep)))
-                return rc;
-            hipEventRecord(evp.e[0], st);
-            if ((rc = launch(kStageFwd, &graphs.fwd)))
-                return rc;
-            hipEventRecord(evp.e[1], st);
-            if (opt.fp64_rescue && (rc = launch(kStageRescue, &graphs.rescue)))
-                return rc;
-            hipEventRecord(evp.e[2], st);
-        }
+        rc = graph_of(c.graphs[act == &tiles_small ? 1 : 0], [&](int which, hipStream_t cs) -> int {
+            int r2 = PHMM_OK;
+            if (which & kStagePrep)
+                r2 = enqueue_prep(bp, hd, true, cs);
+            if (!r2 && (which & kStageFwd))
+                r2 = enqueue_fwd(fp, bp, false, cs);
+            if (!r2 && (which & kStageRescue) && opt.fp64_rescue)
+                r2 = enqueue_rescue(fp, bp, false, cs);
+            return r2;
+        });
+        if (rc)
+            return rc;
     }
     if (timed)
         ev_pending.push_back(evp);
@@ -881,7 +972,7 @@ int Engine::enqueue_rescue(const FwdParams& fp, const BinParams& bp, bool plain,
     for (int src = 0; src < 2; ++src)
         if (wave[src].n &&
             (rc = check(launch_fwd_wave_f64(fp, wave[src], bp.hmax, spill64, n64, bp.error_flag,
-                                            num_cus * 8, st),
+                                            num_cus * 8, st, false),
                         "FP64 wave kernel")))
             return rc;
     BinSet fin;
@@ -892,7 +983,7 @@ int Engine::enqueue_rescue(const FwdParams& fp, const BinParams& bp, bool plain,
     fin.counts = fp.final_count;
     fin.count_stride = 0;
     if ((rc = check(launch_fwd_wave_f64(fp, fin, bp.hmax, spill64, n64, bp.error_flag, num_cus * 8,
-                                        st),
+                                        st, true),
                     "FP64 final kernel")))
         return rc;
     // statistics: the rescue lists; in FP64: the retry lists and the rescue
@@ -913,10 +1004,88 @@ int Engine::enqueue_rescue(const FwdParams& fp, const BinParams& bp, bool plain,
     return PHMM_OK;
 }
 
-// Captures the given stages of the batched sequence (fixed grids) on a
-// private stream and instantiates the graph.
-int Engine::capture(int stages, const BinParams& bp, const FwdParams& fp, const BatchDesc& hd,
-                    hipGraphExec_t* out)
+double Engine::tiny_columns(const phmm_batch_view& v) const
+{
+    if (v.num_reads <= 0 || v.num_haps <= 0)
+        return 0.0;
+    const double mean_rl = (double)v.read_bytes / v.num_reads;
+    const double lanes = std::ceil(mean_rl / kTinyRows);
+    // reads side by side in a sweep, or the strips of one read in turn
+    const double side = lanes <= 64.0 ? std::floor(64.0 / std::max(1.0, lanes))
+                                      : 1.0 / std::ceil(mean_rl / kStripTileRows);
+    return (double)v.num_alignments * ((double)v.hap_bytes / v.num_haps) / side / (num_cus * 8);
+}
+
+bool Engine::tiny_call(const phmm_batch_view& v) const
+{
+    if (opt.mode == PHMM_MODE_PLAIN || !scaled_pass() || act != &tiles_small ||
+        v.num_alignments > kTinyAlignments || v.num_groups > kTinyGroups ||
+        tiny_columns(v) > kTinyColumns)
+        return false;
+    // records of few reads that share a sweep leave their last chunk part empty
+    if (v.num_reads < 64 * (int64_t)v.num_groups && tiny_columns(v) > kTinyColumnsFew &&
+        v.read_bytes <= (int64_t)v.num_reads * 64 * kTinyRows)
+        return false;
+    for (const phmm_tile_config& t : *act)
+        if (t.rows != kTinyRows)  // a caller's table with wider tiles than 64 x 16 rows
+            return false;
+    return true;
+}
+
+int Engine::enqueue_tiny(int stages, const BinParams& bp, const FwdParams& fp, const TinyLists& tl,
+                         const BatchDesc* src, hipStream_t st)
+{
+    int rc;
+    const int waves = num_cus * 8;
+    if ((stages & kStagePrep) &&
+        ((rc = check(launch_tiny_prep(bp, tl, src, (int)(tl.late - fp.final_items), st), "preparation kernel")) ||
+         (rc = check(launch_tiny_plan(bp, tl, 512, st), "planning kernel"))))
+        return rc;
+    if (stages & kStageFwd) {
+        SpecialSet ss;
+        ss.strip_bin = 2 * bp.ntiles;
+        ss.next_task = bp.task_ctr;
+        ss.hmax = bp.hmax;
+        ss.border = static_cast<float4*>(cur->call_spill);
+        ss.border_entries = (int64_t)(cur->call_spill_bytes / sizeof(float4));
+        ss.error_flag = bp.error_flag;
+        if ((rc = check(launch_fwd_tiny(fp, ss, tl, waves, st), "forward kernel")))
+            return rc;
+        if (opt.semantics != PHMM_SEM_GPU) {  // bytes that match nothing but themselves
+            BinSet ws;
+            ws.n = 1;
+            ws.lanes[0] = 64;
+            ws.items = tl.exact;
+            ws.counts = tl.counts + kTinyExact;
+            if ((rc = check(launch_fwd_wave_f32(fp, ws, bp.hmax, static_cast<float*>(cur->call_spill),
+                                                (int64_t)(cur->call_spill_bytes / sizeof(float)),
+                                                bp.error_flag, waves, st),
+                            "exact kernel")))
+                return rc;
+        }
+    }
+    if (stages & kStageRescue) {
+        BinSet fin;
+        fin.n = 2;
+        fin.bin[0] = 0;
+        fin.bin[1] = 1;
+        fin.lanes[0] = fin.lanes[1] = 64;
+        fin.items = fp.final_items;
+        fin.range = tl.counts + kTinyFinalRange;
+        fin.counts = fp.final_count;
+        fin.count_stride = 1;
+        if ((rc = check(launch_rescue_tiny(fp, tl, waves, d_rescued_total, st), "FP64 tile kernel")) ||
+            (rc = check(launch_fwd_wave_f64(fp, fin, bp.hmax, static_cast<double*>(cur->call_spill),
+                                            (int64_t)(cur->call_spill_bytes / sizeof(double)),
+                                            bp.error_flag, waves, st, true, d_rescued_total),
+                        "FP64 final kernel")))
+            return rc;
+    }
+    return PHMM_OK;
+}
+
+template <typename F>
+int Engine::capture(F enqueue, hipGraphExec_t* out)
 {
     int rc;
     if (!cap_stream &&
@@ -925,13 +1094,7 @@ int Engine::capture(int stages, const BinParams& bp, const FwdParams& fp, const 
     if ((rc = check(hipStreamBeginCapture(cap_stream, hipStreamCaptureModeRelaxed),
                     "begin capture")))
         return rc;
-    int r2 = PHMM_OK;
-    if (stages & kStagePrep)
-        r2 = enqueue_prep(bp, hd, true, cap_stream);
-    if (!r2 && (stages & kStageFwd))
-        r2 = enqueue_fwd(fp, bp, false, cap_stream);
-    if (!r2 && (stages & kStageRescue) && opt.fp64_rescue)
-        r2 = enqueue_rescue(fp, bp, false, cap_stream);
+    const int r2 = enqueue(cap_stream);
     hipGraph_t g = nullptr;
     const hipError_t e = hipStreamEndCapture(cap_stream, &g);
     if (r2) {
@@ -963,19 +1126,17 @@ void Engine::derive_small_tiles()
 
 void Engine::drop_graphs(CallCtx& c)
 {
-    Graphs* graphs = c.graphs;
-    hipGraphExec_t* all[] = {&graphs[0].all, &graphs[0].prep, &graphs[0].fwd, &graphs[0].rescue,
-                             &graphs[1].all, &graphs[1].prep, &graphs[1].fwd, &graphs[1].rescue};
-    bool any = false;
-    for (auto* x : all)
-        any = any || *x;
-    if (any)
+    std::vector<hipGraphExec_t*> all;
+    for (Graphs* g : {&c.graphs[0], &c.graphs[1], &c.tiny[0], &c.tiny[1]})
+        for (hipGraphExec_t* x : {&g->all, &g->prep, &g->fwd, &g->rescue})
+            if (*x)
+                all.push_back(x);
+    if (!all.empty())
         hipDeviceSynchronize();  // launched replays may still run
-    for (auto* x : all)
-        if (*x) {
-            hipGraphExecDestroy(*x);
-            *x = nullptr;
-        }
+    for (hipGraphExec_t* x : all) {
+        hipGraphExecDestroy(*x);
+        *x = nullptr;
+    }
 }
 
 void Engine::free_slot(Slot& s)

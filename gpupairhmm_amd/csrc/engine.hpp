@@ -58,7 +58,7 @@ struct Engine {
     enum ScratchBuf {
         kRows, kHapc, kMeta, kGbCount, kGbStart, kReadPerm, kAlignOff, kKeyCount, kKeyCursor,
         kBinRange, kItems, kAlignRange, kSuperTasks, kRescueItems, kFinalItems, kHapFlag,
-        kRescueExps, kNumScratch
+        kRescueExps, kTinyScratch, kNumScratch
     };
     // An arena must leave at least this much for the spill arena (one block
     // of the FP64 wave kernel holds 32 bytes per column of the longest hap).
@@ -98,6 +98,14 @@ struct Engine {
         // are captured again.
         uint64_t generation = 0;
         Graphs graphs[2];  // [0]: tuned table, [1]: small-batch table
+        // The few-launch sequence of small calls reads its descriptor from
+        // pinned memory, so a captured graph belongs to one of two slots,
+        // used in turn; a slot is rewritten once its last call is done.
+        Graphs tiny[2];
+        BatchDesc* h_tiny = nullptr;
+        hipEvent_t tiny_ev[2] = {};
+        bool tiny_used[2] = {};
+        int tiny_next = 0;
         // the current call's spill arena (spill, or the rest of an arena)
         void* call_spill = nullptr;
         size_t call_spill_bytes = 0;
@@ -203,8 +211,26 @@ struct Engine {
     int enqueue_fwd(const FwdParams& fp, const BinParams& bp, bool plain, hipStream_t st);
     int enqueue_rescue(const FwdParams& fp, const BinParams& bp, bool plain, hipStream_t st);
     enum { kStagePrep = 1, kStageFwd = 2, kStageRescue = 4 };
-    int capture(int stages, const BinParams& bp, const FwdParams& fp, const BatchDesc& hd,
-                hipGraphExec_t* out);
+    // Captures what `enqueue` puts on a private stream and instantiates it.
+    template <typename F>
+    int capture(F enqueue, hipGraphExec_t* out);
+    // The few-launch sequence of small calls (on a small-batch table of 16
+    // rows per lane, where the FP32 pass scales).  Its tasks are unsorted, so
+    // it takes calls of few hap columns per resident wave: tiny_columns, all
+    // sweeps' columns (reads of the mean length side by side) over the waves.
+    // us before -> with it, by that measure: 1000 records of 8 x 4 (229) 300 ->
+    // 128, 8 mixed records of up to 500 reads (2100) 610 -> 517, 650 of 25 x 4
+    // (1320) 556 -> 515; but 1000 of 25 x 4 (2040) 664 -> 703, where one sweep in
+    // five holds a record's last read alone, and 100 of 16 x 8 with 2-5 kb haps
+    // (5470) 1397 -> 1735: the lower line is that of records of few reads.
+    static constexpr double kTinyColumns = 4096.0, kTinyColumnsFew = 1600.0;
+    static constexpr int64_t kTinyAlignments = 1 << 18;
+    static constexpr int kTinyGroups = 8192;
+    static constexpr size_t kTinyBytes = sizeof(SuperTask) + 5 * sizeof(WorkItem);  // per alignment
+    double tiny_columns(const phmm_batch_view& v) const;
+    bool tiny_call(const phmm_batch_view& v) const;
+    int enqueue_tiny(int stages, const BinParams& bp, const FwdParams& fp, const TinyLists& tl,
+                     const BatchDesc* src, hipStream_t st);
     void drop_graphs(CallCtx& c);
     void free_ctx(CallCtx& c);
     int score_batch(const phmm_batch_view& v, float* out);

@@ -979,7 +979,7 @@ __device__ __forceinline__ int tile_super_task(const FwdParams& p, typename Tile
     const int W = 64 / G;
     const int grp = lane / G;
     const int t = lane - grp * G;
-    const bool active = grp < W && grp < st.nc;
+    const bool active = grp < W && grp < (st.nc & 0xff);
     const int rd = active ? p.read_perm[st.perm + grp] : 0;
     TileRead<T, NR, ROWEPS> R;
     tile_setup<T, NR, FAST, ROWEPS>(p, tab, active, rd, t, R);
@@ -1388,11 +1388,11 @@ __device__ __forceinline__ void pack_task(const FwdParams& p, typename TileTrait
 // T = float (multi-tile first pass) appends results below the rescue
 // threshold (as the tile kernels define it) to the final list, which the
 // T = double instance recomputes.
-// PACK (one bin): runs of items that pack_task takes go to it instead.
+// PACK: runs of items that pack_task takes go to it instead.
 template <typename T, int NR, bool PACK = false>
 __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const int32_t* hmax_ptr,
                                                  T* spill, int64_t spill_elems,
-                                                 int32_t* error_flag)
+                                                 int32_t* error_flag, int64_t* totals)
 {
     using S = WaveScalar<T>;
     const BatchDesc& bd = *p.bd;
@@ -1401,6 +1401,9 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
     const int lane = threadIdx.x;
     SetLane sl;
     const int n = set_lanes(bs, 1, sl);  // one item per wave
+    const int n0 = __shfl(sl.ntask, 0, 64);
+    if (totals && blockIdx.x == 0 && lane < 2 && n0 > 0)
+        atomicAdd(reinterpret_cast<unsigned long long*>(totals + lane), (unsigned long long)n0);
     const int hmax = *hmax_ptr;
     // per block: 3*(hmax+1) values of T, then 2*(hmax+1) int32 exponents,
     // in units of T (rounded up to 16 bytes)
@@ -1427,8 +1430,10 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
     for (int w = v; w < min(n, v + run); ++w) {
         if constexpr (PACK) {
             __shared__ typename TileTraits<T>::V tab[5 * (NR / TileTraits<T>::K) * 64];
-            const WorkItem* q = bs.items + __shfl(sl.begin, 0, 64) + w;
-            const int rem = min(n, v + run) - w;
+            const int kq = set_find(sl, w);
+            const int wq = __shfl(sl.incl - sl.ntask, kq, 64);
+            const WorkItem* q = bs.items + __shfl(sl.begin, kq, 64) + (w - wq);
+            const int rem = min(__shfl(sl.incl, kq, 64), v + run) - w;  // within the bin
             int L = 0;
             bool ok = true;
             if (lane < rem) {
@@ -1679,7 +1684,6 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
 // instead of compares, and the letters loaded four columns ahead.  The items
 // are sorted by (read class, hap length) and a wave takes a run of them.  908k
 // mixed alignments of which 5% have such a hap: 20.0 -> 7.2 ms per call.
-constexpr int kStripRows = 12;
 constexpr int kStripPad = 256;  // border entries beyond the longest hap
 // Long reads meet more of the steepest growths between two checks than the
 // tiles' reads do: the strips scale down from 2^40 (at 2^kDsGuard, 2 of 2,560
@@ -1887,61 +1891,186 @@ __device__ __forceinline__ int strip_task(const FwdParams& p, float4* tab, float
     return __ballot(done) ? 1 : 0;
 }
 
+// LDS of both: the wildcard tiles' emission table; a strip's, with its window
+// after it, is smaller.
+constexpr int kSpecialTab = TabShape<float, kWildRows, 5>::kWords;
+static_assert(TabShape<float, kStripRows, 5>::kWords + 32 <= kSpecialTab, "the window beside the table");
+
+// Items per wildcard task: 12 or 24 fill whole waves for most reads (4, 6 or
+// 12 side by side); the longer run where every wave gets several, the shorter
+// (or, for few items, 4) to spread them over the device.
+__device__ __forceinline__ int wild_run(int nw)
+{
+    const int per_wave = nw / (int)gridDim.x;
+    return per_wave >= 72 ? 24 : per_wave >= 4 ? 12 : 4;
+}
+// Task `task` of the strips (nm of them, one each) and then the wildcard
+// items' runs.
+__device__ __forceinline__ int special_task(const FwdParams& p, float4* tab, float4* border,
+                                            const WorkItem* strips, int nm, const WorkItem* wilds,
+                                            int nw, int run, int strip_bin, int task)
+{
+    const BatchDesc& bd = *p.bd;
+    if (task < nm) {
+        const WorkItem it = strips[task];
+        float4* win = tab + TabShape<float, kStripRows, 5>::kWords;
+        const ReadMeta m = p.meta[it.read];
+        const bool fast = m.bin == strip_bin ? m.nl > 0.f : (m.bin & 1) == 0;
+        return fast ? strip_task<true>(p, tab, win, border, it)
+                    : strip_task<false>(p, tab, win, border, it);
+    }
+    int i = (task - nm) * run;
+    const int end = min(i + run, nw);
+    while (i < end) {  // as many of the next items as fit side by side
+        const int n = end - i;  // at most 24: one lane each
+        const int L = (int)threadIdx.x < n ? bd.read_len[wilds[i + threadIdx.x].read] : 0;
+        const int G = (wave_max(L) + kWildRows) / kWildRows;  // ceil((L + 1) / rows)
+        const int take = min(n, 64 / G);
+        pack_task<float, kWildRows>(p, tab, wilds + i, take, G);
+        i += take;
+    }
+    return 0;
+}
+// The block's border row: false where the arena holds none for it (the
+// launch's first block then reports it).
+__device__ __forceinline__ bool border_row(const SpecialSet& ss, float4*& border)
+{
+    const int64_t stride = (int64_t)*ss.hmax + kStripPad;
+    if ((int64_t)blockIdx.x >= ss.border_entries / stride) {
+        if (blockIdx.x == 0 && threadIdx.x == 0)
+            atomicOr(ss.error_flag, 1);
+        return false;
+    }
+    border = ss.border + blockIdx.x * stride;
+    return true;
+}
+
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_fwd_special(
     FwdParams p, SpecialSet ss)
 {
-    constexpr int kTab = TabShape<float, kWildRows, 5>::kWords;
-    static_assert(TabShape<float, kStripRows, 5>::kWords + 32 <= kTab, "the window beside the table");
-    __shared__ float4 tab[kTab];
-    const BatchDesc& bd = *p.bd;
+    __shared__ float4 tab[kSpecialTab];
     const int nm = ss.range[2 * ss.strip_bin + 1], nw = ss.range[2 * ss.wild_bin + 1];
     if (nm + nw == 0)
         return;
     const WorkItem* strips = ss.items + ss.range[2 * ss.strip_bin];
     const WorkItem* wilds = ss.items + ss.range[2 * ss.wild_bin];
-    float4* border = ss.border;
-    if (nm > 0) {  // a border row per block, for as many blocks as the arena holds
-        const int64_t stride = (int64_t)*ss.hmax + kStripPad;
-        const int64_t cap = ss.border_entries / stride;
-        if ((int64_t)blockIdx.x >= cap) {
-            if (blockIdx.x == 0 && threadIdx.x == 0)
-                atomicOr(ss.error_flag, 1);
-            return;
-        }
-        border += blockIdx.x * stride;
-    }
-    // a run of items per task: 12 or 24 fill whole waves for most reads (4, 6
-    // or 12 side by side); the longer run where every wave gets several, the
-    // shorter (or, for few items, 4) to spread them over the device
-    const int per_wave = nw / (int)gridDim.x;
-    const int run = per_wave >= 72 ? 24 : per_wave >= 4 ? 12 : 4;
+    float4* border = nullptr;
+    if (nm > 0 && !border_row(ss, border))
+        return;
+    const BatchDesc bd = *p.bd;
+    p.bd = &bd;
+    const int run = wild_run(nw);
     const int total = nm + (nw + run - 1) / run;
+    int done = 0;
+    for (int task = next_task(ss.next_task, total, true); task < total;
+         task = next_task(ss.next_task, total, false))
+        done += special_task(p, tab, border, strips, nm, wilds, nw, run, ss.strip_bin,
+                             __builtin_amdgcn_readfirstlane(task));
+    if (done > 0 && threadIdx.x == 0)
+        atomicAdd(p.scaled_total, (unsigned long long)done);
+}
+
+// The FP32 pass of a small call in one launch: FAST super-tasks, SAFE ones,
+// strips and wildcard items, in that order from one counter.
+template <bool GE>
+__device__ __forceinline__ int tiny_tasks(const FwdParams& p, const SpecialSet& ss,
+                                          const TinyLists& tl, float4* tab, float4* border)
+{
+    const int nf = tl.counts[kTinyFast], ns = tl.counts[kTinySafe];
+    const int nm = tl.counts[kTinyStrips], nw = tl.counts[kTinyWilds];
+    const int run = wild_run(nw);
+    const int total = nf + ns + nm + (nw + run - 1) / run;
     int done = 0;
     for (int task = next_task(ss.next_task, total, true); task < total;
          task = next_task(ss.next_task, total, false)) {
         task = __builtin_amdgcn_readfirstlane(task);
-        if (task < nm) {
-            const WorkItem it = strips[task];
-            float4* win = tab + TabShape<float, kStripRows, 5>::kWords;
-            const ReadMeta m = p.meta[it.read];
-            const bool fast = m.bin == ss.strip_bin ? m.nl > 0.f : (m.bin & 1) == 0;
-            done += fast ? strip_task<true>(p, tab, win, border, it)
-                         : strip_task<false>(p, tab, win, border, it);
-            continue;
+        if (task < nf + ns) {
+            const bool fast = task < nf;
+            const SuperTask st = fast ? tl.st[0][task] : tl.st[1][task - nf];
+            const int G = __builtin_amdgcn_readfirstlane(st.nc >> 8);
+            // what the scaling refuses: the FP64 tiles hold 512 rows, the
+            // classes above them have more than 32 lanes
+            FwdParams q = p;
+            const bool tiles = G <= 512 / kTinyRows;
+            q.rescue_items = !tiles ? p.final_items : fast ? tl.rescue[0] : tl.rescue[1];
+            q.rescue_counts = !tiles ? p.final_count
+                                     : tl.counts + (fast ? kTinyRescueFast : kTinyRescueSafe);
+            done += fast ? tile_super_task<float, kTinyRows, true, false, true, GE>(q, tab, st, G, 0, 0)
+                         : tile_super_task<float, kTinyRows, false, false, true, GE>(q, tab, st, G, 0, 0);
+        } else {
+            done += special_task(p, tab, border, tl.strips, nm, tl.wilds, nw, run, ss.strip_bin,
+                                 task - nf - ns);
         }
-        int i = (task - nm) * run;
-        const int end = min(i + run, nw);
-        while (i < end) {  // as many of the next items as fit side by side
-            const int n = end - i;  // at most 24: one lane each
-            const int L = (int)threadIdx.x < n ? bd.read_len[wilds[i + threadIdx.x].read] : 0;
-            const int G = (wave_max(L) + kWildRows) / kWildRows;  // ceil((L + 1) / rows)
-            const int take = min(n, 64 / G);
-            pack_task<float, kWildRows>(p, tab, wilds + i, take, G);
+    }
+    return done;
+}
+
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_fwd_tiny(
+    FwdParams p, SpecialSet ss, TinyLists tl)
+{
+    static_assert(TabShape<float, kTinyRows>::kWords <= kSpecialTab, "one table for all");
+    __shared__ float4 tab[kSpecialTab];
+    float4* border = nullptr;
+    if (tl.counts[kTinyStrips] > 0 && !border_row(ss, border))
+        return;
+    const BatchDesc bd = *p.bd;
+    p.bd = &bd;
+    const int done = p.semantics == 0 ? tiny_tasks<true>(p, ss, tl, tab, border)
+                                      : tiny_tasks<false>(p, ss, tl, tab, border);
+    if (done > 0 && threadIdx.x == 0)
+        atomicAdd(p.scaled_total, (unsigned long long)done);
+}
+
+// FP64 recompute of a small call's rescue lists, usually empty: the 10-row
+// FAST and 8-row SAFE tiles (the rows of the small-batch table's FP64 sets),
+// runs of a few items per wave.  What they cannot finish joins the late list.
+template <int NR, bool FAST>
+__device__ __forceinline__ void rescue_list(const FwdParams& p, double2* tab, const WorkItem* items,
+                                            int n)
+{
+    constexpr int kRun = 6;
+    for (int v = blockIdx.x * kRun; v < n; v += gridDim.x * kRun) {
+        const int end = min(n, v + kRun);
+        for (int i = v; i < end;) {
+            const int rem = end - i;
+            const int L = (int)threadIdx.x < rem ? p.bd->read_len[items[i + threadIdx.x].read] : 0;
+            const int G = (wave_max(L) + NR) / NR;  // ceil((L + 1) / NR)
+            const int take = min(rem, 64 / G);
+            tile_items_task<double, NR, FAST, false>(p, tab, items, i, take, G, 0, 0, 0);
             i += take;
         }
     }
-    if (done > 0 && threadIdx.x == 0)
-        atomicAdd(p.scaled_total, (unsigned long long)done);
+}
+__global__ __launch_bounds__(64) void k_rescue_tiny(FwdParams p, TinyLists tl, int64_t* totals)
+{
+    __shared__ double2 tab[TabShape<double, 10>::kWords];
+    const int nf = tl.counts[kTinyRescueFast], ns = tl.counts[kTinyRescueSafe];
+    if (nf + ns == 0)
+        return;
+    if (blockIdx.x == 0 && threadIdx.x < 2)
+        atomicAdd(reinterpret_cast<unsigned long long*>(totals + threadIdx.x),
+                  (unsigned long long)(nf + ns));
+    p.final_items = tl.late;
+    p.final_count = tl.counts + kTinyLate;
+    rescue_list<10, true>(p, tab, tl.rescue[0], nf);
+    rescue_list<8, false>(p, tab, tl.rescue[1], ns);
+}
+
+hipError_t launch_rescue_tiny(const FwdParams& p, const TinyLists& tl, int grid, int64_t* totals,
+                              hipStream_t st)
+{
+    hipLaunchKernelGGL(k_rescue_tiny, dim3(grid), dim3(64), 0, st, p, tl, totals);
+    return hipGetLastError();
+}
+
+hipError_t launch_fwd_tiny(const FwdParams& p, const SpecialSet& ss, const TinyLists& tl, int grid,
+                           hipStream_t st)
+{
+    if (!p.scaled_total || !p.rescue_on || !ss.next_task || !ss.hmax || !ss.border ||
+        !ss.error_flag || grid <= 0)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_fwd_tiny, dim3(grid), dim3(64), 0, st, p, ss, tl);
+    return hipGetLastError();
 }
 
 hipError_t launch_fwd_special(const FwdParams& p, const SpecialSet& ss, int grid, hipStream_t st)
@@ -2138,22 +2267,22 @@ hipError_t launch_fwd_wave_f32(const FwdParams& p, const BinSet& bs, const int32
     if (bs.n < 1 || bs.n > 64 || !bs.counts || !bs.items || blocks <= 0)
         return hipErrorInvalidValue;
     hipLaunchKernelGGL((k_fwd_wave<float, 16>), dim3(blocks), dim3(64), 0, st, p, bs, hmax_ptr,
-                       spill, spill_elems, error_flag);
+                       spill, spill_elems, error_flag, (int64_t*)nullptr);
     return hipGetLastError();
 }
 
 hipError_t launch_fwd_wave_f64(const FwdParams& p, const BinSet& bs, const int32_t* hmax_ptr,
                                double* spill, int64_t spill_elems, int32_t* error_flag, int blocks,
-                               hipStream_t st)
+                               hipStream_t st, bool pack, int64_t* totals)
 {
     if (bs.n < 1 || bs.n > 64 || !bs.counts || !bs.items || blocks <= 0)
         return hipErrorInvalidValue;
-    if (bs.n == 1)
+    if (pack)
         hipLaunchKernelGGL((k_fwd_wave<double, 8, true>), dim3(blocks), dim3(64), 0, st, p, bs,
-                           hmax_ptr, spill, spill_elems, error_flag);
+                           hmax_ptr, spill, spill_elems, error_flag, totals);
     else
         hipLaunchKernelGGL((k_fwd_wave<double, 8>), dim3(blocks), dim3(64), 0, st, p, bs, hmax_ptr,
-                           spill, spill_elems, error_flag);
+                           spill, spill_elems, error_flag, totals);
     return hipGetLastError();
 }
 

@@ -288,6 +288,33 @@ struct BinParams {
     int32_t allow_fast;
 };
 
+// The few-launch sequence of small calls (k_tiny_prep, k_tiny_plan,
+// k_fwd_tiny, k_rescue_tiny and the final pass): its work lists, unsorted,
+// and their counters.  The tables hold 16 rows per lane throughout.
+struct TinyLists {
+    SuperTask* st[2];     // FAST, SAFE: nc holds reads | lanes << 8
+    WorkItem* strips;     // multi-tile bin
+    WorkItem* wilds;      // wildcard bin
+    WorkItem* exact;      // exact bin
+    WorkItem* rescue[2];  // what the scaling refused, by form: FP64 tiles
+    WorkItem* late;       // what the FP64 tiles could not finish
+    int32_t* counts;      // kTinyCounts counters, zeroed by k_tiny_prep
+};
+enum {
+    kTinyFast, kTinySafe, kTinyStrips, kTinyWilds, kTinyExact, kTinyRescueFast, kTinyRescueSafe,
+    kTinyFinal, kTinyLate,  // the final list (FwdParams::final_count) and `late`
+    kTinyCounts,
+    // then the two lists' begins in BinSet's form, from final_items
+    kTinyFinalRange = kTinyCounts, kTinyWords = kTinyFinalRange + 4
+};
+constexpr int kTinyHapBlocks = 128;   // grid of k_tiny_prep: one control block,
+constexpr int kTinyReadBlocks = 384;  // these for the haps and these for the reads
+constexpr int kTinyRows = 16;
+// src: the batch descriptor in host memory the device reads (copied to bp.bd)
+hipError_t launch_tiny_prep(const BinParams& bp, const TinyLists& tl, const BatchDesc* src,
+                            int late_begin, hipStream_t st);
+hipError_t launch_tiny_plan(const BinParams& bp, const TinyLists& tl, int grid, hipStream_t st);
+
 // Binning launches.  `hd` is the host copy of the descriptor bp.bd points to;
 // with fixed_grids every grid is independent of the batch sizes (graph
 // capture; `small`: the smaller grids of the small-batch sequence), else
@@ -357,6 +384,8 @@ hipError_t launch_fwd_tile_set_scaled(int NR, bool fast, const FwdParams& p, con
                                       int grid, hipStream_t st);
 // Rows per lane of the wildcard tiles.
 constexpr int kWildRows = 16;
+// Rows per lane, and per tile, of the strips of a long read.
+constexpr int kStripRows = 12, kStripTileRows = 64 * kStripRows;
 // The multi-tile and wildcard bins on the scaled sweep (k_fwd_special).
 struct SpecialSet {
     const WorkItem* items = nullptr;
@@ -369,12 +398,21 @@ struct SpecialSet {
     int32_t* error_flag = nullptr;
 };
 hipError_t launch_fwd_special(const FwdParams& p, const SpecialSet& ss, int grid, hipStream_t st);
+// The whole FP32 pass of a small call; ss: items, range and next_task unused
+// but the task counter, border row and error flag.  What the scaling refuses
+// goes to the rescue lists or, past the FP64 tiles' 512 rows, the final list.
+hipError_t launch_rescue_tiny(const FwdParams& p, const TinyLists& tl, int grid, int64_t* totals,
+                              hipStream_t st);
+hipError_t launch_fwd_tiny(const FwdParams& p, const SpecialSet& ss, const TinyLists& tl, int grid,
+                           hipStream_t st);
 hipError_t launch_fwd_wave_f32(const FwdParams& p, const BinSet& bs, const int32_t* hmax_ptr,
                                float* spill, int64_t spill_elems, int32_t* error_flag, int blocks,
                                hipStream_t st);
+// pack: reads that fit share waves.  totals (may be null): {rescued, of them in FP64}, to which the launch adds
+// the items of its first bin.
 hipError_t launch_fwd_wave_f64(const FwdParams& p, const BinSet& bs, const int32_t* hmax_ptr,
                                double* spill, int64_t spill_elems, int32_t* error_flag, int blocks,
-                               hipStream_t st);
+                               hipStream_t st, bool pack, int64_t* totals = nullptr);
 // Resident blocks of 64 threads per CU for a tile-set instance.
 int tile_set_blocks_per_cu(int NR, bool fast, bool f64, bool roweps = false, bool scaled = false);
 
