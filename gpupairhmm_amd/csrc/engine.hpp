@@ -103,6 +103,7 @@ struct Engine {
         // used in turn; a slot is rewritten once its last call is done.
         Graphs tiny[2];
         BatchDesc* h_tiny = nullptr;
+        int32_t* h_error = nullptr;  // pinned: error flags that kernels set, one word per kind
         hipEvent_t tiny_ev[2] = {};
         bool tiny_used[2] = {};
         int tiny_next = 0;
@@ -156,6 +157,7 @@ struct Engine {
         phmm_batch_view dv{};          // the staged batch on the device
         int64_t table_n = -1;
         bool eager = false;            // launch its kernels one by one (a pipelined piece)
+        bool in_order = false;         // the call's only piece: copied on its own stream
     };
     static constexpr int kSlots = 3;
     Slot slots[kSlots];

@@ -1418,7 +1418,7 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
     const int nblk = (int)(cap_blocks < (int64_t)gridDim.x ? cap_blocks : (int64_t)gridDim.x);
     if (nblk <= 0) {
         if (blockIdx.x == 0 && lane == 0 && n > 0)
-            atomicOr(error_flag, 1);
+            *(volatile int32_t*)error_flag = 1;
         return;
     }
     if ((int)blockIdx.x >= nblk)
@@ -1469,7 +1469,7 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
         }
         if (HL > hmax) {
             if (lane == 0) {
-                atomicOr(error_flag, 2);
+                *(volatile int32_t*)(error_flag + 1) = 1;
                 bd.scores[it.out] = __int_as_float(0x7fc00000);
             }
             continue;
@@ -1943,7 +1943,7 @@ __device__ __forceinline__ bool border_row(const SpecialSet& ss, float4*& border
     const int64_t stride = (int64_t)*ss.hmax + kStripPad;
     if ((int64_t)blockIdx.x >= ss.border_entries / stride) {
         if (blockIdx.x == 0 && threadIdx.x == 0)
-            atomicOr(ss.error_flag, 1);
+            *(volatile int32_t*)ss.error_flag = 1;
         return false;
     }
     border = ss.border + blockIdx.x * stride;

@@ -272,7 +272,7 @@ struct BinParams {
     int32_t* rescue_counts;    // [NB]
     int32_t* retry_counts;     // [kRetrySlots]: retry lists' counts per bin
     int32_t* final_count;      // [1]
-    int32_t* error_flag;       // [1]
+    int32_t* error_flag;       // [2], pinned host memory
     int32_t* task_ctr;         // [kTaskCounters]: task counters of the set launches
     SuperTask* st;             // tile bins' work, in bin_range units
     int32_t* align_range;      // [2*NB]: per bin, begin / count in alignments
