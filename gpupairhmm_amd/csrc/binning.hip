@@ -18,18 +18,18 @@
 
 namespace phmm {
 
-// Several counter arrays zeroed by one launch (a fill kernel rather than
-// memsets, so the sequence can be captured and replayed as a graph).
+// Counter arrays that k_prep zeroes (in a kernel rather than by memsets, so
+// the sequence can be captured and replayed as a graph).
 struct ClearList {
-    int32_t* p[7];
-    int32_t n[7];
+    int32_t* p[6];
+    int32_t n[6];
     int32_t count;
 };
-__global__ void k_clear_list(ClearList cl)
+__device__ __forceinline__ void clear_list(const ClearList& cl, int block, int nblocks)
 {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    const int64_t stride = (int64_t)nblocks * blockDim.x;
     for (int k = 0; k < cl.count; ++k)
-        for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < cl.n[k]; i += stride)
+        for (int64_t i = block * (int64_t)blockDim.x + threadIdx.x; i < cl.n[k]; i += stride)
             cl.p[k][i] = 0;
 }
 
@@ -100,12 +100,6 @@ __device__ __forceinline__ int hap_pass(const BinParams& bp, const BatchDesc& b,
     for (int k = 0; k < (int)(blockDim.x >> 6); ++k)
         bm = max(bm, wmax[k]);
     return bm;
-}
-__global__ __launch_bounds__(256) void k_hap_pass(BinParams bp)
-{
-    const int bm = hap_pass(bp, *bp.bd, blockIdx.x, gridDim.x);
-    if (threadIdx.x == 0 && bm > 0)  // the parts start at 0: blocks without haps skip the atomic
-        atomicMax(&bp.hmax_part[blockIdx.x & (kHmaxParts - 1)], bm);
 }
 
 // Per read (16 lanes each, four reads per wave): its packed rows and its
@@ -258,16 +252,12 @@ __device__ __forceinline__ void read_meta(const BinParams& bp, const BatchDesc& 
         bp.meta[i] = m;
     }
 }
-__global__ __launch_bounds__(256) void k_read_meta(BinParams bp)
-{
-    read_meta(bp, *bp.bd, blockIdx.x, gridDim.x);
-}
-
 // Exclusive prefix of R_g*H_g (the reference's resultOffsetsPerBatch,
-// gpuworker.cuh:802-815), one block of up to 1024 threads, four consecutive
-// groups per thread and pass.
+// gpuworker.cuh:802-815), one block, 16 consecutive groups per thread
+// and pass.
 __device__ __forceinline__ void align_offsets(const BinParams& bp, const BatchDesc& b)
 {
+    constexpr int kPer = 16;
     const int G = b.G, nt = blockDim.x, nwv = nt >> 6;
     __shared__ int64_t wsum[16];
     __shared__ int64_t carry;
@@ -275,13 +265,16 @@ __device__ __forceinline__ void align_offsets(const BinParams& bp, const BatchDe
         carry = 0;
     __syncthreads();
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    for (int base = 0; base < G; base += 4 * nt) {
-        const int g0 = base + 4 * (int)threadIdx.x;
-        int64_t p[4];
+    for (int base = 0; base < G; base += kPer * nt) {
+        const int g0 = base + kPer * (int)threadIdx.x;
+        int64_t p[kPer];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
+        for (int u = 0; u < kPer; ++u)
             p[u] = g0 + u < G ? (int64_t)b.nreads[g0 + u] * b.nhaps[g0 + u] : 0;
-        const int64_t v = p[0] + p[1] + p[2] + p[3];
+        int64_t v = 0;
+#pragma unroll
+        for (int u = 0; u < kPer; ++u)
+            v += p[u];
         int64_t x = v;
         for (int o = 1; o < 64; o <<= 1) {
             const int64_t y = __shfl_up(x, o, 64);
@@ -303,7 +296,7 @@ __device__ __forceinline__ void align_offsets(const BinParams& bp, const BatchDe
         const int64_t incl = x + wsum[wv] + carry;
         int64_t run = incl - v;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
+        for (int u = 0; u < kPer; ++u) {
             if (g0 + u < G)
                 bp.align_off[g0 + u] = run;
             run += p[u];
@@ -316,9 +309,34 @@ __device__ __forceinline__ void align_offsets(const BinParams& bp, const BatchDe
     if (threadIdx.x == 0)
         bp.align_off[G] = carry;
 }
-__global__ __launch_bounds__(1024) void k_align_offsets(BinParams bp)
+// Counters, haps, reads and alignment offsets side by side: none of them needs
+// another's result.  Block 0 forms the offsets (a serial chain over the
+// records), the next nclear blocks clear, nhap blocks take the haps (one
+// maximum each) and the rest the reads, by far the longest.  As four launches
+// in turn: 156 us for 10,000 records of 25 reads of 150 bases, 60 us for 1,000.
+__global__ __launch_bounds__(256) void k_prep(BinParams bp, ClearList cl, int nclear, int nhap)
 {
-    align_offsets(bp, *bp.bd);
+    const BatchDesc b = *bp.bd;
+    int block = blockIdx.x;
+    if (block == 0) {
+        for (int q = nhap + (int)threadIdx.x; q < kHmaxParts; q += blockDim.x)
+            bp.hmax_part[q] = 0;
+        align_offsets(bp, b);
+        return;
+    }
+    block -= 1;
+    if (block < nclear) {
+        clear_list(cl, block, nclear);
+        return;
+    }
+    block -= nclear;
+    if (block < nhap) {
+        const int bm = hap_pass(bp, b, block, nhap);
+        if (threadIdx.x == 0)
+            bp.hmax_part[block] = bm;
+        return;
+    }
+    read_meta(bp, b, block - nhap, (int)gridDim.x - 1 - nclear - nhap);
 }
 
 // Sort key of a unit of group g: bin, then descending hap length (or
@@ -973,7 +991,7 @@ __global__ __launch_bounds__(64 * NW) void k_scatter_t(BinParams bp)
 // the counting sort's passes are latency (a record's runs in turn, atomics of
 // many records on one hap length).  Its tasks need no order -- they are fewer
 // than the device's waves or not many more -- so three kernels write them:
-// k_tiny_desc takes the descriptor from host memory, k_tiny_prep encodes haps
+// k_tiny_desc takes the descriptor from host memory, k_prep encodes haps
 // and reads side by side, k_tiny_plan cuts one record per block into tasks.
 // Before -> after, us per call: 250 reads x 32 haps 226 -> 153, 1000 records of
 // 8 x 4 300 -> 128, 50 records of 8 x 4 133 -> 68.
@@ -992,24 +1010,6 @@ __global__ __launch_bounds__(256) void k_tiny_desc(BinParams bp, TinyLists tl, c
         tl.counts[kTinyFinalRange + i] = i == 2 ? late_begin : 0;
     if (i == 0)
         *bp.task_ctr = 0;
-}
-
-__global__ __launch_bounds__(256) void k_tiny_prep(BinParams bp)
-{
-    const BatchDesc b = *bp.bd;
-    int block = blockIdx.x;
-    if (block == 0) {
-        align_offsets(bp, b);
-        return;
-    }
-    block -= 1;
-    if (block < kTinyHapBlocks) {
-        const int bm = hap_pass(bp, b, block, kTinyHapBlocks);
-        if (threadIdx.x == 0)
-            bp.hmax_part[block] = bm;
-        return;
-    }
-    read_meta(bp, b, block - kTinyHapBlocks, kTinyReadBlocks);
 }
 
 // A record's hap segments for k_tiny_plan (one wave): n = columns / budget of
@@ -1274,7 +1274,8 @@ hipError_t launch_tiny_prep(const BinParams& bp, const TinyLists& tl, const Batc
 {
     static_assert(kTinyHapBlocks <= kHmaxParts, "one maximum per block");
     hipLaunchKernelGGL(k_tiny_desc, dim3(1), dim3(256), 0, st, bp, tl, src, late_begin);
-    hipLaunchKernelGGL(k_tiny_prep, dim3(1 + kTinyHapBlocks + kTinyReadBlocks), dim3(256), 0, st, bp);
+    hipLaunchKernelGGL(k_prep, dim3(1 + kTinyHapBlocks + kTinyReadBlocks), dim3(256), 0, st, bp,
+                       ClearList{}, 0, kTinyHapBlocks);
     return hipGetLastError();
 }
 
@@ -1333,25 +1334,21 @@ hipError_t run_binning(const BinParams& bp, const BatchDesc& hd, bool fixed_grid
     ClearList cl{};
     cl.p[0] = bp.key_count;
     cl.n[0] = bp.NW * kKeysPerBin;
-    cl.p[1] = bp.hmax_part;
-    cl.n[1] = kHmaxParts;
-    cl.p[2] = bp.rescue_counts;
-    cl.n[2] = bp.NB;
-    cl.p[3] = bp.final_count;
-    cl.n[3] = 1;
-    cl.p[4] = bp.task_ctr;
-    cl.n[4] = kTaskCounters;
-    cl.p[5] = bp.align_part;
-    cl.n[5] = kAlignParts * bp.NB;
-    cl.p[6] = bp.retry_counts;
-    cl.n[6] = kRetrySlots;
-    cl.count = 7;
-    hipLaunchKernelGGL(k_clear_list, dim3(fixed_grids && small ? 128 : 512), dim3(tpb), 0, st, cl);
-    if (fixed_grids || hd.nH > 0)  // one wave per hap
-        hipLaunchKernelGGL(k_hap_pass, dim3(grid(hd.nH, tpb / 64, 4096)), dim3(tpb), 0, st, bp);
-    if (fixed_grids || hd.nR > 0)  // 16 lanes per read: rows and bins
-        hipLaunchKernelGGL(k_read_meta, dim3(grid(hd.nR, tpb / 16, 4096)), dim3(tpb), 0, st, bp);
-    hipLaunchKernelGGL(k_align_offsets, dim3(1), dim3(1024), 0, st, bp);
+    cl.p[1] = bp.rescue_counts;
+    cl.n[1] = bp.NB;
+    cl.p[2] = bp.final_count;
+    cl.n[2] = 1;
+    cl.p[3] = bp.task_ctr;
+    cl.n[3] = kTaskCounters;
+    cl.p[4] = bp.align_part;
+    cl.n[4] = kAlignParts * bp.NB;
+    cl.p[5] = bp.retry_counts;
+    cl.n[5] = kRetrySlots;
+    cl.count = 6;
+    const int nclear = 64;
+    const int nhap = std::min(kHmaxParts, grid(hd.nH, tpb / 64, 4096));  // one wave per hap
+    const int nread = grid(hd.nR, tpb / 16, 4096);                       // 16 lanes per read
+    hipLaunchKernelGGL(k_prep, dim3(1 + nclear + nhap + nread), dim3(tpb), 0, st, bp, cl, nclear, nhap);
     if (fixed_grids || hd.G > 0) {
         hipLaunchKernelGGL(k_count_keys_t<1>, dim3(grid(hd.G, 1, 8192)), dim3(64), 0, st, bp);
         hipLaunchKernelGGL(k_count_keys_t<4>, dim3(grid(hd.G, 1, 2048)), dim3(256), 0, st, bp);

@@ -288,7 +288,7 @@ struct BinParams {
     int32_t allow_fast;
 };
 
-// The few-launch sequence of small calls (k_tiny_prep, k_tiny_plan,
+// The few-launch sequence of small calls (k_tiny_desc, k_prep, k_tiny_plan,
 // k_fwd_tiny, k_rescue_tiny and the final pass): its work lists, unsorted,
 // and their counters.  The tables hold 16 rows per lane throughout.
 struct TinyLists {
@@ -298,7 +298,7 @@ struct TinyLists {
     WorkItem* exact;      // exact bin
     WorkItem* rescue[2];  // what the scaling refused, by form: FP64 tiles
     WorkItem* late;       // what the FP64 tiles could not finish
-    int32_t* counts;      // kTinyCounts counters, zeroed by k_tiny_prep
+    int32_t* counts;      // kTinyCounts counters, zeroed by k_tiny_desc
 };
 enum {
     kTinyFast, kTinySafe, kTinyStrips, kTinyWilds, kTinyExact, kTinyRescueFast, kTinyRescueSafe,
@@ -307,7 +307,7 @@ enum {
     // then the two lists' begins in BinSet's form, from final_items
     kTinyFinalRange = kTinyCounts, kTinyWords = kTinyFinalRange + 4
 };
-constexpr int kTinyHapBlocks = 128;   // grid of k_tiny_prep: one control block,
+constexpr int kTinyHapBlocks = 128;   // grid of a small call's k_prep: block 0,
 constexpr int kTinyReadBlocks = 384;  // these for the haps and these for the reads
 constexpr int kTinyRows = 16;
 // src: the batch descriptor in host memory the device reads (copied to bp.bd)
