@@ -1070,11 +1070,11 @@ __device__ __forceinline__ int set_find(const SetLane& s, int task)
 // the end).  In between neither holds: from the end, large tasks start too late
 // (400 records of 16 x 8 with 2-5 kb haps: 5417 us, 5312 from the counter), and
 // from the front they are held back (300 records of the mixed batch: 13290 us,
-// 13100 from the counter).
+// 13100 from the counter).  `blocks`: the blocks that take tasks, the first
+// ones of the launch.
 constexpr int kFrontRounds = 4, kTailRounds = 8;  // tasks per block
-__device__ __forceinline__ int next_task(int32_t* ctr, int total, bool first)
+__device__ __forceinline__ int next_task(int32_t* ctr, int total, int blocks, bool first)
 {
-    const int blocks = gridDim.x;
     const bool front = total < kFrontRounds * blocks, tail = total >= kTailRounds * blocks;
     if (first && (front || tail))
         return tail ? total - 1 - (int)blockIdx.x : (int)blockIdx.x;
@@ -1112,8 +1112,8 @@ __device__ __forceinline__ int tile_set_tasks(const FwdParams& p, const BinSet& 
                                               int total)
 {
     int done = 0;
-    for (int task = next_task(bs.next_task, total, true); task < total;
-         task = next_task(bs.next_task, total, false)) {
+    for (int task = next_task(bs.next_task, total, gridDim.x, true); task < total;
+         task = next_task(bs.next_task, total, gridDim.x, false)) {
         // the task's bin, in scalar registers (uniform across the wave)
         const int k = set_find(sl, task);
         const int bin = __builtin_amdgcn_readfirstlane(__shfl(sl.bin, k, 64));
@@ -1936,18 +1936,18 @@ __device__ __forceinline__ int special_task(const FwdParams& p, float4* tab, flo
     }
     return 0;
 }
-// The block's border row: false where the arena holds none for it (the
-// launch's first block then reports it).
-__device__ __forceinline__ bool border_row(const SpecialSet& ss, float4*& border)
+
+// The block's border row; returns how many of the launch's first blocks the
+// arena holds one for (the others take no task; none: the first block reports
+// it).
+__device__ __forceinline__ int border_row(const SpecialSet& ss, float4*& border)
 {
     const int64_t stride = (int64_t)*ss.hmax + kStripPad;
-    if ((int64_t)blockIdx.x >= ss.border_entries / stride) {
-        if (blockIdx.x == 0 && threadIdx.x == 0)
-            *(volatile int32_t*)ss.error_flag = 1;
-        return false;
-    }
+    const int64_t rows = ss.border_entries / stride;
+    if (rows <= 0 && blockIdx.x == 0 && threadIdx.x == 0)
+        *(volatile int32_t*)ss.error_flag = 1;
     border = ss.border + blockIdx.x * stride;
-    return true;
+    return (int)(rows < (int64_t)gridDim.x ? rows : (int64_t)gridDim.x);
 }
 
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_fwd_special(
@@ -1960,15 +1960,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
     const WorkItem* strips = ss.items + ss.range[2 * ss.strip_bin];
     const WorkItem* wilds = ss.items + ss.range[2 * ss.wild_bin];
     float4* border = nullptr;
-    if (nm > 0 && !border_row(ss, border))
+    const int blocks = nm > 0 ? border_row(ss, border) : (int)gridDim.x;
+    if ((int)blockIdx.x >= blocks)
         return;
     const BatchDesc bd = *p.bd;
     p.bd = &bd;
     const int run = wild_run(nw);
     const int total = nm + (nw + run - 1) / run;
     int done = 0;
-    for (int task = next_task(ss.next_task, total, true); task < total;
-         task = next_task(ss.next_task, total, false))
+    for (int task = next_task(ss.next_task, total, blocks, true); task < total;
+         task = next_task(ss.next_task, total, blocks, false))
         done += special_task(p, tab, border, strips, nm, wilds, nw, run, ss.strip_bin,
                              __builtin_amdgcn_readfirstlane(task));
     if (done > 0 && threadIdx.x == 0)
@@ -1979,15 +1980,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 // strips and wildcard items, in that order from one counter.
 template <bool GE>
 __device__ __forceinline__ int tiny_tasks(const FwdParams& p, const SpecialSet& ss,
-                                          const TinyLists& tl, float4* tab, float4* border)
+                                          const TinyLists& tl, float4* tab, float4* border,
+                                          int blocks)
 {
     const int nf = tl.counts[kTinyFast], ns = tl.counts[kTinySafe];
     const int nm = tl.counts[kTinyStrips], nw = tl.counts[kTinyWilds];
     const int run = wild_run(nw);
     const int total = nf + ns + nm + (nw + run - 1) / run;
     int done = 0;
-    for (int task = next_task(ss.next_task, total, true); task < total;
-         task = next_task(ss.next_task, total, false)) {
+    for (int task = next_task(ss.next_task, total, blocks, true); task < total;
+         task = next_task(ss.next_task, total, blocks, false)) {
         task = __builtin_amdgcn_readfirstlane(task);
         if (task < nf + ns) {
             const bool fast = task < nf;
@@ -2016,12 +2018,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
     static_assert(TabShape<float, kTinyRows>::kWords <= kSpecialTab, "one table for all");
     __shared__ float4 tab[kSpecialTab];
     float4* border = nullptr;
-    if (tl.counts[kTinyStrips] > 0 && !border_row(ss, border))
+    const int blocks = tl.counts[kTinyStrips] > 0 ? border_row(ss, border) : (int)gridDim.x;
+    if ((int)blockIdx.x >= blocks)
         return;
     const BatchDesc bd = *p.bd;
     p.bd = &bd;
-    const int done = p.semantics == 0 ? tiny_tasks<true>(p, ss, tl, tab, border)
-                                      : tiny_tasks<false>(p, ss, tl, tab, border);
+    const int done = p.semantics == 0 ? tiny_tasks<true>(p, ss, tl, tab, border, blocks)
+                                      : tiny_tasks<false>(p, ss, tl, tab, border, blocks);
     if (done > 0 && threadIdx.x == 0)
         atomicAdd(p.scaled_total, (unsigned long long)done);
 }

@@ -51,3 +51,25 @@ def test_every_copy_once(lib, oracle, copies):
     assert np.isfinite(got).all()
     assert (got == got[0]).all()
     assert np.max(np.abs(got[0].astype(np.float64) - ref)) <= TOL
+
+
+@pytest.mark.parametrize("small_batch", [0, 1 << 18])
+@pytest.mark.parametrize("hap_len", [600, 120000])
+def test_more_long_reads_than_border_rows(lib, oracle, small_batch, hap_len):
+    """The longest hap of a batch sets the size of a border row, so one long
+    hap leaves rows for 139 blocks only (256 MiB at 16 bytes a column): every
+    long read must still be scored, also those after the last block's.  Reads
+    of 1,030 rows against 600 columns: 1,630 roundings of 2^-24, 5e-5 in
+    log10."""
+    import gpupairhmm_amd as G
+    rng = np.random.default_rng(29)
+    text = _record(rng, (12,), ["".join(rng.choice(list("ACGT"), hap_len))])
+    text += _record(rng, (1030,) * 300, ["".join(rng.choice(list("ACGT"), 600))])
+    text += _record(rng, (40,) * 20, ["".join(rng.choice(list("ACGT"), 90)),
+                                      "".join(rng.choice(list("ACGTN"), 90))])
+    b = G.HostBatch.parse(text)
+    say(f"case: hap {hap_len}, small_batch {small_batch}, {b.num_alignments} alignments")
+    ref = oracle.score_batch(b.oracle_arrays(), oracle.F64, semantics=G.SEM_GPU)
+    with G.Engine(small_batch=small_batch) as e:
+        got = e.score_batch(b)
+    assert np.max(np.abs(got.astype(np.float64) - ref)) <= TOL
