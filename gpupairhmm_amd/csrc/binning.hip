@@ -991,19 +991,18 @@ __global__ __launch_bounds__(64 * NW) void k_scatter_t(BinParams bp)
 // the counting sort's passes are latency (a record's runs in turn, atomics of
 // many records on one hap length).  Its tasks need no order -- they are fewer
 // than the device's waves or not many more -- so three kernels write them:
-// k_tiny_desc takes the descriptor from host memory, k_prep encodes haps
+// k_tiny_desc brings the descriptor in its arguments, k_prep encodes haps
 // and reads side by side, k_tiny_plan cuts one record per block into tasks.
 // Before -> after, us per call: 250 reads x 32 haps 226 -> 153, 1000 records of
 // 8 x 4 300 -> 128, 50 records of 8 x 4 133 -> 68.
-// late_begin: where tl.late starts, counted from the final list.
-__global__ __launch_bounds__(256) void k_tiny_desc(BinParams bp, TinyLists tl, const BatchDesc* src,
+// (The descriptor first lay in pinned memory that the kernel read, which held
+// a caller back after two calls: 131 us for the 1000 records, 125 so.)
+__global__ __launch_bounds__(256) void k_tiny_desc(BinParams bp, TinyLists tl, BatchDesc d,
                                                    int late_begin)
 {
-    static_assert(sizeof(BatchDesc) % 4 == 0 && sizeof(BatchDesc) / 4 <= 256, "one word per thread");
     const int i = threadIdx.x;
-    if (i < (int)(sizeof(BatchDesc) / 4))
-        reinterpret_cast<uint32_t*>(const_cast<BatchDesc*>(bp.bd))[i] =
-            reinterpret_cast<const volatile uint32_t*>(src)[i];
+    if (i == 0)
+        *const_cast<BatchDesc*>(bp.bd) = d;
     if (i < kTinyCounts)
         tl.counts[i] = 0;
     if (i < 4)
@@ -1269,11 +1268,16 @@ __global__ __launch_bounds__(256) void k_tiny_plan(BinParams bp, TinyLists tl)
     }
 }
 
-hipError_t launch_tiny_prep(const BinParams& bp, const TinyLists& tl, const BatchDesc* src,
+hipError_t launch_tiny_desc(const BinParams& bp, const TinyLists& tl, const BatchDesc& d,
                             int late_begin, hipStream_t st)
 {
+    hipLaunchKernelGGL(k_tiny_desc, dim3(1), dim3(256), 0, st, bp, tl, d, late_begin);
+    return hipGetLastError();
+}
+
+hipError_t launch_tiny_prep(const BinParams& bp, hipStream_t st)
+{
     static_assert(kTinyHapBlocks <= kHmaxParts, "one maximum per block");
-    hipLaunchKernelGGL(k_tiny_desc, dim3(1), dim3(256), 0, st, bp, tl, src, late_begin);
     hipLaunchKernelGGL(k_prep, dim3(1 + kTinyHapBlocks + kTinyReadBlocks), dim3(256), 0, st, bp,
                        ClearList{}, 0, kTinyHapBlocks);
     return hipGetLastError();

@@ -119,14 +119,9 @@ void Engine::free_ctx(CallCtx& c)
         hipHostFree(c.h_desc);
     if (c.h_bin_range)
         hipHostFree(c.h_bin_range);
-    if (c.h_tiny)
-        hipHostFree(c.h_tiny);
     if (c.h_error)
         hipHostFree(c.h_error);
     for (auto& ev : c.desc_ev)
-        if (ev)
-            hipEventDestroy(ev);
-    for (auto& ev : c.tiny_ev)
         if (ev)
             hipEventDestroy(ev);
     if (c.call_done)
@@ -180,9 +175,6 @@ int Engine::init_ctx(int k)
         (rc = check(hipHostMalloc(reinterpret_cast<void**>(&c.h_desc),
                                   sizeof(BatchDesc) * kDescRing, hipHostMallocDefault),
                     "pinned descriptors")) ||
-        (rc = check(hipHostMalloc(reinterpret_cast<void**>(&c.h_tiny), sizeof(BatchDesc) * 2,
-                                  hipHostMallocDefault),
-                    "pinned descriptors")) ||
         (rc = check(hipHostMalloc(reinterpret_cast<void**>(&c.h_error), sizeof(int32_t) * 2,
                                   hipHostMallocDefault),
                     "pinned error flags")) ||
@@ -193,9 +185,6 @@ int Engine::init_ctx(int k)
         return rc;
     for (int i = 0; i < kDescRing; ++i)
         if ((rc = check(hipEventCreateWithFlags(&c.desc_ev[i], hipEventDisableTiming), "event")))
-            return rc;
-    for (hipEvent_t& ev : c.tiny_ev)
-        if ((rc = check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "event")))
             return rc;
     c.h_error[0] = c.h_error[1] = 0;
     if ((rc = check(hipEventCreateWithFlags(&c.call_done, hipEventDisableTiming), "event")))
@@ -452,7 +441,7 @@ int Engine::score_device(const phmm_batch_view& v, float* d_scores, hipStream_t 
     const bool plain = opt.mode == PHMM_MODE_PLAIN;
     const bool eager = plain || !opt.graphs || arena || eager_hint;
     const int dk = c.desc_next;
-    if (!tiny || eager) {
+    if (!tiny) {
         const int k = dk;
         c.desc_next = (c.desc_next + 1) % kDescRing;
         if (c.desc_used[k] && (rc = check(hipEventSynchronize(c.desc_ev[k]), "descriptor slot")))
@@ -580,7 +569,7 @@ int Engine::score_device(const phmm_batch_view& v, float* d_scores, hipStream_t 
     };
     if (!eager && c.graphs[0].gen != c.generation) {
         drop_graphs(c);
-        for (Graphs* g : {&c.graphs[0], &c.graphs[1], &c.tiny[0], &c.tiny[1]})
+        for (Graphs* g : {&c.graphs[0], &c.graphs[1], &c.tiny})
             g->gen = c.generation;
     }
     if (tiny) {
@@ -599,25 +588,12 @@ int Engine::score_device(const phmm_batch_view& v, float* d_scores, hipStream_t 
         tl.counts = bp.task_ctr + 1;
         static_assert(1 + kTinyWords <= kTaskCounters, "counters");
         fp.final_count = tl.counts + kTinyFinal;
-        if (eager) {
-            if ((rc = stages([&](int which) {
-                     return enqueue_tiny(which, bp, fp, tl, &c.h_desc[dk], st);
-                 })) ||
-                (rc = check(hipEventRecord(c.desc_ev[dk], st), "event")))
-                return rc;
-        } else {
-            const int k = c.tiny_next;
-            c.tiny_next ^= 1;
-            if (c.tiny_used[k] && (rc = check(hipEventSynchronize(c.tiny_ev[k]), "descriptor slot")))
-                return rc;
-            c.h_tiny[k] = hd;
-            if ((rc = graph_of(c.tiny[k], [&](int which, hipStream_t cs) {
-                     return enqueue_tiny(which, bp, fp, tl, &c.h_tiny[k], cs);
-                 })) ||
-                (rc = check(hipEventRecord(c.tiny_ev[k], st), "event")))
-                return rc;
-            c.tiny_used[k] = true;
-        }
+        if ((rc = check(launch_tiny_desc(bp, tl, hd, (int)(tl.late - fp.final_items), st), "descriptor kernel")) ||
+            (rc = eager ? stages([&](int which) { return enqueue_tiny(which, bp, fp, tl, st); })
+                        : graph_of(c.tiny, [&](int which, hipStream_t cs) {
+                              return enqueue_tiny(which, bp, fp, tl, cs);
+                          })))
+            return rc;
     } else if (eager) {
         if ((rc = enqueue_prep(bp, hd, false, st)))
             return rc;
@@ -1038,12 +1014,12 @@ bool Engine::tiny_call(const phmm_batch_view& v) const
 }
 
 int Engine::enqueue_tiny(int stages, const BinParams& bp, const FwdParams& fp, const TinyLists& tl,
-                         const BatchDesc* src, hipStream_t st)
+                         hipStream_t st)
 {
     int rc;
     const int waves = num_cus * 8;
     if ((stages & kStagePrep) &&
-        ((rc = check(launch_tiny_prep(bp, tl, src, (int)(tl.late - fp.final_items), st), "preparation kernel")) ||
+        ((rc = check(launch_tiny_prep(bp, st), "preparation kernel")) ||
          (rc = check(launch_tiny_plan(bp, tl, 512, st), "planning kernel"))))
         return rc;
     if (stages & kStageFwd) {
@@ -1132,7 +1108,7 @@ void Engine::derive_small_tiles()
 void Engine::drop_graphs(CallCtx& c)
 {
     std::vector<hipGraphExec_t*> all;
-    for (Graphs* g : {&c.graphs[0], &c.graphs[1], &c.tiny[0], &c.tiny[1]})
+    for (Graphs* g : {&c.graphs[0], &c.graphs[1], &c.tiny})
         for (hipGraphExec_t* x : {&g->all, &g->prep, &g->fwd, &g->rescue})
             if (*x)
                 all.push_back(x);

@@ -98,15 +98,8 @@ struct Engine {
         // are captured again.
         uint64_t generation = 0;
         Graphs graphs[2];  // [0]: tuned table, [1]: small-batch table
-        // The few-launch sequence of small calls reads its descriptor from
-        // pinned memory, so a captured graph belongs to one of two slots,
-        // used in turn; a slot is rewritten once its last call is done.
-        Graphs tiny[2];
-        BatchDesc* h_tiny = nullptr;
+        Graphs tiny;  // the few-launch sequence of small calls
         int32_t* h_error = nullptr;  // pinned: error flags that kernels set, one word per kind
-        hipEvent_t tiny_ev[2] = {};
-        bool tiny_used[2] = {};
-        int tiny_next = 0;
         // the current call's spill arena (spill, or the rest of an arena)
         void* call_spill = nullptr;
         size_t call_spill_bytes = 0;
@@ -232,7 +225,7 @@ struct Engine {
     double tiny_columns(const phmm_batch_view& v) const;
     bool tiny_call(const phmm_batch_view& v) const;
     int enqueue_tiny(int stages, const BinParams& bp, const FwdParams& fp, const TinyLists& tl,
-                     const BatchDesc* src, hipStream_t st);
+                     hipStream_t st);
     void drop_graphs(CallCtx& c);
     void free_ctx(CallCtx& c);
     int score_batch(const phmm_batch_view& v, float* out);

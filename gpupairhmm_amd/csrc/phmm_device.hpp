@@ -310,9 +310,11 @@ enum {
 constexpr int kTinyHapBlocks = 128;   // grid of a small call's k_prep: block 0,
 constexpr int kTinyReadBlocks = 384;  // these for the haps and these for the reads
 constexpr int kTinyRows = 16;
-// src: the batch descriptor in host memory the device reads (copied to bp.bd)
-hipError_t launch_tiny_prep(const BinParams& bp, const TinyLists& tl, const BatchDesc* src,
+// d: the call's descriptor, written to bp.bd by a kernel that has it as an
+// argument; late_begin: where tl.late starts, counted from the final list
+hipError_t launch_tiny_desc(const BinParams& bp, const TinyLists& tl, const BatchDesc& d,
                             int late_begin, hipStream_t st);
+hipError_t launch_tiny_prep(const BinParams& bp, hipStream_t st);
 hipError_t launch_tiny_plan(const BinParams& bp, const TinyLists& tl, int grid, hipStream_t st);
 
 // Binning launches.  `hd` is the host copy of the descriptor bp.bd points to;
