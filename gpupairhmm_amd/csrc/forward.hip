@@ -273,7 +273,7 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
         }
         T pb[NR], de[NR], si[NR], er[ROWEPS ? NR + 1 : 1];
 #pragma unroll
-        for (int j = 0; j < NR; ++j) {  // (the packed rows' qualities are at most 127)
+        for (int j = 0; j < NR; ++j) {  // (row accessors stay within the table)
             pb[j] = (T)p.ph2pr[row_bq(w[j])];
             de[j] = (T)p.ph2pr[row_iq(w[j])];
             si[j] = (T)p.ph2pr[row_dq(w[j])];

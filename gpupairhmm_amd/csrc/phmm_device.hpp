@@ -98,11 +98,14 @@ constexpr float kEpsGpu = 0.1f;
 constexpr float kBetaGpu = 0.9f;
 
 // Packed read row: base code | base q << 8 | ins q << 16 | del q << 24,
-// qualities clamped to 127.
+// qualities clamped to 127.  The quality accessors take 7 bits, so that any
+// word indexes the 128-entry probability table within its bounds: lanes
+// without a read load row 0 of the batch, which nothing has written where the
+// first read is empty.
 __host__ __device__ inline int row_code(uint32_t w) { return (int)(w & 0xffu); }
-__host__ __device__ inline int row_bq(uint32_t w) { return (int)((w >> 8) & 0xffu); }
-__host__ __device__ inline int row_iq(uint32_t w) { return (int)((w >> 16) & 0xffu); }
-__host__ __device__ inline int row_dq(uint32_t w) { return (int)(w >> 24); }
+__host__ __device__ inline int row_bq(uint32_t w) { return (int)((w >> 8) & 0x7fu); }
+__host__ __device__ inline int row_iq(uint32_t w) { return (int)((w >> 16) & 0x7fu); }
+__host__ __device__ inline int row_dq(uint32_t w) { return (int)((w >> 24) & 0x7fu); }
 
 // A/C/G/T -> 0..3, every other byte -> 4 (utility_kernels.cuh:16-20).
 __host__ __device__ inline int base_code(uint8_t b)

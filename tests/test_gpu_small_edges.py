@@ -1,0 +1,97 @@
+"""Small calls at the edges of their inputs."""
+import numpy as np
+import pytest
+
+from conftest import say
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-3  # the parity bar; rows x columns as in test_gpu_small
+
+
+def _seq(rng, n, letters="ACGT"):
+    return "".join(rng.choice(list(letters), n))
+
+
+NAMES = ("read_data", "hap_data", "base_quals", "ins_quals", "del_quals", "gcp_quals",
+         "read_lengths", "hap_lengths", "read_offsets", "hap_offsets", "num_reads_per_group",
+         "num_haps_per_group", "reads_prefix", "haps_prefix")
+
+
+def _batch(rng, records):
+    """A batch of (reads, haps) records, sequences given as text, which may be
+    empty; qualities 2 to 40, gaps 45 or, every other read, 25 to 45."""
+    import gpupairhmm_amd as G
+    reads = [r for rs, _ in records for r in rs]
+    haps = [h for _, hs in records for h in hs]
+
+    def pack(seqs, make, pad):
+        out = []
+        for i, s in enumerate(seqs):
+            out.append(np.asarray(make(i, s), np.uint8))
+            out.append(np.full(4 - len(s) % 4, pad, np.uint8))
+        return np.concatenate(out)
+
+    def offsets(seqs):
+        return np.concatenate([[0], np.cumsum([len(s) + 4 - len(s) % 4 for s in seqs])])
+
+    def text(_, s):
+        return np.frombuffer(s.encode(), np.uint8)
+
+    def gaps(i, s):
+        return np.full(len(s), 45) if i % 2 == 0 else rng.integers(25, 46, len(s))
+
+    gap = pack(reads, gaps, 45)
+    return G.HostBatch.from_arrays(
+        read_data=pack(reads, text, ord("N")), hap_data=pack(haps, text, ord("N")),
+        base_quals=pack(reads, lambda i, s: rng.integers(2, 41, len(s)), 45),
+        ins_quals=gap, del_quals=gap,
+        gcp_quals=pack(reads, lambda i, s: np.full(len(s), 10), 45),
+        read_lengths=[len(r) for r in reads], hap_lengths=[len(h) for h in haps],
+        read_offsets=offsets(reads), hap_offsets=offsets(haps),
+        num_reads_per_group=[len(rs) for rs, _ in records],
+        num_haps_per_group=[len(hs) for _, hs in records],
+        reads_prefix=np.concatenate([[0], np.cumsum([len(rs) for rs, _ in records])]),
+        haps_prefix=np.concatenate([[0], np.cumsum([len(hs) for _, hs in records])]))
+
+
+def _bits(a):
+    return np.asarray(a, np.float32).view(np.uint32)
+
+
+@pytest.mark.parametrize("semantics", [0, 1])
+def test_empty_reads_and_haps(lib, oracle, semantics):
+    """Empty reads, the batch's first among them (whose packed row nothing
+    writes, and lanes without a read load it), empty haps and records of
+    nothing else: -inf where the oracle says so, on every route."""
+    import gpupairhmm_amd as G
+    rng = np.random.default_rng(41)
+    hap = _seq(rng, 260)
+    b = _batch(rng, [
+        (["", hap[:150], "", hap[40:190]], [hap, "", _seq(rng, 90), ""]),
+        (["", ""], [hap[:70], ""]),
+        ([hap[:30]], [""]),
+        ([hap[10:110], "", hap[:61]] + [hap[i:i + 101] for i in range(20)], ["", hap, hap[:200] + "N"]),
+        (["", _seq(rng, 1100)], [_seq(rng, 1200), ""]),
+    ])
+    say(f"case: empty reads and haps, semantics {semantics}, {b.num_alignments} alignments")
+    ref = oracle.score_batch(b.oracle_arrays(), oracle.F64, semantics=semantics)
+    fin = np.isfinite(ref)
+    assert 0 < fin.sum() < len(ref)
+    with G.Engine(semantics=semantics, mode=G.MODE_PLAIN) as e:
+        want = e.score_batch(b)
+    assert np.all(want[~fin] == -np.inf)
+    assert np.max(np.abs(want[fin].astype(np.float64) - ref[fin])) <= TOL
+    for kw in ({}, {"graphs": False}, {"small_batch": 0}, {"time_kernels": True}):
+        with G.Engine(semantics=semantics, **kw) as e:
+            got = e.score_batch(b)
+            assert np.all(got[~fin] == -np.inf)
+            assert np.max(np.abs(got[fin].astype(np.float64) - ref[fin])) <= TOL
+            if "small_batch" not in kw:
+                assert np.array_equal(_bits(got), _bits(want)), kw
+            db, out = e.upload(b), e.alloc(4 * b.num_alignments)
+            e.score_device_noalloc(db, out)
+            e.synchronize()
+            assert np.array_equal(_bits(e.download(out, b.num_alignments)), _bits(got)), kw
+            e.free(out)
+            db.free()
