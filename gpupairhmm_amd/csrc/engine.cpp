@@ -253,9 +253,11 @@ void Engine::scratch_sizes(const phmm_batch_view& v, int NB, int NW, size_t out[
     out[kRescueExps] = (size_t)kReKnownLanes * nA;
     // small calls: the SAFE super-tasks, strips, exact-bin items, SAFE rescue
     // list, final and late lists (their other lists are in the arrays above),
-    // at offsets that follow from the buffer's size
+    // at offsets that follow from the buffer's size.  A larger batch never
+    // needs less, also where it is no small call itself: a server reserves
+    // for its largest launch, and the launches below that must fit.
     size_t cap = 1 << 16;
-    while (nA <= (size_t)kTinyAlignments && cap < nA)
+    while (cap < std::min(nA, (size_t)kTinyAlignments))
         cap *= 2;
     out[kTinyScratch] = kTinyBytes * cap;
 }

@@ -1,4 +1,6 @@
 """Small calls at the edges of their inputs."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -95,3 +97,36 @@ def test_empty_reads_and_haps(lib, oracle, semantics):
             assert np.array_equal(_bits(e.download(out, b.num_alignments)), _bits(got)), kw
             e.free(out)
             db.free()
+
+
+def test_server_launches_fit_the_reservation(lib):
+    """A server's launch contexts are reserved at creation for the largest
+    launch; merged launches of every size below it, among them small calls on
+    either side of the powers of two of their lists' capacity, take no more
+    device memory and capture no graph anew."""
+    import gpupairhmm_amd as G
+
+    def free_bytes():  # the library's own HIP runtime
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    rng = np.random.default_rng(43)
+    reads = [_seq(rng, 40) for _ in range(500)]
+    sizes = (40000, 65500, 66000, 131000, 131500, 262000)
+    batches = [_batch(rng, [(reads, [_seq(rng, 60) for _ in range(n // 500)])]) for n in sizes]
+    with G.Engine() as e:
+        alone = [e.score_batch(b) for b in batches]
+    with G.Engine() as e:
+        srv = G.Server(e, hbm_budget_bytes=4 << 30)
+        try:
+            seen = []
+            for n, b, want in zip(sizes, batches, alone):
+                say(f"case: server launch of {n} alignments")
+                assert srv.submit(b, n)
+                tag, got, _ = srv.poll(timeout_ms=20000, capacity=n)
+                assert tag == n and np.array_equal(_bits(got), _bits(want))
+                seen.append((free_bytes(), e.stats().graph_captures))
+            assert len(set(seen)) == 1, seen
+        finally:
+            srv.close()
