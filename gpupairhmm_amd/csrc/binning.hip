@@ -110,9 +110,9 @@ __device__ __forceinline__ int hap_pass(const BinParams& bp, const BatchDesc& b,
 // row whose max_read_len covers the read (its tile has room for one more
 // row); reads beyond the last row go to the multi-tile bin 2*ntiles.  Bin 2k
 // uses the rescaled (FAST) arithmetic when the read's coefficients keep it in
-// range, else bin 2k+1 (SAFE; a multi-tile read's form is the sign of its
-// nl); under per-position gcp every row's eps enters the check.  Reference CPU and per-position gcp semantics: a read
-// holding a byte other than A/C/G/T/N goes to the exact bin 2*ntiles+1.  The slot
+// range, else bin 2k+1 (SAFE); under per-position gcp every row's eps enters
+// the check.  Reference CPU and per-position gcp semantics: a read holding a
+// byte other than A/C/G/T/N goes to the exact bin 2*ntiles+1.  The slot
 // combines its lanes' verdicts and the product of alpha with row-local
 // reductions.
 // Block `block` of `nblocks` (256 threads).
@@ -241,17 +241,19 @@ __device__ __forceinline__ void read_meta(const BinParams& bp, const BatchDesc& 
             m.bin = -1;
         } else if (bp.semantics != 0 && exv) {
             m.bin = 2 * bp.ntiles + 1;
+        } else if (k == bp.ntiles) {
+            m.bin = 2 * bp.ntiles;
         } else {
             bool fast = okv && bp.allow_fast != 0 && eps <= 0.5f;
             if (fast && !(nl >= 1e-30))  // the start constant must stay a normal float
                 fast = false;
-            const bool multi = k == bp.ntiles;
-            m.nl = fast ? (float)nl : multi ? -1.0f : 1.0f;
-            m.bin = multi ? 2 * k : 2 * k + (fast ? 0 : 1);
+            m.nl = fast ? (float)nl : 1.0f;
+            m.bin = 2 * k + (fast ? 0 : 1);
         }
         bp.meta[i] = m;
     }
 }
+
 // Exclusive prefix of R_g*H_g (the reference's resultOffsetsPerBatch,
 // gpuworker.cuh:802-815), one block, 16 consecutive groups per thread
 // and pass.
@@ -309,6 +311,7 @@ __device__ __forceinline__ void align_offsets(const BinParams& bp, const BatchDe
     if (threadIdx.x == 0)
         bp.align_off[G] = carry;
 }
+
 // Counters, haps, reads and alignment offsets side by side: none of them needs
 // another's result.  Block 0 forms the offsets (a serial chain over the
 // records), the next nclear blocks clear, nhap blocks take the haps (one

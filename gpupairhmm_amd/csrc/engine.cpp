@@ -1026,7 +1026,6 @@ int Engine::enqueue_tiny(int stages, const BinParams& bp, const FwdParams& fp, c
         return rc;
     if (stages & kStageFwd) {
         SpecialSet ss;
-        ss.strip_bin = 2 * bp.ntiles;
         ss.next_task = bp.task_ctr;
         ss.hmax = bp.hmax;
         ss.border = static_cast<float4*>(cur->call_spill);

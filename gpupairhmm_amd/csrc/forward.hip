@@ -182,6 +182,8 @@ struct TileRead {
     // factors (each <= 1) are left out, which can only put the estimate below
     // the true floor.  (In-pass scaling; one gap continuation per read.)
     float floor2;
+    float drift;  // strips: sum over the lane's rows of what rounding took from
+                  // the factors of a match, relative
 };
 
 // Gap continuation of the D chain of row j.
@@ -219,7 +221,9 @@ __device__ __forceinline__ T beta_of(T e)
 // c3 = eps_r beta_{r+1} / beta_r, and D chain Dh = M< + eps_r Dh<; the last
 // row's beta_{L+1} is taken as beta_L, which the epilogue divides out.
 //
-// row0: the first row of the tile (reads of several tiles).
+// row0: the first row of the tile (reads of several tiles).  NL 5: the strips'
+// setup, once per 768 rows, with correctly rounded quotients and the rows'
+// drift (see strip_task).
 template <typename T, int NR, bool FAST, bool ROWEPS, int NL = 4>
 __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTraits<T>::V* tab,
                                            bool active, int read, int t,
@@ -237,6 +241,7 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
         if (FAST)
             nl = p.meta[read].nl;
     }
+    auto div = [](T a, T b) { return NL == 5 ? a / b : qdiv(a, b); };
     T eps = (T)kEpsGpu, beta = (T)kBetaGpu;
     if (p.semantics != 0 && active && L > 0) {
         // reference CPU semantics: the read's first gcp quality; per-position
@@ -293,6 +298,7 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
         R.floor2 = (float)lrow * __log2f((float)eps);
         if (FAST && lrow > 0)
             R.floor2 += __log2f(p.ph2pr[row_iq(p.rows[roff])]) - __log2f((float)de[NR - 1]);
+        R.drift = 0.f;
         T lm[NR], lx[NR];
         int code[NR];
 #pragma unroll
@@ -310,11 +316,17 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
             }
             code[j] = in ? row_code(w[j]) : 4;
             lm[j] = in ? (T)1 - pb[j] : (T)0;
-            lx[j] = in ? qdiv(pb[j], (T)3) : (T)0;
+            lx[j] = in ? div(pb[j], (T)3) : (T)0;
+            if constexpr (NL == 5) {
+                const double da = (1.0 - ((double)delta + (double)sigma)) - (double)alpha;
+                const double dm = (1.0 - (double)pb[j]) - (double)lm[j];
+                R.drift += (in && alpha > 0 ? qdiv((float)da, alpha) : 0.f) +
+                           (in && lm[j] > 0 ? qdiv((float)dm, lm[j]) : 0.f);
+            }
             if (FAST) {
-                const T c0 = qdiv(br * pdelta, palpha * alpha);
-                const T c1 = qdiv(top ? br : br * psigma, alpha);
-                const T c2 = qdiv(in ? e * pdelta : pdelta, in ? delta * palpha : palpha);
+                const T c0 = div(br * pdelta, palpha * alpha);
+                const T c1 = div(top ? br : br * psigma, alpha);
+                const T c2 = div(in ? e * pdelta : pdelta, in ? delta * palpha : palpha);
                 R.c10[j].y = in && !top ? c0 : (T)0;
                 R.c10[j].x = in ? c1 : (T)0;
                 R.c32[j].y = in ? (top ? (T)0 : c2) : firstoob ? c2 : (T)1;
@@ -324,7 +336,7 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
                 R.c10[j].x = in ? (top ? br : br * psigma) : (T)0;
                 R.c32[j].y = in ? bn * delta : firstoob ? beta : (T)0;
                 // equal betas keep eps exactly (no rounding of bn / br)
-                R.c32[j].x = in ? (bn == br ? e : qdiv(e * bn, br)) : (T)1;
+                R.c32[j].x = in ? (bn == br ? e : div(e * bn, br)) : (T)1;
                 if constexpr (ROWEPS)
                     R.c4[j] = in ? e : (T)0;
             }
@@ -1679,7 +1691,7 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
 // fifth letter.  Bound by the VALU like the tile kernels.  The one-wave
 // kernel, with 1024-row tiles, an exponent check of every row per column and
 // FP64 for what falls below the FP32 range, took 23.5 ms for 2,560 alignments
-// of 1100-1500-base reads with 1500-2000-base haps; the strips take 1.5 ms
+// of 1100-1500-base reads with 1500-2000-base haps; the strips take 1.66 ms
 // (whole calls).  12 rows per lane waste less of the last tile than 16
 // (768-row steps instead of 1024).
 //
@@ -1698,7 +1710,21 @@ constexpr float kStripGuard = 0x1p40f;
 // One alignment on the whole wave.  win: 32 entries of LDS; border: the
 // block's border row.  Returns 1 when the sum fell below the rescue threshold
 // and was finished by the scaling.
-template <bool FAST>
+//
+// Long sums have to be as good as the FP64 recompute that took them before
+// there were strips, which FP32 rounding spoils in two ways that grow with the
+// read's length; both are kept out.  A row's alpha and match emission are off by
+// up to 2^-25, by the same amount in every row of like qualities (1,300 rows of
+// indel quality 40: 1.5e-5 in log10).  A path is in a match in all but a few
+// rows, so the rows' rounding errors, summed (TileRead::drift), correct the
+// score.  And the FAST form adds what gaps contribute, less than half an ulp
+// per row, to a value that no multiplication has rounded since, where it is
+// lost every time (4e-6 low); the SAFE form's product with alpha keeps it in
+// the mean.  Scores of 1,100-1,500-base reads against 64 bits, rms in log10,
+// below the FP32 range and above it: FP64 and the one-wave kernel 4.63e-6 and
+// 1.55e-5, FAST 1.29e-5 and 1.25e-5, FAST corrected 6.35e-6 and 3.55e-6, SAFE
+// corrected 4.67e-6 (a float's rounding) and 1.39e-6.  FAST would be 9%
+// faster.
 __device__ __forceinline__ int strip_task(const FwdParams& p, float4* tab, float4* win,
                                           float4* border, const WorkItem& it)
 {
@@ -1725,14 +1751,15 @@ __device__ __forceinline__ int strip_task(const FwdParams& p, float4* tab, float
     const float4* seen = win + (first ? 0 : 16);
 
     TileRead<float, NR, false> R;
-    float acc = 0.f, C0 = 0.f;
+    float acc = 0.f, drift = 0.f;
+    const float C0 = kScale / (float)HL;
     int E = 0;
     bool bad = false;
     for (int k = 0; k < ntiles; ++k) {
         const int row0 = k * TR;
         const bool top = k == 0, last = k == ntiles - 1;
-        tile_setup<float, NR, FAST, false, NL>(p, tab, true, it.read, t, R, row0);
-        C0 = FAST ? (kScale / (float)HL) * (R.nl * (1.0f / kFastKappa)) : kScale / (float)HL;
+        tile_setup<float, NR, false, false, NL>(p, tab, true, it.read, t, R, row0);
+        drift += R.drift;
         // exponents: the insertion floor of the lane's last row, none for the
         // read's first lane
         int x = 0;
@@ -1808,7 +1835,7 @@ __device__ __forceinline__ int strip_task(const FwdParams& p, float4* tab, float
                     TT::unpack(lam[cur][q], lv);
 #pragma unroll
                     for (int x4 = 0; x4 < 4; ++x4)
-                        tile_cell<float, NR, FAST, false>(R, 4 * q + x4, lv[x4], R.eps,
+                        tile_cell<float, NR, false, false>(R, 4 * q + x4, lv[x4], R.eps,
                                                           MD[4 * q + x4], up, chain);
                 }
                 if (bounded)
@@ -1879,15 +1906,19 @@ __device__ __forceinline__ int strip_task(const FwdParams& p, float4* tab, float
         __syncthreads();  // the border row is visible to the next tile
     }
     const bool ok = __ballot(bad) == 0;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+        drift += __shfl_xor(drift, o, 64);
     bool done = false;
     if (t == (L - (ntiles - 1) * TR) / NR) {
         if (ok && acc >= 0x1p-100f && acc <= 3.4028234663852886e38f) {
             // acc * 2^-E in the start constant's units
             int e2 = 0;
             const double m = (double)frexpf(acc, &e2);
-            bd.scores[it.out] = (float)(log10(FAST ? m * (double)kFastKappa : m / (double)R.beta) +
-                                        (double)(e2 - E) * 0.30102999566398119521 - kLog10ScaleD);
-            done = !(ldexpf(FAST ? acc * R.nl : acc / R.beta, -E) >= p.rescue_min);
+            bd.scores[it.out] =
+                (float)(log10(m / (double)R.beta) + (double)drift * 0.43429448190325182765 +
+                        (double)(e2 - E) * 0.30102999566398119521 - kLog10ScaleD);
+            done = !(ldexpf(acc / R.beta, -E) >= p.rescue_min);
         } else {
             bd.scores[it.out] = -INFINITY;
             p.final_items[atomicAdd(p.final_count, 1)] = it;
@@ -1913,16 +1944,13 @@ __device__ __forceinline__ int wild_run(int nw)
 // items' runs.
 __device__ __forceinline__ int special_task(const FwdParams& p, float4* tab, float4* border,
                                             const WorkItem* strips, int nm, const WorkItem* wilds,
-                                            int nw, int run, int strip_bin, int task)
+                                            int nw, int run, int task)
 {
     const BatchDesc& bd = *p.bd;
     if (task < nm) {
         const WorkItem it = strips[task];
         float4* win = tab + TabShape<float, kStripRows, 5>::kWords;
-        const ReadMeta m = p.meta[it.read];
-        const bool fast = m.bin == strip_bin ? m.nl > 0.f : (m.bin & 1) == 0;
-        return fast ? strip_task<true>(p, tab, win, border, it)
-                    : strip_task<false>(p, tab, win, border, it);
+        return strip_task(p, tab, win, border, it);
     }
     int i = (task - nm) * run;
     const int end = min(i + run, nw);
@@ -1970,7 +1998,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
     int done = 0;
     for (int task = next_task(ss.next_task, total, blocks, true); task < total;
          task = next_task(ss.next_task, total, blocks, false))
-        done += special_task(p, tab, border, strips, nm, wilds, nw, run, ss.strip_bin,
+        done += special_task(p, tab, border, strips, nm, wilds, nw, run,
                              __builtin_amdgcn_readfirstlane(task));
     if (done > 0 && threadIdx.x == 0)
         atomicAdd(p.scaled_total, (unsigned long long)done);
@@ -2005,7 +2033,7 @@ __device__ __forceinline__ int tiny_tasks(const FwdParams& p, const SpecialSet& 
             done += fast ? tile_super_task<float, kTinyRows, true, false, true, GE>(q, tab, st, G, 0, 0)
                          : tile_super_task<float, kTinyRows, false, false, true, GE>(q, tab, st, G, 0, 0);
         } else {
-            done += special_task(p, tab, border, tl.strips, nm, tl.wilds, nw, run, ss.strip_bin,
+            done += special_task(p, tab, border, tl.strips, nm, tl.wilds, nw, run,
                                  task - nf - ns);
         }
     }

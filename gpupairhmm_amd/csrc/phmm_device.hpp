@@ -127,8 +127,7 @@ __host__ __device__ inline int base_code_sem(uint8_t b, int semantics)
 // Per-read metadata from the read pass.
 struct __attribute__((aligned(8))) ReadMeta {
     int32_t bin;     // work-list bin; -1: empty read
-    float nl;        // product of alpha over the read (rescaled form); -1: a
-                     // read of several tiles that the rescaled form does not admit
+    float nl;        // product of alpha over the read (rescaled kernel)
 };
 
 // The per-call part of a batch: device pointers of a self-contained batch

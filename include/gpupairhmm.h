@@ -114,8 +114,10 @@ typedef struct phmm_options {
                                   pass's per-lane magnitudes (tuned table
                                   only), then FP64.  0: every such result is
                                   recomputed in FP64.  Tiles of 12, 13, 16,
-                                  19 and 20 rows per lane only; not under
-                                  PHMM_SEM_GCP. */
+                                  19 and 20 rows per lane only, and with 1
+                                  also reads of several tiles, whose scores
+                                  are then as near to 64 bits as an FP64
+                                  recompute's; not under PHMM_SEM_GCP. */
     int32_t reserved[2];
 } phmm_options;
 
