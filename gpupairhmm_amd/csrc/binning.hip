@@ -78,10 +78,12 @@ __device__ __forceinline__ int hap_pass(const BinParams& bp, const BatchDesc& b,
             uint32_t c = 0;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
-                const uint32_t code = (uint32_t)base_code_sem((uint8_t)(w >> (8 * k)), bp.semantics);
+                // (the padding's bytes, whatever they are, become base 0)
+                const uint32_t code =
+                    4 * d + k < hl ? (uint32_t)base_code_sem((uint8_t)(w >> (8 * k)), bp.semantics) : 0u;
                 c |= code << (8 * k);
-                wild = wild | ((4 * d + k < hl) & (code == 4u));
-                exotic = exotic | ((4 * d + k < hl) & (code > 4u));
+                wild = wild | (code == 4u);
+                exotic = exotic | (code > 4u);
             }
             out[d0 + d] = c;
         }
@@ -110,8 +112,8 @@ __device__ __forceinline__ int hap_pass(const BinParams& bp, const BatchDesc& b,
 // row whose max_read_len covers the read (its tile has room for one more
 // row); reads beyond the last row go to the multi-tile bin 2*ntiles.  Bin 2k
 // uses the rescaled (FAST) arithmetic when the read's coefficients keep it in
-// range, else bin 2k+1 (SAFE); under per-position gcp every row's eps enters
-// the check.  Reference CPU and per-position gcp semantics: a read holding a
+// range, else bin 2k+1 (SAFE; a multi-tile read's form is the sign of its
+// nl); under per-position gcp every row's eps enters the check.  Reference CPU and per-position gcp semantics: a read holding a
 // byte other than A/C/G/T/N goes to the exact bin 2*ntiles+1.  The slot
 // combines its lanes' verdicts and the product of alpha with row-local
 // reductions.
@@ -241,14 +243,13 @@ __device__ __forceinline__ void read_meta(const BinParams& bp, const BatchDesc& 
             m.bin = -1;
         } else if (bp.semantics != 0 && exv) {
             m.bin = 2 * bp.ntiles + 1;
-        } else if (k == bp.ntiles) {
-            m.bin = 2 * bp.ntiles;
         } else {
             bool fast = okv && bp.allow_fast != 0 && eps <= 0.5f;
             if (fast && !(nl >= 1e-30))  // the start constant must stay a normal float
                 fast = false;
-            m.nl = fast ? (float)nl : 1.0f;
-            m.bin = 2 * k + (fast ? 0 : 1);
+            const bool multi = k == bp.ntiles;
+            m.nl = fast ? (float)nl : multi ? -1.0f : 1.0f;
+            m.bin = multi ? 2 * k : 2 * k + (fast ? 0 : 1);
         }
         bp.meta[i] = m;
     }

@@ -764,8 +764,8 @@ int Engine::enqueue_fwd(const FwdParams& fp, const BinParams& bp, bool plain, hi
             return set_error(PHMM_ERANGE, "too many set launches");
         ss.next_task = bp.task_ctr + ctr++;
         ss.hmax = bp.hmax;
-        ss.border = static_cast<float4*>(cur->call_spill);
-        ss.border_entries = (int64_t)(cur->call_spill_bytes / sizeof(float4));
+        ss.border = static_cast<double2*>(cur->call_spill);
+        ss.border_entries = (int64_t)(cur->call_spill_bytes / sizeof(double2));
         ss.error_flag = bp.error_flag;
         if (n_special > 0 &&
             (rc = check(launch_fwd_special(fp, ss, plain ? std::min(waves, n_special) : waves, st),
@@ -1026,10 +1026,11 @@ int Engine::enqueue_tiny(int stages, const BinParams& bp, const FwdParams& fp, c
         return rc;
     if (stages & kStageFwd) {
         SpecialSet ss;
+        ss.strip_bin = 2 * bp.ntiles;
         ss.next_task = bp.task_ctr;
         ss.hmax = bp.hmax;
-        ss.border = static_cast<float4*>(cur->call_spill);
-        ss.border_entries = (int64_t)(cur->call_spill_bytes / sizeof(float4));
+        ss.border = static_cast<double2*>(cur->call_spill);
+        ss.border_entries = (int64_t)(cur->call_spill_bytes / sizeof(double2));
         ss.error_flag = bp.error_flag;
         if ((rc = check(launch_fwd_tiny(fp, ss, tl, waves, st), "forward kernel")))
             return rc;

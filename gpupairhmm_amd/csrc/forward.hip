@@ -182,8 +182,7 @@ struct TileRead {
     // factors (each <= 1) are left out, which can only put the estimate below
     // the true floor.  (In-pass scaling; one gap continuation per read.)
     float floor2;
-    float drift;  // strips: sum over the lane's rows of what rounding took from
-                  // the factors of a match, relative
+    double prod;  // strips: product of alpha over the lane's rows
 };
 
 // Gap continuation of the D chain of row j.
@@ -221,9 +220,7 @@ __device__ __forceinline__ T beta_of(T e)
 // c3 = eps_r beta_{r+1} / beta_r, and D chain Dh = M< + eps_r Dh<; the last
 // row's beta_{L+1} is taken as beta_L, which the epilogue divides out.
 //
-// row0: the first row of the tile (reads of several tiles).  NL 5: the strips'
-// setup, once per 768 rows, with correctly rounded quotients and the rows'
-// drift (see strip_task).
+// row0: the first row of the tile (reads of several tiles).
 template <typename T, int NR, bool FAST, bool ROWEPS, int NL = 4>
 __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTraits<T>::V* tab,
                                            bool active, int read, int t,
@@ -241,7 +238,6 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
         if (FAST)
             nl = p.meta[read].nl;
     }
-    auto div = [](T a, T b) { return NL == 5 ? a / b : qdiv(a, b); };
     T eps = (T)kEpsGpu, beta = (T)kBetaGpu;
     if (p.semantics != 0 && active && L > 0) {
         // reference CPU semantics: the read's first gcp quality; per-position
@@ -298,7 +294,7 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
         R.floor2 = (float)lrow * __log2f((float)eps);
         if (FAST && lrow > 0)
             R.floor2 += __log2f(p.ph2pr[row_iq(p.rows[roff])]) - __log2f((float)de[NR - 1]);
-        R.drift = 0.f;
+        R.prod = 1.0;
         T lm[NR], lx[NR];
         int code[NR];
 #pragma unroll
@@ -316,17 +312,13 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
             }
             code[j] = in ? row_code(w[j]) : 4;
             lm[j] = in ? (T)1 - pb[j] : (T)0;
-            lx[j] = in ? div(pb[j], (T)3) : (T)0;
-            if constexpr (NL == 5) {
-                const double da = (1.0 - ((double)delta + (double)sigma)) - (double)alpha;
-                const double dm = (1.0 - (double)pb[j]) - (double)lm[j];
-                R.drift += (in && alpha > 0 ? qdiv((float)da, alpha) : 0.f) +
-                           (in && lm[j] > 0 ? qdiv((float)dm, lm[j]) : 0.f);
-            }
+            lx[j] = in ? qdiv(pb[j], (T)3) : (T)0;
+            if constexpr (NL == 5)
+                R.prod *= in ? (double)alpha : 1.0;
             if (FAST) {
-                const T c0 = div(br * pdelta, palpha * alpha);
-                const T c1 = div(top ? br : br * psigma, alpha);
-                const T c2 = div(in ? e * pdelta : pdelta, in ? delta * palpha : palpha);
+                const T c0 = qdiv(br * pdelta, palpha * alpha);
+                const T c1 = qdiv(top ? br : br * psigma, alpha);
+                const T c2 = qdiv(in ? e * pdelta : pdelta, in ? delta * palpha : palpha);
                 R.c10[j].y = in && !top ? c0 : (T)0;
                 R.c10[j].x = in ? c1 : (T)0;
                 R.c32[j].y = in ? (top ? (T)0 : c2) : firstoob ? c2 : (T)1;
@@ -336,7 +328,7 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
                 R.c10[j].x = in ? (top ? br : br * psigma) : (T)0;
                 R.c32[j].y = in ? bn * delta : firstoob ? beta : (T)0;
                 // equal betas keep eps exactly (no rounding of bn / br)
-                R.c32[j].x = in ? (bn == br ? e : div(e * bn, br)) : (T)1;
+                R.c32[j].x = in ? (bn == br ? e : qdiv(e * bn, br)) : (T)1;
                 if constexpr (ROWEPS)
                     R.c4[j] = in ? e : (T)0;
             }
@@ -1675,25 +1667,36 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
 // ---------------------------------------------------------------------------
 // k_fwd_special
 // ---------------------------------------------------------------------------
-// What the tile bins cannot take: reads of several tiles (strips, on the
-// scaled tile sweep) and haps holding the wildcard.
+// What the tile bins cannot take: reads of several tiles (strips) and haps
+// holding the wildcard.
 //
 // Strips: one wave per alignment, the read cut into tiles of 64 lanes x
-// kStripRows rows swept one after another.  A tile's last lane writes its
-// last row's (M, D, I) and its exponent per column to a border row in global
-// memory; the next tile's first lane takes them in instead of row 0.  It
-// scales like every other lane, so the values are put on its exponent as they
-// are read, 16 columns at a time between two checks (v_ldexp: exact unless a
-// value leaves the normal range, which the checks keep it from as they do
-// from lane to lane), through an LDS window that the other lanes read zeros
-// beside.  The border row is written 64 columns behind where it is read, so
-// the tiles of a read share one.  The emission table holds the wildcard as a
-// fifth letter.  Bound by the VALU like the tile kernels.  The one-wave
-// kernel, with 1024-row tiles, an exponent check of every row per column and
-// FP64 for what falls below the FP32 range, took 23.5 ms for 2,560 alignments
-// of 1100-1500-base reads with 1500-2000-base haps; the strips take 1.66 ms
-// (whole calls).  12 rows per lane waste less of the last tile than 16
-// (768-row steps instead of 1024).
+// kStripRows rows swept one after another with the tile sweep's arithmetic.  A
+// tile's last lane writes its last row's (M, I) per column to a border row in
+// global memory; the next tile's first lane takes them in instead of row 0 and
+// forms D, a chain along the row, itself.  Sixteen columns are read at a time,
+// ahead of their use, one per lane, and broadcast from there.  The border row is
+// written 64 columns behind where it is read, so the tiles of a read share one.
+// The emission table holds the wildcard as a fifth letter.
+//
+// In FP64 from the start: a deletion's run decays within one lane, so in FP32
+// one of 80 bases is flushed whatever the lane's scale, and the long flanks on
+// either side of it then cost hundreds in log10 (a 1,200-base read against a
+// hap with 80 more bases: -86.5, and -597 in scaled FP32; up to 70 is exact).
+// Scores of long reads are mostly below the FP32 range anyway.  A lane's
+// power-of-two scale only ever raises what it holds: a score above -596 (2^94
+// above double's least value in an unscaled lane, while all that is flushed is
+// less than that value per cell) is as good as double is; below, a lane's
+// range under its largest value is 2^1274, the wave kernel's is 2^1042.
+//
+// Bound by the VALU, whose FP64 instructions take four cycles each.  2,560
+// alignments of 1100-1500-base reads with 1500-2000-base haps, whole calls: the
+// one-wave kernel, with 1024-row tiles, an exponent check of every row per
+// column in FP32 and FP64 for what falls below its range, 23.2 ms; scaled FP32
+// strips 1.5 ms; these 2.2 ms (without a scale, and the wave kernel for all
+// below -596, 1.96 ms, or 5 to 10 ms where a call has such scores).  8 rows per
+// lane keep the emission table at 20 KiB, eight blocks per CU, and waste less
+// of a read's last tile than 10.
 //
 // Wildcard haps: the one-wave kernel's arithmetic (its 64 steps past the hap
 // included; 177 of 908k scores differ, by at most 8e-6) with as many alignments side by side on the wave as
@@ -1701,236 +1704,255 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
 // instead of compares, and the letters loaded four columns ahead.  The items
 // are sorted by (read class, hap length) and a wave takes a run of them.  908k
 // mixed alignments of which 5% have such a hap: 20.0 -> 7.2 ms per call.
-constexpr int kStripPad = 256;  // border entries beyond the longest hap
-// Long reads meet more of the steepest growths between two checks than the
-// tiles' reads do: the strips scale down from 2^40 (at 2^kDsGuard, 2 of 2,560
-// alignments overflowed and cost an FP64 pass of 3 ms).
-constexpr float kStripGuard = 0x1p40f;
+// Border entries: the longest hap's columns, four exponents each for 64 of them,
+// and kStripPad.
+constexpr int kStripPad = 256;
+// A strip's lane holds its values times 2^E, E >= 0: every 16 columns, where
+// the largest of them has left 2^kStripLow .. 2^kStripHigh, E puts it at
+// 2^kStripAim again (not below 0).  Between two checks values grow by 2^13 and
+// the gap extension per column at most (see kDsEvery), far less than what is
+// left above 2^kStripHigh.
+constexpr int kStripEvery = 16, kStripLow = 200, kStripAim = 600, kStripHigh = 700;
+constexpr int kStripSpan = 1000;  // largest |E_t - E_{t-1}|
+// The smallest sum that a strip finishes, in its lane's scale.
+constexpr double kStripMin = 0x1p-900;
 
-// One alignment on the whole wave.  win: 32 entries of LDS; border: the
-// block's border row.  Returns 1 when the sum fell below the rescue threshold
-// and was finished by the scaling.
-//
-// Long sums have to be as good as the FP64 recompute that took them before
-// there were strips, which FP32 rounding spoils in two ways that grow with the
-// read's length; both are kept out.  A row's alpha and match emission are off by
-// up to 2^-25, by the same amount in every row of like qualities (1,300 rows of
-// indel quality 40: 1.5e-5 in log10).  A path is in a match in all but a few
-// rows, so the rows' rounding errors, summed (TileRead::drift), correct the
-// score.  And the FAST form adds what gaps contribute, less than half an ulp
-// per row, to a value that no multiplication has rounded since, where it is
-// lost every time (4e-6 low); the SAFE form's product with alpha keeps it in
-// the mean.  Scores of 1,100-1,500-base reads against 64 bits, rms in log10,
-// below the FP32 range and above it: FP64 and the one-wave kernel 4.63e-6 and
-// 1.55e-5, FAST 1.29e-5 and 1.25e-5, FAST corrected 6.35e-6 and 3.55e-6, SAFE
-// corrected 4.67e-6 (a float's rounding) and 1.39e-6.  FAST would be 9%
-// faster.
-__device__ __forceinline__ int strip_task(const FwdParams& p, float4* tab, float4* win,
-                                          float4* border, const WorkItem& it)
+// Lane `src`'s value, in scalar registers.
+__device__ __forceinline__ double lane_value(double v, int src)
 {
-    using TT = TileTraits<float>;
-    constexpr int NR = kStripRows, NL = 5, TR = 64 * NR;
-    using Shape = TabShape<float, NR, NL>;
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), src),
+                            __builtin_amdgcn_readlane(__double2loint(v), src));
+}
+
+// Every lane's `v` moves one lane down; the last lane takes `top`.
+__device__ __forceinline__ double push_top(double v, double top)
+{
+    // DPP wave_shl:1, the last lane, without a source, keeps `top`
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(top), __double2loint(v), 0x130, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(top), __double2hiint(v), 0x130, 0xf, 0xf, false);
+    return __hiloint2double(hi, lo);
+}
+
+// One alignment on the whole wave; border: the block's border row, which ends
+// with lane 63's exponent for every 16 columns.  Returns 1 when the sum is below
+// the rescue threshold and finished.
+template <bool FAST>
+__device__ __forceinline__ int strip_task(const FwdParams& p, double2* tab, double2* border,
+                                           const WorkItem& it)
+{
+    using TT = TileTraits<double>;
+    constexpr int NR = kStripRows, NL = 5, TR = kStripTileRows, K = TT::K;
+    using Shape = TabShape<double, NR, NL>;
+    using S = WaveScalar<double>;
     constexpr int NV = Shape::NV;
-    static_assert(!Shape::kTail && NR % 4 == 0, "whole vectors");
+    static_assert(!Shape::kTail && NR % K == 0, "whole vectors");
     const BatchDesc& bd = *p.bd;
     const int t = threadIdx.x;
     const bool first = t == 0;
+    const double f = first ? 1.0 : 0.0;  // what enters from above, in the first lane only
     const int L = bd.read_len[it.read], HL = bd.hap_len[it.hap];
     const int ntiles = (L + TR) / TR;  // tiles of the read's rows and one more
     const uint32_t* hdw = reinterpret_cast<const uint32_t*>(p.hapc + bd.hap_off[it.hap]);
     const int hdw_last = HL >> 2;
     const uint32_t shift = (uint32_t)(-t) & 3u;
-    // letters past the hap read as base 0 (the wildcard, which every row
-    // matches, would let values grow there and scale the lanes down)
-    auto hap_dword = [&](int q) { return q > hdw_last ? 0u : hdw[max(q, 0)]; };
-    // this lane's view of the window: the first lane's columns, zeros for
-    // the others (in entries 16 ..)
-    if (t >= 16 && t < 32)
-        win[t] = make_float4(0.f, 0.f, 0.f, 0.f);
-    const float4* seen = win + (first ? 0 : 16);
+    // (columns outside the hap take some letter of it, or the padding's base 0:
+    // nothing of theirs is used)
+    auto hap_dword = [&](int q) { return hdw[min(max(q, 0), hdw_last)]; };
+    // FAST: nl only scales the start, where its rounding does not matter
+    const double scale = FAST ? 0.5 * (double)p.meta[it.read].nl : 1.0;
+    const double C0 = kStartF64 / (double)HL * scale;
+    const float log2_c0 = (float)log2(C0);
+    int32_t* border_exp = reinterpret_cast<int32_t*>(border + HL + 128);
 
-    TileRead<float, NR, false> R;
-    float acc = 0.f, drift = 0.f;
-    const float C0 = kScale / (float)HL;
-    int E = 0;
+    TileRead<double, NR, false> R;
+    double prod = 1.0, sum = 0.0;  // sum: the result lane's, times 2^sum_E
+    int E = 0, sum_E = 0;
     bool bad = false;
     for (int k = 0; k < ntiles; ++k) {
         const int row0 = k * TR;
         const bool top = k == 0, last = k == ntiles - 1;
-        tile_setup<float, NR, false, false, NL>(p, tab, true, it.read, t, R, row0);
-        drift += R.drift;
-        // exponents: the insertion floor of the lane's last row, none for the
-        // read's first lane
-        int x = 0;
-        if (!(top && first))
-            x = ds_start(C0, R.floor2);
-        if (__ballot(!first && x - ds_above(x) > kDsSpan))
-            x = ds_span_cap(x, t);
-        E = x;
-        auto factor = [&]() {
-            const int d = E - ds_above(E);
-            return first ? 0.f : ldexpf(1.0f, d);
-        };
-        float nf = factor();
-        bool any = __ballot(E > 0) != 0;
-
-        // border columns c0 .. c0+15 (lanes 0-15), raw and on the first
-        // lane's exponent; row 0 has D = C0 in every column
+        tile_setup<double, NR, FAST, false, NL>(p, tab, true, it.read, t, R, row0);
+        prod *= R.prod;
+        // border columns c0 .. c0+15 in lanes 0-15; row 0 has D = C0 in every
+        // column, and column HL still carries the chain of the last one (a
+        // row's chain runs one column behind)
         auto fetch = [&](int c0) {
-            return top || t >= 16 ? make_float4(0.f, C0, 0.f, 0.f) : border[64 + c0 + t];
+            const int c = c0 + t;
+            return top || t >= 16 || c > HL ? make_double2(0.0, 0.0) : border[64 + c];
         };
-        auto scaled = [&](const float4& r, int c) {
-            if (top)
-                return r;
-            const int sh = __builtin_amdgcn_readfirstlane(E) - __float_as_int(r.w);
-            // column HL still carries the chain of the last one (a row's chain
-            // runs one column behind); past it nothing was written
-            const bool in = c <= HL;
-            return make_float4(in ? ldexpf(r.x, sh) : 0.f, in ? ldexpf(r.y, sh) : 0.f,
-                               in ? ldexpf(r.z, sh) : 0.f, 0.f);
+        const int res_t = last ? (L - row0) / NR : 63;
+        // a lane's first values are those of the insertion floor (see kDsFloor)
+        E = top && first ? 0 : max(0, kStripAim - (int)floorf(log2_c0 + R.floor2));
+        double nf;  // what the lane above is multiplied by
+        auto set_factor = [&]() {
+            const int d = E - ds_above(E);
+            bad = bad || (!first && t <= res_t && (d > kStripSpan || d < -kStripSpan));
+            nf = first ? 0.0 : ldexp(1.0, d);
         };
-        TT::P MD[NR], MDr[2];
+        set_factor();
+        // the exponent of the 16 columns up to 16 b - 48, and a fetched value on
+        // the first lane's
+        auto fetch_exp = [&](int b) { return top ? 0 : border_exp[b]; };
+        auto scaled = [&](const double2& v, int e) {
+            const int sh = __builtin_amdgcn_readfirstlane(E) - e;
+            return make_double2(ldexp(v.x, sh), ldexp(v.y, sh));
+        };
+        typename TT::P MD[NR], MDr[2];
 #pragma unroll
         for (int j = 0; j < NR; ++j)
-            MD[j] = 0.f;
+            MD[j] = 0.0;
         // before step 0 the first lane holds the row above at columns -1 (row
         // 0 only) and 0
-        const float4 raw0 = fetch(0);
-        const float4 b0 = scaled(raw0, t);
-        MDr[0].x = 0.f;
-        MDr[0].y = first && top ? C0 : 0.f;
-        MDr[1].x = first ? b0.x : 0.f;
-        MDr[1].y = first ? b0.y : 0.f;
-        float Iin = first ? b0.z : 0.f;
-        float4 raw = fetch(1);
-        acc = 0.f;
-        const int res_t = last ? (L - row0) / NR : 63;
+        const double2 b0 = scaled(fetch(0), fetch_exp(3));
+        const double eb = top ? 1.0 : R.eps;
+        double Ma = lane_value(b0.x, 0), Da = top ? C0 : 0.0;  // the row above's last M and D
+        MDr[0].x = 0.0;
+        MDr[0].y = f * Da;
+        MDr[1].x = f * Ma;
+        MDr[1].y = f * Da;
+        double Iin = f * lane_value(b0.y, 0);
+        double2 raw = fetch(1);
+        int raw_exp = fetch_exp(4);
+        double2 out = make_double2(0.0, 0.0);  // the last 16 columns of the last row, lanes 48-63
+        double acc = 0.0;
+        sum = 0.0;
+        sum_E = E;
         const int nsteps = HL + res_t + 1;
         const int acc_last = t + HL;
 
         const int q0 = (0 - t) >> 2;
         uint32_t wlo = hap_dword(q0), whi = hap_dword(q0 + 1), wnx = hap_dword(q0 + 2);
         uint32_t letters = __builtin_amdgcn_alignbyte(whi, wlo, shift);
-        float4 lam[2][NV];
+        double2 lam[2][NV];
 #pragma unroll
         for (int q = 0; q < NV; ++q)
             lam[0][q] = (tab + (((letters & 7u) << 6) | t))[q * (NL * 64)];
-        auto sweep4 = [&](int s4, int w4, bool bounded) {
+        auto sweep4 = [&](int s4, int w4, const double2& win, bool bounded) {
             const uint32_t next = __builtin_amdgcn_alignbyte(wnx, whi, shift);
+            const uint32_t wn2 = hap_dword(((s4 - t) >> 2) + 3);
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int cur = u & 1, nxt = cur ^ 1;
                 const uint32_t nletter = u < 3 ? (letters >> (8 * (u + 1))) & 7u : next & 7u;
-                const float4* trow = tab + ((nletter << 6) | t);
+                const double2* trow = tab + ((nletter << 6) | t);
 #pragma unroll
                 for (int q = 0; q < NV; ++q)
                     lam[nxt][q] = trow[q * (NL * 64)];
-                const float4 in = seen[w4 + u];  // the row above at column s + 1
+                // the row above at column s + 1
+                const double in_m = lane_value(win.x, w4 + u), in_i = lane_value(win.y, w4 + u);
+                Da = fma(eb, Da, Ma);
+                Ma = in_m;
                 TT::P up = MDr[cur];
-                float chain = Iin;
+                double chain = Iin;
 #pragma unroll
                 for (int q = 0; q < NV; ++q) {
-                    float lv[4];
+                    double lv[K];
                     TT::unpack(lam[cur][q], lv);
 #pragma unroll
-                    for (int x4 = 0; x4 < 4; ++x4)
-                        tile_cell<float, NR, false, false>(R, 4 * q + x4, lv[x4], R.eps,
-                                                          MD[4 * q + x4], up, chain);
+                    for (int x = 0; x < K; ++x)
+                        tile_cell<double, NR, FAST, false>(R, K * q + x, lv[x], R.eps, MD[K * q + x],
+                                                           up, chain);
                 }
                 if (bounded)
-                    acc += (s4 + u <= acc_last) ? chain : 0.f;
+                    acc += (s4 + u <= acc_last) ? chain : 0.0;
                 else
                     acc += chain;
-                if (!last && t == 63)  // column s - 63
-                    border[s4 + u + 1] =
-                        make_float4(MD[NR - 1].x, MD[NR - 1].y, chain, __int_as_float(E));
+                out.x = push_top(out.x, MD[NR - 1].x);
+                out.y = push_top(out.y, chain);
                 __builtin_amdgcn_s_setprio(3);  // as in tile_sweep
-                MDr[cur].x = fmaf(shr1f(MD[NR - 1].x), nf, in.x);
-                MDr[cur].y = fmaf(shr1f(MD[NR - 1].y), nf, in.y);
-                Iin = fmaf(shr1f(chain), nf, in.z);
-                TT::pin(MDr[cur]);
+                MDr[cur].x = fma(f, in_m, shr1d(MD[NR - 1].x) * nf);
+                MDr[cur].y = fma(f, Da, shr1d(MD[NR - 1].y) * nf);
+                Iin = fma(f, in_i, shr1d(chain) * nf);
                 __builtin_amdgcn_s_setprio(0);
             }
             letters = next;
             wlo = whi;
             whi = wnx;
-            wnx = hap_dword(((s4 - t) >> 2) + 3);
+            wnx = wn2;
         };
+        static_assert(kStripEvery == 16, "one window between two checks");
         for (int s0 = 0; s0 < nsteps; s0 += 16) {
             // columns s0+1 .. s0+16 for the steps below; the next 16 are
             // fetched over them
-            const float4 v = scaled(raw, s0 + 1 + t);
-            if (t < 16)
-                win[t] = v;
-            __builtin_amdgcn_wave_barrier();
+            const double2 win = scaled(raw, raw_exp);
             raw = fetch(s0 + 17);
+            raw_exp = fetch_exp((s0 >> 4) + 5);
             if (s0 + 16 <= HL + 1) {
 #pragma unroll
                 for (int w4 = 0; w4 < 16; w4 += 4)
-                    sweep4(s0 + w4, w4, false);
+                    sweep4(s0 + w4, w4, win, false);
             } else {
                 for (int w4 = 0; w4 < 16; w4 += 4)
-                    sweep4(s0 + w4, w4, true);
+                    sweep4(s0 + w4, w4, win, true);
             }
-            __builtin_amdgcn_wave_barrier();
-            if (any) {
-                const float m = fmaxf(fmaxf(fmaxf(MDr[0].x, MDr[1].x), fmaxf(MDr[0].y, MDr[1].y)), Iin);
-                x = ds_lowered(E, m, kStripGuard);
-                if (__ballot(x != E)) {
-                    if (__ballot(!first && x - ds_above(x) > kDsSpan))
-                        x = ds_span_cap(x, t);
-                    const int S = x - E;
+            if (!last && t >= 48)  // columns s0 - 63 .. s0 - 48
+                border[s0 + 1 + t - 48] = out;
+            if (!last && t == 63)
+                border_exp[s0 >> 4] = E;
+            // the sum on the larger value's scale, so that it does not hold back
+            // the lane's own
+            const int lower = min(sum_E, E);
+            sum = ldexp(sum, lower - sum_E) + ldexp(acc, lower - E);
+            sum_E = lower;
+            acc = 0.0;
+            double my = fmax(fmax(fmax(MDr[0].x, MDr[0].y), fmax(MDr[1].x, MDr[1].y)), Iin);
 #pragma unroll
-                    for (int j = 0; j < NR; ++j) {
-                        MD[j].x = ldexpf(MD[j].x, S);
-                        MD[j].y = ldexpf(MD[j].y, S);
-                    }
+            for (int j = 0; j < NR; ++j)
+                my = fmax(my, fmax(MD[j].x, MD[j].y));
+            const int e = S::expo(my);
+            int x = E;
+            if (my > 0.0 && (e < kStripLow || (e > kStripHigh && E > 0)))
+                x = max(0, E + kStripAim - e);
+            if (__ballot(x != E)) {
+                const int sh = x - E;
 #pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        MDr[u].x = ldexpf(MDr[u].x, S);
-                        MDr[u].y = ldexpf(MDr[u].y, S);
-                    }
-                    Iin = ldexpf(Iin, S);
-                    acc = ldexpf(acc, S);
-                    E = x;
-                    nf = factor();
-                    any = __ballot(E > 0) != 0;
+                for (int j = 0; j < NR; ++j) {
+                    MD[j].x = ldexp(MD[j].x, sh);
+                    MD[j].y = ldexp(MD[j].y, sh);
                 }
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    MDr[u].x = ldexp(MDr[u].x, sh);
+                    MDr[u].y = ldexp(MDr[u].y, sh);
+                }
+                Iin = ldexp(Iin, sh);
+                const int sh0 = __builtin_amdgcn_readfirstlane(sh);
+                Ma = ldexp(Ma, sh0);
+                Da = ldexp(Da, sh0);
+                E = x;
+                set_factor();
             }
         }
-        const int dl = E - ds_above(E);
-        if (t <= res_t)
-            bad = bad || (E > 0 && !(acc <= 3.4028234663852886e38f)) ||
-                  (t >= 1 && (dl > 127 || dl < -126));
         __syncthreads();  // the border row is visible to the next tile
     }
-    const bool ok = __ballot(bad) == 0;
+    double lp = FAST ? log10(prod) : 0.0;
+    if (FAST) {
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-        drift += __shfl_xor(drift, o, 64);
+        for (int o = 32; o > 0; o >>= 1)
+            lp += __shfl_xor(lp, o, 64);
+    }
+    const bool ok = __ballot(bad) == 0;
     bool done = false;
     if (t == (L - (ntiles - 1) * TR) / NR) {
-        if (ok && acc >= 0x1p-100f && acc <= 3.4028234663852886e38f) {
-            // acc * 2^-E in the start constant's units
-            int e2 = 0;
-            const double m = (double)frexpf(acc, &e2);
-            bd.scores[it.out] =
-                (float)(log10(m / (double)R.beta) + (double)drift * 0.43429448190325182765 +
-                        (double)(e2 - E) * 0.30102999566398119521 - kLog10ScaleD);
-            done = !(ldexpf(acc / R.beta, -E) >= p.rescue_min);
-        } else {
-            bd.scores[it.out] = -INFINITY;
+        const double lg = log10(sum) - (double)sum_E * 0.30102999566398119521 +
+                          (FAST ? lp - log10(scale) : -log10(R.beta)) - kLog10StartF64;
+        bd.scores[it.out] = (float)lg;
+        // gap scores too steep for the checks: the wave kernel checks every step
+        if (!(ok && sum >= kStripMin && sum < 0x1p1020))
             p.final_items[atomicAdd(p.final_count, 1)] = it;
-        }
+        else
+            done = lg < log10((double)p.rescue_min) - kLog10ScaleD;
     }
     return __ballot(done) ? 1 : 0;
 }
 
-// LDS of both: the wildcard tiles' emission table; a strip's, with its window
-// after it, is smaller.
-constexpr int kSpecialTab = TabShape<float, kWildRows, 5>::kWords;
-static_assert(TabShape<float, kStripRows, 5>::kWords + 32 <= kSpecialTab, "the window beside the table");
+// LDS of both (20 KiB, so that eight blocks share a CU): the wildcard tiles'
+// emission table or a strip's.
+union SpecialTab {
+    float4 f32[TabShape<float, kWildRows, 5>::kWords];
+    double2 f64[TabShape<double, kStripRows, 5>::kWords];
+};
+static_assert(sizeof(SpecialTab) <= 20 << 10, "eight blocks per CU");
 
 // Items per wildcard task: 12 or 24 fill whole waves for most reads (4, 6 or
 // 12 side by side); the longer run where every wave gets several, the shorter
@@ -1942,15 +1964,17 @@ __device__ __forceinline__ int wild_run(int nw)
 }
 // Task `task` of the strips (nm of them, one each) and then the wildcard
 // items' runs.
-__device__ __forceinline__ int special_task(const FwdParams& p, float4* tab, float4* border,
+__device__ __forceinline__ int special_task(const FwdParams& p, SpecialTab& tab, double2* border,
                                             const WorkItem* strips, int nm, const WorkItem* wilds,
-                                            int nw, int run, int task)
+                                            int nw, int run, int strip_bin, int task)
 {
     const BatchDesc& bd = *p.bd;
     if (task < nm) {
         const WorkItem it = strips[task];
-        float4* win = tab + TabShape<float, kStripRows, 5>::kWords;
-        return strip_task(p, tab, win, border, it);
+        const ReadMeta m = p.meta[it.read];
+        const bool fast = m.bin == strip_bin ? m.nl > 0.f : (m.bin & 1) == 0;
+        return fast ? strip_task<true>(p, tab.f64, border, it)
+                    : strip_task<false>(p, tab.f64, border, it);
     }
     int i = (task - nm) * run;
     const int end = min(i + run, nw);
@@ -1959,7 +1983,7 @@ __device__ __forceinline__ int special_task(const FwdParams& p, float4* tab, flo
         const int L = (int)threadIdx.x < n ? bd.read_len[wilds[i + threadIdx.x].read] : 0;
         const int G = (wave_max(L) + kWildRows) / kWildRows;  // ceil((L + 1) / rows)
         const int take = min(n, 64 / G);
-        pack_task<float, kWildRows>(p, tab, wilds + i, take, G);
+        pack_task<float, kWildRows>(p, tab.f32, wilds + i, take, G);
         i += take;
     }
     return 0;
@@ -1968,9 +1992,9 @@ __device__ __forceinline__ int special_task(const FwdParams& p, float4* tab, flo
 // The block's border row; returns how many of the launch's first blocks the
 // arena holds one for (the others take no task; none: the first block reports
 // it).
-__device__ __forceinline__ int border_row(const SpecialSet& ss, float4*& border)
+__device__ __forceinline__ int border_row(const SpecialSet& ss, double2*& border)
 {
-    const int64_t stride = (int64_t)*ss.hmax + kStripPad;
+    const int64_t stride = (int64_t)*ss.hmax + (*ss.hmax >> 6) + kStripPad;
     const int64_t rows = ss.border_entries / stride;
     if (rows <= 0 && blockIdx.x == 0 && threadIdx.x == 0)
         *(volatile int32_t*)ss.error_flag = 1;
@@ -1981,13 +2005,13 @@ __device__ __forceinline__ int border_row(const SpecialSet& ss, float4*& border)
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_fwd_special(
     FwdParams p, SpecialSet ss)
 {
-    __shared__ float4 tab[kSpecialTab];
+    __shared__ SpecialTab tab;
     const int nm = ss.range[2 * ss.strip_bin + 1], nw = ss.range[2 * ss.wild_bin + 1];
     if (nm + nw == 0)
         return;
     const WorkItem* strips = ss.items + ss.range[2 * ss.strip_bin];
     const WorkItem* wilds = ss.items + ss.range[2 * ss.wild_bin];
-    float4* border = nullptr;
+    double2* border = nullptr;
     const int blocks = nm > 0 ? border_row(ss, border) : (int)gridDim.x;
     if ((int)blockIdx.x >= blocks)
         return;
@@ -1998,7 +2022,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
     int done = 0;
     for (int task = next_task(ss.next_task, total, blocks, true); task < total;
          task = next_task(ss.next_task, total, blocks, false))
-        done += special_task(p, tab, border, strips, nm, wilds, nw, run,
+        done += special_task(p, tab, border, strips, nm, wilds, nw, run, ss.strip_bin,
                              __builtin_amdgcn_readfirstlane(task));
     if (done > 0 && threadIdx.x == 0)
         atomicAdd(p.scaled_total, (unsigned long long)done);
@@ -2008,7 +2032,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
 // strips and wildcard items, in that order from one counter.
 template <bool GE>
 __device__ __forceinline__ int tiny_tasks(const FwdParams& p, const SpecialSet& ss,
-                                          const TinyLists& tl, float4* tab, float4* border,
+                                          const TinyLists& tl, SpecialTab& tab, double2* border,
                                           int blocks)
 {
     const int nf = tl.counts[kTinyFast], ns = tl.counts[kTinySafe];
@@ -2030,10 +2054,10 @@ __device__ __forceinline__ int tiny_tasks(const FwdParams& p, const SpecialSet& 
             q.rescue_items = !tiles ? p.final_items : fast ? tl.rescue[0] : tl.rescue[1];
             q.rescue_counts = !tiles ? p.final_count
                                      : tl.counts + (fast ? kTinyRescueFast : kTinyRescueSafe);
-            done += fast ? tile_super_task<float, kTinyRows, true, false, true, GE>(q, tab, st, G, 0, 0)
-                         : tile_super_task<float, kTinyRows, false, false, true, GE>(q, tab, st, G, 0, 0);
+            done += fast ? tile_super_task<float, kTinyRows, true, false, true, GE>(q, tab.f32, st, G, 0, 0)
+                         : tile_super_task<float, kTinyRows, false, false, true, GE>(q, tab.f32, st, G, 0, 0);
         } else {
-            done += special_task(p, tab, border, tl.strips, nm, tl.wilds, nw, run,
+            done += special_task(p, tab, border, tl.strips, nm, tl.wilds, nw, run, ss.strip_bin,
                                  task - nf - ns);
         }
     }
@@ -2043,9 +2067,10 @@ __device__ __forceinline__ int tiny_tasks(const FwdParams& p, const SpecialSet& 
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_fwd_tiny(
     FwdParams p, SpecialSet ss, TinyLists tl)
 {
-    static_assert(TabShape<float, kTinyRows>::kWords <= kSpecialTab, "one table for all");
-    __shared__ float4 tab[kSpecialTab];
-    float4* border = nullptr;
+    static_assert(TabShape<float, kTinyRows>::kWords <= TabShape<float, kWildRows, 5>::kWords,
+                  "one table for all");
+    __shared__ SpecialTab tab;
+    double2* border = nullptr;
     const int blocks = tl.counts[kTinyStrips] > 0 ? border_row(ss, border) : (int)gridDim.x;
     if ((int)blockIdx.x >= blocks)
         return;

@@ -127,7 +127,8 @@ __host__ __device__ inline int base_code_sem(uint8_t b, int semantics)
 // Per-read metadata from the read pass.
 struct __attribute__((aligned(8))) ReadMeta {
     int32_t bin;     // work-list bin; -1: empty read
-    float nl;        // product of alpha over the read (rescaled kernel)
+    float nl;        // product of alpha over the read (rescaled form); -1: a
+                     // read of several tiles that the rescaled form does not admit
 };
 
 // The per-call part of a batch: device pointers of a self-contained batch
@@ -389,15 +390,15 @@ hipError_t launch_fwd_tile_set_scaled(int NR, bool fast, const FwdParams& p, con
 // Rows per lane of the wildcard tiles.
 constexpr int kWildRows = 16;
 // Rows per lane, and per tile, of the strips of a long read.
-constexpr int kStripRows = 12, kStripTileRows = 64 * kStripRows;
-// The multi-tile and wildcard bins on the scaled sweep (k_fwd_special).
+constexpr int kStripRows = 8, kStripTileRows = 64 * kStripRows;
+// The multi-tile and wildcard bins (k_fwd_special).
 struct SpecialSet {
     const WorkItem* items = nullptr;
     const int32_t* range = nullptr;  // bin_range
     int32_t strip_bin = 0, wild_bin = 0;
     int32_t* next_task = nullptr;
     const int32_t* hmax = nullptr;
-    float4* border = nullptr;        // border rows of the strips, one per block
+    double2* border = nullptr;       // border rows of the strips, one per block
     int64_t border_entries = 0;
     int32_t* error_flag = nullptr;
 };

@@ -114,10 +114,9 @@ typedef struct phmm_options {
                                   pass's per-lane magnitudes (tuned table
                                   only), then FP64.  0: every such result is
                                   recomputed in FP64.  Tiles of 12, 13, 16,
-                                  19 and 20 rows per lane only, and with 1
-                                  also reads of several tiles, whose scores
-                                  are then as near to 64 bits as an FP64
-                                  recompute's; not under PHMM_SEM_GCP. */
+                                  19 and 20 rows per lane only (with 1,
+                                  reads of several tiles are in FP64 from
+                                  the start); not under PHMM_SEM_GCP. */
     int32_t reserved[2];
 } phmm_options;
 
@@ -177,7 +176,8 @@ typedef struct phmm_stats {
                                   in FP64 */
     int64_t scaled_alignments; /* alignments whose FP32 sum fell below
                                   rescue_min_sum and that the FP32 pass
-                                  finished with per-lane scaling
+                                  finished with per-lane scaling, or in FP64
+                                  where it takes reads of several tiles
                                   (range_rescue 1); not in `rescued` */
     int64_t reserved[3];
 } phmm_stats;

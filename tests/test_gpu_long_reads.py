@@ -64,3 +64,93 @@ def test_precision(lib, oracle, semantics, ins):
             assert abs(d[part].mean()) <= DRIFT
         half = 0.5 * np.spacing(np.abs(ref).astype(np.float32)).astype(np.float64)
         assert np.all(np.abs(d) <= half + PATH + DRIFT)
+
+
+def _line(s, q, gap, gcp):
+    L = len(s)
+    gap = np.broadcast_to(gap, L)
+    return " ".join([s, _phred(np.full(L, q)), _phred(gap), _phred(gap), _phred(np.full(L, gcp))])
+
+
+def _check(lib, oracle, text, semantics):
+    import gpupairhmm_amd as G
+    b = G.HostBatch.parse(text)
+    ref = oracle.score_batch(b.oracle_arrays(), oracle.F64, semantics=semantics)
+    for kw in ({}, {"small_batch": 0}, {"mode": G.MODE_PLAIN}):
+        with G.Engine(semantics=semantics, **kw) as e:
+            d = np.abs(e.score_batch(b).astype(np.float64) - ref)
+        assert np.all(np.isfinite(d))
+        # the parity bar, and a float's own step for scores in the thousands
+        assert np.all(d <= 1e-3 + np.spacing(np.abs(ref).astype(np.float32))), (kw, ref[d > 1e-3])
+    return ref
+
+
+@pytest.mark.parametrize("semantics", [0, 1])
+@pytest.mark.parametrize("L", [1024, 1031, 1032, 1200, 1535, 1536, 1537, 2047, 2048])
+def test_long_gaps(lib, oracle, L, semantics):
+    """A deletion or insertion of up to 400 bases between long flanks, whose run
+    leaves the FP32 range within one row or column: by far the likeliest path
+    all the same.  Lengths at the edges of tiles and lanes."""
+    rng = np.random.default_rng(L)
+    text = ""
+    for k in (30, 75, 80, 100, 200, 400):
+        ref, m = _seq(rng, L + 30), L // 2 + int(rng.integers(-200, 200))
+        reads = [_line(ref[:L], 30, 40, 10),
+                 _line((ref[:m] + _seq(rng, k) + ref[m:])[:L], 30, 40, 10),
+                 _line(ref[:L], 20, rng.integers(25, 46, L), 12)]
+        text += "\n".join([f"{len(reads)} 2"] + reads + [ref, ref[:m] + _seq(rng, k) + ref[m:]]) + "\n"
+    say(f"case: long gaps, reads of {L}, semantics {semantics}")
+    _check(lib, oracle, text, semantics)
+
+
+@pytest.mark.parametrize("gcp", [6, 10, 25, 40, pytest.param(60, marks=pytest.mark.xfail(
+    strict=True, reason="the FP64 wave kernel, which takes what the strips refuse, has always "
+    "given -inf below about -3500 where hundreds of rows hang over at 6 per row"))])
+def test_scores_far_below(lib, oracle, gcp):
+    """Scores down to thousands: reads hanging over either end of their hap,
+    unrelated to it, or joined from two places of it in either order, so that a
+    lane's values fall and rise again by far more than any scale holds."""
+    rng = np.random.default_rng(gcp)
+    text = ""
+    for L in (1100, 1700):
+        a, b = _seq(rng, L), _seq(rng, L)
+        h = L // 2
+        reads = [_line(s, 30, g, gcp) for g in (40, 30) for s in
+                 (a, b[:h] + a[:L - h], a[h:] + a[:h], a[:h] + b[h:], _seq(rng, L))]
+        haps = [a, a[:300], a[-400:], a[:h] + _seq(rng, 900) + a[h:], a[h:] + _seq(rng, 1000) + a[:h]]
+        text += "\n".join([f"{len(reads)} {len(haps)}"] + reads + haps) + "\n"
+    say(f"case: scores far below, gap continuation quality {gcp}")
+    ref = _check(lib, oracle, text, 1)
+    assert ref.min() < -1000 and ref.max() > -60
+
+
+@pytest.mark.parametrize("semantics", [0, 1])
+def test_padding_is_not_read(lib, semantics):
+    """The bytes that pad a hap to whole dwords may be anything: one that is no
+    base has no row in the emission tables, and the scores are the same bit for
+    bit whatever stands there."""
+    import gpupairhmm_amd as G
+    rng = np.random.default_rng(71)
+    text = ""
+    for L in (60, 150, 1030, 1400):
+        ref = _seq(rng, L + 40)
+        reads = [_line(_noisy(rng, ref[o:o + L], 0.01), 30, 40, 10) for o in (0, 39)] + [
+            _line(_seq(rng, L), 20, rng.integers(25, 46, L), 10)]
+        haps = [ref[:n] for n in range(L + 37, L + 41)] + [_seq(rng, n) for n in (1, 2, 3, 62)]
+        haps += [h[:20] + "N" + h[21:] for h in haps[:4]]
+        text += "\n".join([f"{len(reads)} {len(haps)}"] + reads + haps) + "\n"
+    b = G.HostBatch.parse(text)
+    names = list(G._VIEW_ARRAYS)
+    arrays = {k: np.array(b.array(k)) for k in names}
+    within = np.zeros(len(arrays["hap_data"]), bool)
+    for o, n in zip(arrays["hap_offsets"], arrays["hap_lengths"]):
+        within[o:o + n] = True
+    say(f"case: padding bytes, semantics {semantics}")
+    want = {}
+    for pad in (ord("N"), ord("A"), ord("T"), 0, 255):
+        hap_data = np.where(within, arrays["hap_data"], np.uint8(pad))
+        bb = G.HostBatch.from_arrays(**{**arrays, "hap_data": hap_data})
+        for kw in ({}, {"small_batch": 0}, {"range_rescue": 0}):
+            with G.Engine(semantics=semantics, **kw) as e:
+                got = e.score_batch(bb).view(np.uint32)
+            assert np.array_equal(got, want.setdefault(str(kw), got)), (pad, kw)
