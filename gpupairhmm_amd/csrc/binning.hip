@@ -21,8 +21,8 @@ namespace phmm {
 // Counter arrays that k_prep zeroes (in a kernel rather than by memsets, so
 // the sequence can be captured and replayed as a graph).
 struct ClearList {
-    int32_t* p[6];
-    int32_t n[6];
+    int32_t* p[7];
+    int32_t n[7];
     int32_t count;
 };
 __device__ __forceinline__ void clear_list(const ClearList& cl, int block, int nblocks)
@@ -654,6 +654,8 @@ __global__ __launch_bounds__(64 * NW) void k_count_keys_t(BinParams bp)
                 continue;
             }
             atomicAdd(&bp.key_count[run_key_of(bp, k, flag, hl, g)], gb.cnt[e]);
+            if (run_bin_of(bp, k, flag) == 2 * bp.ntiles)
+                atomicMax(bp.strip_hmax, b.hap_len[h0 + h]);
         }
         __syncthreads();
     }
@@ -1221,6 +1223,7 @@ __global__ __launch_bounds__(256) void k_tiny_plan(BinParams bp, TinyLists tl)
             if (tid < 3)
                 item_n[tid] = 0;
             const bool plain_haps = gh.nonempty == nh && gh.wild + gh.exotic == 0;
+            int strip_h = 0;
             // two passes over the pairs, a read per wave: count, then write
             for (int pass = 0; pass < 2; ++pass) {
                 __syncthreads();
@@ -1254,6 +1257,8 @@ __global__ __launch_bounds__(256) void k_tiny_plan(BinParams bp, TinyLists tl)
                             if (lane == 0)
                                 at = atomicAdd(&item_n[l], __popcll(m));
                             at = __shfl(at, 0, 64);
+                            if (pass == 0 && l == 0 && list == 0)
+                                strip_h = max(strip_h, b.hap_len[h0 + h]);
                             if (pass == 0 || list != l)
                                 continue;
                             WorkItem it;
@@ -1267,6 +1272,11 @@ __global__ __launch_bounds__(256) void k_tiny_plan(BinParams bp, TinyLists tl)
                     }
                 }
             }
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1)
+                strip_h = max(strip_h, __shfl_xor(strip_h, o, 64));
+            if (lane == 0 && strip_h > 0)
+                atomicMax(bp.strip_hmax, strip_h);
         }
         __syncthreads();  // the next record rebuilds the tables
     }
@@ -1352,7 +1362,9 @@ hipError_t run_binning(const BinParams& bp, const BatchDesc& hd, bool fixed_grid
     cl.n[4] = kAlignParts * bp.NB;
     cl.p[5] = bp.retry_counts;
     cl.n[5] = kRetrySlots;
-    cl.count = 6;
+    cl.p[6] = bp.strip_hmax;
+    cl.n[6] = 1;
+    cl.count = 7;
     const int nclear = 64;
     const int nhap = std::min(kHmaxParts, grid(hd.nH, tpb / 64, 4096));  // one wave per hap
     const int nread = grid(hd.nR, tpb / 16, 4096);                       // 16 lanes per read

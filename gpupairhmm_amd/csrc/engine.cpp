@@ -460,7 +460,7 @@ int Engine::score_device(const phmm_batch_view& v, float* d_scores, hipStream_t 
             return rc;
     }
 
-    // counters: [0] max hap length, [1] final-list count, [2] error flag,
+    // counters: [0] max hap length, [1] final-list count, [2] the strips' max hap length,
     // [4 .. 4+NB) per-bin rescue counts, [128 .. 128+kTaskCounters) task
     // counters of the set launches, [256 .. 256+kHmaxParts) partial maxima,
     // then kRetrySlots: per-bin retry counts and (last) the exps unit counter
@@ -484,6 +484,7 @@ int Engine::score_device(const phmm_batch_view& v, float* d_scores, hipStream_t 
     bp.hmax = sm + 0;
     bp.hmax_part = sm + 256;
     bp.final_count = sm + 1;
+    bp.strip_hmax = sm + 2;
     bp.error_flag = c.h_error;
     bp.rescue_counts = sm + 4;
     bp.retry_counts = sm + 256 + kHmaxParts;
@@ -590,6 +591,7 @@ int Engine::score_device(const phmm_batch_view& v, float* d_scores, hipStream_t 
         tl.counts = bp.task_ctr + 1;
         static_assert(1 + kTinyWords <= kTaskCounters, "counters");
         fp.final_count = tl.counts + kTinyFinal;
+        bp.strip_hmax = tl.counts + kTinyStripHmax;
         if ((rc = check(launch_tiny_desc(bp, tl, hd, (int)(tl.late - fp.final_items), st), "descriptor kernel")) ||
             (rc = eager ? stages([&](int which) { return enqueue_tiny(which, bp, fp, tl, st); })
                         : graph_of(c.tiny, [&](int which, hipStream_t cs) {
@@ -763,7 +765,7 @@ int Engine::enqueue_fwd(const FwdParams& fp, const BinParams& bp, bool plain, hi
         if (ctr >= kTaskCounters - kF64Sets - kReSets)
             return set_error(PHMM_ERANGE, "too many set launches");
         ss.next_task = bp.task_ctr + ctr++;
-        ss.hmax = bp.hmax;
+        ss.hmax = bp.strip_hmax;
         ss.border = static_cast<double2*>(cur->call_spill);
         ss.border_entries = (int64_t)(cur->call_spill_bytes / sizeof(double2));
         ss.error_flag = bp.error_flag;
@@ -1028,7 +1030,7 @@ int Engine::enqueue_tiny(int stages, const BinParams& bp, const FwdParams& fp, c
         SpecialSet ss;
         ss.strip_bin = 2 * bp.ntiles;
         ss.next_task = bp.task_ctr;
-        ss.hmax = bp.hmax;
+        ss.hmax = bp.strip_hmax;
         ss.border = static_cast<double2*>(cur->call_spill);
         ss.border_entries = (int64_t)(cur->call_spill_bytes / sizeof(double2));
         ss.error_flag = bp.error_flag;

@@ -1991,7 +1991,9 @@ __device__ __forceinline__ int special_task(const FwdParams& p, SpecialTab& tab,
 
 // The block's border row; returns how many of the launch's first blocks the
 // arena holds one for (the others take no task; none: the first block reports
-// it).
+// it).  Its length is that of the longest hap that a strip meets, so that a
+// batch's other haps cost the launch no blocks: 56,000 tile alignments with one
+// long read of 1,100 bases and, elsewhere, a hap of 40,000, 8.1 -> 7.4 ms.
 __device__ __forceinline__ int border_row(const SpecialSet& ss, double2*& border)
 {
     const int64_t stride = (int64_t)*ss.hmax + (*ss.hmax >> 6) + kStripPad;

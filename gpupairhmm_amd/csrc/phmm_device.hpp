@@ -272,6 +272,7 @@ struct BinParams {
     int32_t* bin_range;        // [2*NW]: begin, count (tile bins: super-tasks; others: items)
     int32_t* hmax;             // [1]: the longest hap (k_scan_bins folds hmax_part)
     int32_t* hmax_part;        // [kHmaxParts]: per-block maxima of the hap pass
+    int32_t* strip_hmax;       // [1]: the longest hap of the strips' alignments
     int32_t* rescue_counts;    // [NB]
     int32_t* retry_counts;     // [kRetrySlots]: retry lists' counts per bin
     int32_t* final_count;      // [1]
@@ -306,6 +307,7 @@ struct TinyLists {
 enum {
     kTinyFast, kTinySafe, kTinyStrips, kTinyWilds, kTinyExact, kTinyRescueFast, kTinyRescueSafe,
     kTinyFinal, kTinyLate,  // the final list (FwdParams::final_count) and `late`
+    kTinyStripHmax,         // not a count: BinParams::strip_hmax
     kTinyCounts,
     // then the two lists' begins in BinSet's form, from final_items
     kTinyFinalRange = kTinyCounts, kTinyWords = kTinyFinalRange + 4
@@ -397,7 +399,7 @@ struct SpecialSet {
     const int32_t* range = nullptr;  // bin_range
     int32_t strip_bin = 0, wild_bin = 0;
     int32_t* next_task = nullptr;
-    const int32_t* hmax = nullptr;
+    const int32_t* hmax = nullptr;   // BinParams::strip_hmax
     double2* border = nullptr;       // border rows of the strips, one per block
     int64_t border_entries = 0;
     int32_t* error_flag = nullptr;

@@ -154,3 +154,28 @@ def test_padding_is_not_read(lib, semantics):
             with G.Engine(semantics=semantics, **kw) as e:
                 got = e.score_batch(bb).view(np.uint32)
             assert np.array_equal(got, want.setdefault(str(kw), got)), (pad, kw)
+
+
+@pytest.mark.parametrize("small_batch", [0, 1 << 18])
+def test_border_rows_are_as_long_as_the_strips_need(lib, oracle, small_batch):
+    """A hap of four million bases, which only a read of 12 meets, leaves the
+    scratch of an allocation-free call no border row of its length; the long
+    reads, against haps of 1,300, need none like that."""
+    import gpupairhmm_amd as G
+    rng = np.random.default_rng(81)
+    ref = _seq(rng, 1300)
+    long_hap = rng.choice(np.frombuffer(b"ACGT", np.uint8), 4_000_000).tobytes().decode()
+    text = "1 1\n" + _line(_seq(rng, 12), 30, 40, 10) + "\n" + long_hap + "\n"
+    reads = [_line(_noisy(rng, ref[o:o + 1100], 0.01), 30, 40, 10) for o in range(0, 200, 10)]
+    text += "\n".join([f"{len(reads)} 2"] + reads + [ref, _noisy(rng, ref, 0.02)]) + "\n"
+    b = G.HostBatch.parse(text)
+    say(f"case: border rows beside a very long hap, small_batch {small_batch}")
+    ref = oracle.score_batch(b.oracle_arrays(), oracle.F64)
+    with G.Engine(small_batch=small_batch) as e:
+        db, out = e.upload(b), e.alloc(4 * b.num_alignments)
+        e.score_device_noalloc(db, out)
+        e.synchronize()
+        got = e.download(out, b.num_alignments)
+        e.free(out)
+        db.free()
+    assert np.max(np.abs(got.astype(np.float64) - ref)) <= 1e-3
