@@ -1007,6 +1007,9 @@ bool Engine::tiny_call(const phmm_batch_view& v) const
         v.num_alignments > kTinyAlignments || v.num_groups > kTinyGroups ||
         tiny_columns(v) > kTinyColumns)
         return false;
+    // its FP64 tiles are the small-batch table's own: 10 rows per lane, SAFE 8
+    if (opt.f64_rows != 0 && opt.f64_rows != 10)
+        return false;
     // records of few reads that share a sweep leave their last chunk part empty
     if (v.num_reads < 64 * (int64_t)v.num_groups && tiny_columns(v) > kTinyColumnsFew &&
         v.read_bytes <= (int64_t)v.num_reads * 64 * kTinyRows)

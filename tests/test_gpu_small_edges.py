@@ -130,3 +130,61 @@ def test_server_launches_fit_the_reservation(lib):
             assert len(set(seen)) == 1, seen
         finally:
             srv.close()
+
+
+def _steep(rng, lens):
+    """Reads hanging over their haps under a gap continuation of 40, which the
+    in-pass scaling mostly refuses; the last one lies within its hap."""
+    recs = []
+    for L in lens:
+        ref = _seq(rng, L + 200)
+        recs.append(([ref[o:o + L] for o in (0, 30, 60, 200)],
+                     [ref[90:], ref[:max(8, L // 2)], ref[L // 3:L + 100], ref]))
+    b = _batch(rng, recs)
+    b.gcp_quals[:] = 40
+    return b
+
+
+@pytest.mark.parametrize("f64_rows", [0, 4, 6, 8, 10])
+@pytest.mark.parametrize("lens", [(20, 79, 80, 150, 511), (512, 600, 1023)])
+def test_fp64_of_small_calls(lib, oracle, lens, f64_rows):
+    """What the in-pass scaling refuses is recomputed in FP64: reads of up to
+    511 bases in tiles, of f64_rows rows per lane where the option names them,
+    the others on waves."""
+    import gpupairhmm_amd as G
+    b = _steep(np.random.default_rng(47), lens)
+    say(f"case: FP64 of small calls, reads of {lens}, f64_rows {f64_rows}")
+    ref = oracle.score_batch(b.oracle_arrays(), oracle.F64, semantics=1)
+    assert np.all(np.isfinite(ref))
+    want = None
+    for kw in ({}, {"graphs": False}):
+        with G.Engine(semantics=1, f64_rows=f64_rows, **kw) as e:
+            got = e.score_batch(b)
+            st = e.stats()
+        assert st.f64_alignments >= len(ref) // 4
+        want = got if want is None else want
+        assert np.array_equal(_bits(got), _bits(want))
+    # the parity bar, and a float's own step for scores in the thousands
+    assert np.all(np.abs(got.astype(np.float64) - ref) <= TOL + np.spacing(np.abs(ref).astype(np.float32)))
+
+
+# hap columns per wave at 256 compute units, as the few-launch sequence of small
+# calls reckons them: on either side of its limits for records of few reads and
+# of many, and of the number at which its hap segments shrink
+@pytest.mark.parametrize("reads,haps,hap_len,columns", [
+    (25, 4, 250, (1560, 1640)), (64, 30, 300, (1900, 2200)), (64, 30, 300, (4050, 4140))])
+def test_column_limits(lib, reads, haps, hap_len, columns):
+    import gpupairhmm_amd as G
+    rng = np.random.default_rng(53)
+    hap = [_seq(rng, hap_len) for _ in range(haps)]
+    read = [hap[0][o:o + 147] for o in rng.integers(0, hap_len - 147, reads)]
+    per_record = reads * haps * (hap_len + 4 - hap_len % 4) / 6 / 2048  # six reads side by side
+    counts = [int(c / per_record) + 1 for c in columns]
+    for n in counts:
+        b = _batch(rng, [(read, hap)] * n)
+        say(f"case: {n} records of {reads} x {haps}, {n * per_record:.0f} columns per wave")
+        with G.Engine(mode=G.MODE_PLAIN) as e:
+            want = e.score_batch(b)
+        with G.Engine() as e:
+            got = e.score_batch(b)
+        assert np.all(np.isfinite(want)) and np.array_equal(_bits(got), _bits(want))
