@@ -1196,8 +1196,7 @@ struct WaveScalar<double> {
 // read) side by side on the wave, G lanes each.  What differs is how the
 // emission values are found: in an LDS table of five letters (as
 // tile_setup's), with the letters loaded four columns ahead, where k_fwd_wave
-// compares codes.  It runs k_fwd_wave's 64 steps past the hap as well: the
-// lanes rescale over them, and with them the sum.
+// compares codes.
 template <typename T, int NR>
 __device__ __forceinline__ void pack_task(const FwdParams& p, typename TileTraits<T>::V* tab,
                                           const WorkItem* items, int take, int G)
@@ -1318,8 +1317,7 @@ __device__ __forceinline__ void pack_task(const FwdParams& p, typename TileTrait
         for (int q = 0; q < NV; ++q)
             lam[q] = trow[q * (NL * 64)];
     };
-    const int nsteps = wave_max(active ? HL + 64 : 0);
-    const int s_end = HL + 63;  // the last step of this alignment
+    const int nsteps = wave_max(active ? HL + tr + 1 : 0);
     V lam[2][NV];
     uint32_t letters = __builtin_amdgcn_alignbyte(whi, wlo, shift);
     emission(-t, letters, lam[0]);
@@ -1350,6 +1348,10 @@ __device__ __forceinline__ void pack_task(const FwdParams& p, typename TileTrait
             }
             if (t == tr && c >= 1 && c <= HL)
                 acc += chain;
+            if (c == HL) {  // the sum is complete: see k_fwd_wave
+                acc_end = acc;
+                sc_end = sc;
+            }
             const T sM = S::shr(M[NR - 1]), sD = S::shr(D[NR - 1]), sI = S::shr(chain);
             const int ssc = shr1i(sc);
             int e_in = kNone;
@@ -1366,10 +1368,6 @@ __device__ __forceinline__ void pack_task(const FwdParams& p, typename TileTrait
             Ml = t == 0 ? (T)0 : S::ldexp(sM, d);
             Dl = t == 0 ? C0s : S::ldexp(sD, d);
             Iin = t == 0 ? (T)0 : S::ldexp(sI, d);
-            if (s == s_end) {
-                acc_end = acc;
-                sc_end = sc;
-            }
         }
         letters = next;
     }
@@ -1393,7 +1391,11 @@ __device__ __forceinline__ void pack_task(const FwdParams& p, typename TileTrait
 // lower tile, from the spilled border row) it compares their exponent, in
 // its own scale, with its own largest value and rescales itself when the
 // larger of the two leaves [2^-32, 2^96]; so nothing it receives can
-// overflow or vanish, and the result is finite however low the score.
+// overflow or vanish, and the result is finite however low the score.  The sum
+// is taken at the hap's last column: past it every letter matches, so that the
+// values of a read hanging over the hap grow, and with the sum scaled down
+// beside them its bits were flushed (scores between -75 and -65 off by up to
+// 0.24).
 // T = float (multi-tile first pass) appends results below the rescue
 // threshold (as the tile kernels define it) to the final list, which the
 // T = double instance recomputes.
@@ -1495,8 +1497,8 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
         // (reference CPU semantics, gpuworker.cuh:1063) -- exact for any byte.
         const bool raw = p.semantics != 0;
         const int wild = raw ? (int)'N' : 4;
-        T acc = 0;
-        int sc = 0;
+        T acc = 0, acc_end = 0;
+        int sc = 0, sc_end = 0;
         for (int k = 0; k < ntiles; ++k) {
             const int r0 = k * TR + lane * NR;
             T ca[NR], cb[NR], cdl[NR], cs[NR], ce[NR], lm[NR], lx[NR];
@@ -1547,7 +1549,7 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
             T Ml = 0, Dl = (lane == 0 && top) ? C0 : (T)0, Mul = 0, Dul = Dl, Iin = 0;
             const bool last_tile = (k == ntiles - 1);
             const int tr = last_tile ? (L - k * TR) / NR : -1;
-            const int nsteps = HL + 64;
+            const int nsteps = HL + (last_tile ? tr : 63) + 1;
             auto rescale = [&](int kk) {
 #pragma unroll
                 for (int j = 0; j < NR; ++j) {
@@ -1614,6 +1616,10 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
                 }
                 if (lane == tr && c >= 1 && c <= HL)
                     acc += chain;
+                if (c == HL) {
+                    acc_end = acc;
+                    sc_end = sc;
+                }
                 if (!last_tile && lane == 63) {
                     if (c >= 0 && c < HL) {
                         sp[3 * c + 0] = M[NR - 1];
@@ -1647,16 +1653,16 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
             }
             __syncthreads();  // spilled row visible to the next tile
         }
-        // the result lane of the last tile owns acc
+        // the result lane of the last tile owns the sum
         const int tr = (L - (ntiles - 1) * TR) / NR;
         if (lane == tr) {
-            const double lg = log10((double)acc) + (double)sc * 0.30102999566398119521 -
+            const double lg = log10((double)acc_end) + (double)sc_end * 0.30102999566398119521 -
                               log10((double)C0 * (double)HL);
             bd.scores[it.out] = (float)lg;
             // same criterion as the tile kernels: the sum in the reference's
             // units (start FLT_MAX/16/H) below rescue_min, or not finite
             const double lmin = log10((double)p.rescue_min) - (double)kLog10Scale;
-            if (sizeof(T) == 4 && p.rescue_on && !(acc > (T)0 && lg >= lmin && lg < 1e30)) {
+            if (sizeof(T) == 4 && p.rescue_on && !(acc_end > (T)0 && lg >= lmin && lg < 1e30)) {
                 const int q = atomicAdd(p.final_count, 1);
                 p.final_items[q] = it;
             }
@@ -1698,12 +1704,12 @@ __global__ __launch_bounds__(64) void k_fwd_wave(FwdParams p, BinSet bs, const i
 // lane keep the emission table at 20 KiB, eight blocks per CU, and waste less
 // of a read's last tile than 10.
 //
-// Wildcard haps: the one-wave kernel's arithmetic (its 64 steps past the hap
-// included; 177 of 908k scores differ, by at most 8e-6) with as many alignments side by side on the wave as
-// its lanes hold, the emission values from an LDS table of five letters
-// instead of compares, and the letters loaded four columns ahead.  The items
-// are sorted by (read class, hap length) and a wave takes a run of them.  908k
-// mixed alignments of which 5% have such a hap: 20.0 -> 7.2 ms per call.
+// Wildcard haps: the one-wave kernel's arithmetic with as many alignments side
+// by side on the wave as its lanes hold, the emission values from an LDS table
+// of five letters instead of compares, and the letters loaded four columns
+// ahead.  The items are sorted by (read class, hap length) and a wave takes a
+// run of them.  908k mixed alignments of which 5% have such a hap: 20.0 -> 7.1
+// ms per call.
 // Border entries: the longest hap's columns, four exponents each for 64 of them,
 // and kStripPad.
 constexpr int kStripPad = 256;

@@ -103,9 +103,7 @@ def test_long_gaps(lib, oracle, L, semantics):
     _check(lib, oracle, text, semantics)
 
 
-@pytest.mark.parametrize("gcp", [6, 10, 25, 40, pytest.param(60, marks=pytest.mark.xfail(
-    strict=True, reason="the FP64 wave kernel, which takes what the strips refuse, has always "
-    "given -inf below about -3500 where hundreds of rows hang over at 6 per row"))])
+@pytest.mark.parametrize("gcp", [6, 10, 25, 40, 60])
 def test_scores_far_below(lib, oracle, gcp):
     """Scores down to thousands: reads hanging over either end of their hap,
     unrelated to it, or joined from two places of it in either order, so that a
