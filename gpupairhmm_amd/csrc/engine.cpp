@@ -762,9 +762,10 @@ int Engine::enqueue_fwd(const FwdParams& fp, const BinParams& bp, bool plain, hi
         ss.range = bp.bin_range;
         ss.strip_bin = mb;
         ss.wild_bin = wb;
-        if (ctr >= kTaskCounters - kF64Sets - kReSets)
+        if (ctr + 1 >= kTaskCounters - kF64Sets - kReSets)
             return set_error(PHMM_ERANGE, "too many set launches");
         ss.next_task = bp.task_ctr + ctr++;
+        ss.next_strip = bp.task_ctr + ctr++;
         ss.hmax = bp.strip_hmax;
         ss.border = static_cast<double2*>(cur->call_spill);
         ss.border_entries = (int64_t)(cur->call_spill_bytes / sizeof(double2));
@@ -1033,6 +1034,7 @@ int Engine::enqueue_tiny(int stages, const BinParams& bp, const FwdParams& fp, c
         SpecialSet ss;
         ss.strip_bin = 2 * bp.ntiles;
         ss.next_task = bp.task_ctr;
+        ss.next_strip = tl.counts + kTinyStripTask;
         ss.hmax = bp.strip_hmax;
         ss.border = static_cast<double2*>(cur->call_spill);
         ss.border_entries = (int64_t)(cur->call_spill_bytes / sizeof(double2));

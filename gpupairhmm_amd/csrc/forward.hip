@@ -1076,6 +1076,13 @@ __device__ __forceinline__ int set_find(const SetLane& s, int task)
 // from the front they are held back (300 records of the mixed batch: 13290 us,
 // 13100 from the counter).  `blocks`: the blocks that take tasks, the first
 // ones of the launch.
+__device__ __forceinline__ int counter_task(int32_t* ctr)
+{
+    int t = 0;
+    if (threadIdx.x == 0)
+        t = atomicAdd(ctr, 1);
+    return __shfl(t, 0, 64);
+}
 constexpr int kFrontRounds = 4, kTailRounds = 8;  // tasks per block
 __device__ __forceinline__ int next_task(int32_t* ctr, int total, int blocks, bool first)
 {
@@ -1084,10 +1091,7 @@ __device__ __forceinline__ int next_task(int32_t* ctr, int total, int blocks, bo
         return tail ? total - 1 - (int)blockIdx.x : (int)blockIdx.x;
     if (total <= blocks)
         return total;
-    int t = 0;
-    if (threadIdx.x == 0)
-        t = atomicAdd(ctr, 1);
-    t = __shfl(t, 0, 64) + (front ? blocks : 0);
+    const int t = counter_task(ctr) + (front ? blocks : 0);
     return tail && t >= total - blocks ? total : t;
 }
 
@@ -1968,38 +1972,10 @@ __device__ __forceinline__ int wild_run(int nw)
     const int per_wave = nw / (int)gridDim.x;
     return per_wave >= 72 ? 24 : per_wave >= 4 ? 12 : 4;
 }
-// Task `task` of the strips (nm of them, one each) and then the wildcard
-// items' runs.
-__device__ __forceinline__ int special_task(const FwdParams& p, SpecialTab& tab, double2* border,
-                                            const WorkItem* strips, int nm, const WorkItem* wilds,
-                                            int nw, int run, int strip_bin, int task)
-{
-    const BatchDesc& bd = *p.bd;
-    if (task < nm) {
-        const WorkItem it = strips[task];
-        const ReadMeta m = p.meta[it.read];
-        const bool fast = m.bin == strip_bin ? m.nl > 0.f : (m.bin & 1) == 0;
-        return fast ? strip_task<true>(p, tab.f64, border, it)
-                    : strip_task<false>(p, tab.f64, border, it);
-    }
-    int i = (task - nm) * run;
-    const int end = min(i + run, nw);
-    while (i < end) {  // as many of the next items as fit side by side
-        const int n = end - i;  // at most 24: one lane each
-        const int L = (int)threadIdx.x < n ? bd.read_len[wilds[i + threadIdx.x].read] : 0;
-        const int G = (wave_max(L) + kWildRows) / kWildRows;  // ceil((L + 1) / rows)
-        const int take = min(n, 64 / G);
-        pack_task<float, kWildRows>(p, tab.f32, wilds + i, take, G);
-        i += take;
-    }
-    return 0;
-}
-
 // The block's border row; returns how many of the launch's first blocks the
-// arena holds one for (the others take no task; none: the first block reports
-// it).  Its length is that of the longest hap that a strip meets, so that a
-// batch's other haps cost the launch no blocks: 56,000 tile alignments with one
-// long read of 1,100 bases and, elsewhere, a hap of 40,000, 8.1 -> 7.4 ms.
+// arena holds one for (none: the first block reports it).  Its length is that
+// of the longest hap that a strip meets, so that a batch's other haps cost the
+// strips no blocks.
 __device__ __forceinline__ int border_row(const SpecialSet& ss, double2*& border)
 {
     const int64_t stride = (int64_t)*ss.hmax + (*ss.hmax >> 6) + kStripPad;
@@ -2008,6 +1984,51 @@ __device__ __forceinline__ int border_row(const SpecialSet& ss, double2*& border
         *(volatile int32_t*)ss.error_flag = 1;
     border = ss.border + blockIdx.x * stride;
     return (int)(rows < (int64_t)gridDim.x ? rows : (int64_t)gridDim.x);
+}
+// A launch's strips (nm > 0), one each per task, on the blocks that have a
+// border row.  They come before the launch's other tasks: a strip takes longest,
+// and the blocks without a border row start on the others at once.  (57,600
+// alignments of 150-base reads with 4 and with 300 of 1,100 bases, where the
+// others came first and on the blocks with a border row only: 1167 -> 860 and
+// 1298 -> 983 us.)
+__device__ __forceinline__ int strip_tasks(const FwdParams& p, const SpecialSet& ss, SpecialTab& tab,
+                                           const WorkItem* strips, int nm)
+{
+    double2* border = nullptr;
+    const int blocks = border_row(ss, border);
+    if ((int)blockIdx.x >= blocks)
+        return 0;
+    int done = 0;
+    for (int task = next_task(ss.next_strip, nm, blocks, true); task < nm;
+         task = next_task(ss.next_strip, nm, blocks, false)) {
+        const WorkItem it = strips[__builtin_amdgcn_readfirstlane(task)];
+        const ReadMeta m = p.meta[it.read];
+        const bool fast = m.bin == ss.strip_bin ? m.nl > 0.f : (m.bin & 1) == 0;
+        done += fast ? strip_task<true>(p, tab.f64, border, it)
+                     : strip_task<false>(p, tab.f64, border, it);
+    }
+    return done;
+}
+// The next of the launch's other tasks.  Where there are strips, no block has
+// one of its own, which a strip would hold back.
+__device__ __forceinline__ int next_other(const SpecialSet& ss, int total, bool strips, bool first)
+{
+    return strips ? counter_task(ss.next_task) : next_task(ss.next_task, total, gridDim.x, first);
+}
+// Run `q` of the wildcard items.
+__device__ __forceinline__ void wild_task(const FwdParams& p, SpecialTab& tab, const WorkItem* wilds,
+                                          int nw, int run, int q)
+{
+    int i = q * run;
+    const int end = min(i + run, nw);
+    while (i < end) {  // as many of the next items as fit side by side
+        const int n = end - i;  // at most 24: one lane each
+        const int L = (int)threadIdx.x < n ? p.bd->read_len[wilds[i + threadIdx.x].read] : 0;
+        const int G = (wave_max(L) + kWildRows) / kWildRows;  // ceil((L + 1) / rows)
+        const int take = min(n, 64 / G);
+        pack_task<float, kWildRows>(p, tab.f32, wilds + i, take, G);
+        i += take;
+    }
 }
 
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void k_fwd_special(
@@ -2019,37 +2040,30 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
         return;
     const WorkItem* strips = ss.items + ss.range[2 * ss.strip_bin];
     const WorkItem* wilds = ss.items + ss.range[2 * ss.wild_bin];
-    double2* border = nullptr;
-    const int blocks = nm > 0 ? border_row(ss, border) : (int)gridDim.x;
-    if ((int)blockIdx.x >= blocks)
-        return;
     const BatchDesc bd = *p.bd;
     p.bd = &bd;
+    const int done = nm > 0 ? strip_tasks(p, ss, tab, strips, nm) : 0;
     const int run = wild_run(nw);
-    const int total = nm + (nw + run - 1) / run;
-    int done = 0;
-    for (int task = next_task(ss.next_task, total, blocks, true); task < total;
-         task = next_task(ss.next_task, total, blocks, false))
-        done += special_task(p, tab, border, strips, nm, wilds, nw, run, ss.strip_bin,
-                             __builtin_amdgcn_readfirstlane(task));
+    const int total = (nw + run - 1) / run;
+    for (int task = next_other(ss, total, nm > 0, true); task < total;
+         task = next_other(ss, total, nm > 0, false))
+        wild_task(p, tab, wilds, nw, run, __builtin_amdgcn_readfirstlane(task));
     if (done > 0 && threadIdx.x == 0)
         atomicAdd(p.scaled_total, (unsigned long long)done);
 }
 
-// The FP32 pass of a small call in one launch: FAST super-tasks, SAFE ones,
-// strips and wildcard items, in that order from one counter.
+// The FP32 pass of a small call in one launch: the strips, then FAST
+// super-tasks, SAFE ones and wildcard items, in that order from one counter.
 template <bool GE>
 __device__ __forceinline__ int tiny_tasks(const FwdParams& p, const SpecialSet& ss,
-                                          const TinyLists& tl, SpecialTab& tab, double2* border,
-                                          int blocks)
+                                          const TinyLists& tl, SpecialTab& tab, bool strips)
 {
-    const int nf = tl.counts[kTinyFast], ns = tl.counts[kTinySafe];
-    const int nm = tl.counts[kTinyStrips], nw = tl.counts[kTinyWilds];
+    const int nf = tl.counts[kTinyFast], ns = tl.counts[kTinySafe], nw = tl.counts[kTinyWilds];
     const int run = wild_run(nw);
-    const int total = nf + ns + nm + (nw + run - 1) / run;
+    const int total = nf + ns + (nw + run - 1) / run;
     int done = 0;
-    for (int task = next_task(ss.next_task, total, blocks, true); task < total;
-         task = next_task(ss.next_task, total, blocks, false)) {
+    for (int task = next_other(ss, total, strips, true); task < total;
+         task = next_other(ss, total, strips, false)) {
         task = __builtin_amdgcn_readfirstlane(task);
         if (task < nf + ns) {
             const bool fast = task < nf;
@@ -2065,8 +2079,7 @@ __device__ __forceinline__ int tiny_tasks(const FwdParams& p, const SpecialSet& 
             done += fast ? tile_super_task<float, kTinyRows, true, false, true, GE>(q, tab.f32, st, G, 0, 0)
                          : tile_super_task<float, kTinyRows, false, false, true, GE>(q, tab.f32, st, G, 0, 0);
         } else {
-            done += special_task(p, tab, border, tl.strips, nm, tl.wilds, nw, run, ss.strip_bin,
-                                 task - nf - ns);
+            wild_task(p, tab, tl.wilds, nw, run, task - nf - ns);
         }
     }
     return done;
@@ -2078,14 +2091,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) void
     static_assert(TabShape<float, kTinyRows>::kWords <= TabShape<float, kWildRows, 5>::kWords,
                   "one table for all");
     __shared__ SpecialTab tab;
-    double2* border = nullptr;
-    const int blocks = tl.counts[kTinyStrips] > 0 ? border_row(ss, border) : (int)gridDim.x;
-    if ((int)blockIdx.x >= blocks)
-        return;
     const BatchDesc bd = *p.bd;
     p.bd = &bd;
-    const int done = p.semantics == 0 ? tiny_tasks<true>(p, ss, tl, tab, border, blocks)
-                                      : tiny_tasks<false>(p, ss, tl, tab, border, blocks);
+    const int nm = tl.counts[kTinyStrips];
+    int done = nm > 0 ? strip_tasks(p, ss, tab, tl.strips, nm) : 0;
+    done += p.semantics == 0 ? tiny_tasks<true>(p, ss, tl, tab, nm > 0)
+                             : tiny_tasks<false>(p, ss, tl, tab, nm > 0);
     if (done > 0 && threadIdx.x == 0)
         atomicAdd(p.scaled_total, (unsigned long long)done);
 }
@@ -2135,7 +2146,7 @@ hipError_t launch_rescue_tiny(const FwdParams& p, const TinyLists& tl, int grid,
 hipError_t launch_fwd_tiny(const FwdParams& p, const SpecialSet& ss, const TinyLists& tl, int grid,
                            hipStream_t st)
 {
-    if (!p.scaled_total || !p.rescue_on || !ss.next_task || !ss.hmax || !ss.border ||
+    if (!p.scaled_total || !p.rescue_on || !ss.next_task || !ss.next_strip || !ss.hmax || !ss.border ||
         !ss.error_flag || grid <= 0)
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_fwd_tiny, dim3(grid), dim3(64), 0, st, p, ss, tl);
@@ -2144,7 +2155,7 @@ hipError_t launch_fwd_tiny(const FwdParams& p, const SpecialSet& ss, const TinyL
 
 hipError_t launch_fwd_special(const FwdParams& p, const SpecialSet& ss, int grid, hipStream_t st)
 {
-    if (!p.scaled_total || !p.rescue_on || !ss.items || !ss.range || !ss.next_task || !ss.hmax ||
+    if (!p.scaled_total || !p.rescue_on || !ss.items || !ss.range || !ss.next_task || !ss.next_strip || !ss.hmax ||
         !ss.border || !ss.error_flag || grid <= 0)
         return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_fwd_special, dim3(grid), dim3(64), 0, st, p, ss);

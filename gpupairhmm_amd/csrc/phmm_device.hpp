@@ -307,7 +307,8 @@ struct TinyLists {
 enum {
     kTinyFast, kTinySafe, kTinyStrips, kTinyWilds, kTinyExact, kTinyRescueFast, kTinyRescueSafe,
     kTinyFinal, kTinyLate,  // the final list (FwdParams::final_count) and `late`
-    kTinyStripHmax,         // not a count: BinParams::strip_hmax
+    kTinyStripHmax,         // not counts: BinParams::strip_hmax,
+    kTinyStripTask,         // SpecialSet::next_strip
     kTinyCounts,
     // then the two lists' begins in BinSet's form, from final_items
     kTinyFinalRange = kTinyCounts, kTinyWords = kTinyFinalRange + 4
@@ -398,15 +399,15 @@ struct SpecialSet {
     const WorkItem* items = nullptr;
     const int32_t* range = nullptr;  // bin_range
     int32_t strip_bin = 0, wild_bin = 0;
-    int32_t* next_task = nullptr;
+    int32_t* next_strip = nullptr;   // task counters: the strips',
+    int32_t* next_task = nullptr;    // and the other tasks'
     const int32_t* hmax = nullptr;   // BinParams::strip_hmax
     double2* border = nullptr;       // border rows of the strips, one per block
     int64_t border_entries = 0;
     int32_t* error_flag = nullptr;
 };
 hipError_t launch_fwd_special(const FwdParams& p, const SpecialSet& ss, int grid, hipStream_t st);
-// The whole FP32 pass of a small call; ss: items, range and next_task unused
-// but the task counter, border row and error flag.  What the scaling refuses
+// The whole FP32 pass of a small call; ss: items and range unused.  What the scaling refuses
 // goes to the rescue lists or, past the FP64 tiles' 512 rows, the final list.
 hipError_t launch_rescue_tiny(const FwdParams& p, const TinyLists& tl, int grid, int64_t* totals,
                               hipStream_t st);

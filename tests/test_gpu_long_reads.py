@@ -177,3 +177,39 @@ def test_border_rows_are_as_long_as_the_strips_need(lib, oracle, small_batch):
         e.free(out)
         db.free()
     assert np.max(np.abs(got.astype(np.float64) - ref)) <= 1e-3
+
+
+@pytest.mark.parametrize("small_batch", [0, 1 << 18])
+def test_few_border_rows(lib, oracle, small_batch):
+    """A long read against a hap of 60,000 bases leaves border rows for 260
+    blocks; the strips share these, and the launch's other tasks, more than the
+    blocks, are every block's: each is scored once, also a second time over
+    another batch's scores."""
+    import gpupairhmm_amd as G
+    rng = np.random.default_rng(83)
+
+    def batch():
+        far = rng.choice(np.frombuffer(b"ACGT", np.uint8), 60_000).tobytes().decode()
+        text = "1 1\n" + _line(far[:500] + far[700:1300], 30, 40, 10) + "\n" + far + "\n"
+        ref = _seq(rng, 1300)
+        reads = [_line(_noisy(rng, ref[o % 200:o % 200 + 1100], 0.01), 30, 40, 10) for o in range(400)]
+        text += "\n".join([f"{len(reads)} 1"] + reads + [ref]) + "\n"
+        ref = _seq(rng, 120)
+        reads = [_line(_noisy(rng, ref[o % 60:o % 60 + 60], 0.01), 30, 40, 10) for o in range(90)]
+        haps = [ref, ref[:70], ref[:40] + "N" + ref[41:]]
+        text += ("\n".join([f"{len(reads)} {len(haps)}"] + reads + haps) + "\n") * 60
+        return G.HostBatch.parse(text)
+
+    b, other = batch(), batch()
+    say(f"case: few border rows, small_batch {small_batch}, {b.num_alignments} alignments")
+    ref = oracle.score_batch(b.oracle_arrays(), oracle.F64)
+    with G.Engine(small_batch=small_batch) as e:
+        db, odb, out = e.upload(b), e.upload(other), e.alloc(4 * b.num_alignments)
+        for x in (odb, db):
+            e.score_device(x, out)
+        e.synchronize()
+        got = e.download(out, b.num_alignments)
+        e.free(out)
+        db.free()
+        odb.free()
+    assert np.max(np.abs(got.astype(np.float64) - ref)) <= 1e-3
