@@ -437,7 +437,7 @@ struct GroupHaps {
     int nonempty, wild, exotic, nseg;
     int hs[kMaxSegs], he[kMaxSegs], work[kMaxSegs];
     int cols[64];         // staging: columns of 64 haps (0: not cut into segments)
-    int info[kMaxSegs];   // haps < kMaxSegs: length (0 if empty) | hapflag << 29
+    uint32_t info[kMaxSegs];  // haps < kMaxSegs: hap_word
 };
 // Length (<= 0: empty) and flag of record hap h, from the LDS copy where
 // group_haps made one.
@@ -445,9 +445,9 @@ __device__ __forceinline__ void hap_info(const BinParams& bp, const BatchDesc& b
                                          const GroupHaps& gh, int h0, int h, int& hl, int& flag)
 {
     if (h < kMaxSegs) {
-        const int v = gh.info[h];
-        hl = v & 0x1fffffff;
-        flag = v >> 29;
+        const uint32_t v = gh.info[h];
+        hl = hap_word_len(v);
+        flag = hap_word_flagged(v) ? bp.hapflag[h0 + h] : 0;
     } else {
         hl = b.hap_len[h0 + h];
         flag = bp.hapflag[h0 + h];
@@ -491,7 +491,7 @@ __device__ __forceinline__ void group_haps(const BinParams& bp, const BatchDesc&
             const int flag = hl > 0 ? bp.hapflag[h0 + h] : 0;
             cols = (hl > 0 && flag == 0) ? hl : 0;
             if (h < kMaxSegs)
-                gh.info[h] = (hl > 0 ? hl : 0) | flag << 29;
+                gh.info[h] = hap_word(hl, flag);
         }
         gh.cols[threadIdx.x & 63] = cols;
         __syncthreads();
@@ -1028,7 +1028,7 @@ __device__ __forceinline__ void tiny_haps(const BinParams& bp, const BatchDesc& 
     for (int h = lane; h < nh; h += 64) {
         const int hl = max(b.hap_len[h0 + h], 0), flag = bp.hapflag[h0 + h];
         if (h < kMaxSegs)
-            gh.info[h] = hl | (hl > 0 ? flag : 0) << 29;
+            gh.info[h] = hap_word(hl, flag);
         ne += hl > 0;
         wi += (hl > 0) & (flag == 1);
         ex += (hl > 0) & (flag == 2);

@@ -107,6 +107,15 @@ __host__ __device__ inline int row_bq(uint32_t w) { return (int)((w >> 8) & 0x7f
 __host__ __device__ inline int row_iq(uint32_t w) { return (int)((w >> 16) & 0x7fu); }
 __host__ __device__ inline int row_dq(uint32_t w) { return (int)((w >> 24) & 0x7fu); }
 
+// A hap's length (0: empty) and whether it holds a letter other than A/C/G/T
+// (which kind, its hapflag says) in one word: any length leaves one bit.
+__host__ __device__ inline uint32_t hap_word(int hl, int flag)
+{
+    return hl > 0 ? (uint32_t)hl | (flag ? 0x80000000u : 0u) : 0u;
+}
+__host__ __device__ inline int hap_word_len(uint32_t v) { return (int)(v & 0x7fffffffu); }
+__host__ __device__ inline bool hap_word_flagged(uint32_t v) { return (v >> 31) != 0; }
+
 // A/C/G/T -> 0..3, every other byte -> 4 (utility_kernels.cuh:16-20).
 __host__ __device__ inline int base_code(uint8_t b)
 {

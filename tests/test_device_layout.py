@@ -34,3 +34,16 @@ for (uint32_t b = 0; b < 256; ++b) {
         if (q[k] < 0 || q[k] > 127 || (b < 128 && q[k] != (int)b))
             printf("accessor %d of byte %u: %d\\n", k, b, q[k]);
 }""")
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="needs hipcc")
+def test_hap_words_hold_any_length(tmp_path):
+    """Lengths up to the largest an int32 holds, with and without a flag."""
+    _run(tmp_path, """
+const int lens[] = {-1, 0, 1, 4095, (1 << 29) - 1, 1 << 29, 1 << 30, 0x7fffffff};
+for (int hl : lens)
+    for (int flag = 0; flag < 3; ++flag) {
+        const uint32_t v = hap_word(hl, flag);
+        if (hap_word_len(v) != (hl > 0 ? hl : 0) || hap_word_flagged(v) != (hl > 0 && flag))
+            printf("length %d, flag %d\\n", hl, flag);
+    }""")
