@@ -113,10 +113,10 @@ __device__ __forceinline__ int hap_pass(const BinParams& bp, const BatchDesc& b,
 // row); reads beyond the last row go to the multi-tile bin 2*ntiles.  Bin 2k
 // uses the rescaled (FAST) arithmetic when the read's coefficients keep it in
 // range, else bin 2k+1 (SAFE; a multi-tile read's form is the sign of its
-// nl); under per-position gcp every row's eps enters the check.  Reference CPU and per-position gcp semantics: a read holding a
-// byte other than A/C/G/T/N goes to the exact bin 2*ntiles+1.  The slot
-// combines its lanes' verdicts and the product of alpha with row-local
-// reductions.
+// nl); under per-position gcp every row's eps enters the check.  Reference CPU
+// and per-position gcp semantics: a read holding a byte other than A/C/G/T/N
+// goes to the exact bin 2*ntiles+1.  The slot combines its lanes' verdicts and
+// the product of alpha with row-local reductions.
 // Block `block` of `nblocks` (256 threads).
 __device__ __forceinline__ void read_meta(const BinParams& bp, const BatchDesc& b, int block,
                                           int nblocks)

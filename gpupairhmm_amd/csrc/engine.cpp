@@ -442,17 +442,13 @@ int Engine::score_device(const phmm_batch_view& v, float* d_scores, hipStream_t 
     hd.num_alignments = nA;
     const bool plain = opt.mode == PHMM_MODE_PLAIN;
     const bool eager = plain || !opt.graphs || arena || eager_hint;
-    const int dk = c.desc_next;
-    if (!tiny) {
-        const int k = dk;
+    if (!tiny) {  // (a small call's descriptor is an argument of its first kernel)
+        const int k = c.desc_next;
         c.desc_next = (c.desc_next + 1) % kDescRing;
         if (c.desc_used[k] && (rc = check(hipEventSynchronize(c.desc_ev[k]), "descriptor slot")))
             return rc;
         c.h_desc[k] = hd;
         c.desc_used[k] = true;
-    }
-    if (!tiny) {
-        const int k = dk;
         if ((rc = check(hipMemcpyAsync(c.desc.p, &c.h_desc[k], sizeof(BatchDesc),
                                        hipMemcpyHostToDevice, st),
                         "descriptor copy")) ||
@@ -460,10 +456,11 @@ int Engine::score_device(const phmm_batch_view& v, float* d_scores, hipStream_t 
             return rc;
     }
 
-    // counters: [0] max hap length, [1] final-list count, [2] the strips' max hap length,
-    // [4 .. 4+NB) per-bin rescue counts, [128 .. 128+kTaskCounters) task
-    // counters of the set launches, [256 .. 256+kHmaxParts) partial maxima,
-    // then kRetrySlots: per-bin retry counts and (last) the exps unit counter
+    // counters: [0] max hap length, [1] final-list count, [2] the strips' max
+    // hap length, [4 .. 4+NB) per-bin rescue counts, [128 .. 128+kTaskCounters)
+    // task counters of the set launches, [256 .. 256+kHmaxParts) partial
+    // maxima, then kRetrySlots: per-bin retry counts and (last) the exps unit
+    // counter
     static_assert(4 + kMaxBins <= 128 && 128 + kTaskCounters <= 256 && kMaxBins < kRetrySlots,
                   "counter layout");
     int32_t* sm = static_cast<int32_t*>(c.smallints.p);
@@ -656,8 +653,9 @@ int Engine::enqueue_prep(const BinParams& bp, const BatchDesc& hd, bool fixed, h
 // Pass 1: FP32 tile kernels over the tile bins' super-tasks (results below
 // the rescue threshold go to the bin's rescue list), then the strips and
 // packed waves of the multi-tile and wildcard bins and the one-wave kernel
-// over the exact bin's items (over all three where the pass does not scale).  Batched: one persistent launch
-// per kernel template covering all of its bins, larger tiles first.  Plain:
+// over the exact bin's items (over all three where the pass does not scale).
+// Batched: one persistent launch per kernel template covering all of its
+// bins, larger tiles first.  Plain:
 // one launch per non-empty bin after the host has read the bin sizes back
 // (the reference's per-partition launches).
 int Engine::enqueue_fwd(const FwdParams& fp, const BinParams& bp, bool plain, hipStream_t st)

@@ -1095,9 +1095,6 @@ __device__ __forceinline__ int next_task(int32_t* ctr, int total, int blocks, bo
     return tail && t >= total - blocks ? total : t;
 }
 
-// Bins of one template in one persistent launch.  Waves take tasks in order
-// from a counter: consecutive tasks of a length-sorted bin have similar
-// lengths, and a wave that finishes early takes the next one.
 // Waves per SIMD a tile kernel is built for: the 12-row tiles and the
 // 13-row FAST tile fit three (at most 168 VGPRs, no spills) and issue more
 // of their dependent FMA chains per cycle that way; the larger tiles need
@@ -1112,8 +1109,10 @@ constexpr int tile_waves_per_simd()
     return (sizeof(T) == 4 && !RE && (NR == 12 || (NR == 13 && FAST))) ? 3 : DS ? 2 : 1;
 }
 
-// The tasks of one launch, taken in order from the launch's counter.
-// Returns the alignments the scaling finished below the threshold (DS).
+// Bins of one template in one persistent launch: each wave takes a task, then
+// the next one (next_task).  Consecutive tasks of a length-sorted bin have
+// similar lengths, and a wave that finishes early takes the next one.  Returns
+// the alignments the scaling finished below the threshold (DS).
 template <typename T, int NR, bool FAST, bool ROWEPS, bool RE, bool DS, bool GE>
 __device__ __forceinline__ int tile_set_tasks(const FwdParams& p, const BinSet& bs,
                                               typename TileTraits<T>::V* tab, const SetLane& sl,
@@ -1966,7 +1965,9 @@ static_assert(sizeof(SpecialTab) <= 20 << 10, "eight blocks per CU");
 
 // Items per wildcard task: 12 or 24 fill whole waves for most reads (4, 6 or
 // 12 side by side); the longer run where every wave gets several, the shorter
-// (or, for few items, 4) to spread them over the device.
+// (or, for few items, 4) to spread them over the device.  Runs of 4 / 12 / 24,
+// us per call of wildcard haps only, by items per wave: 3.8: 817 / 1294 / 2190,
+// 40: 3257 / 3014 / 3594, 132: 8951 / 8182 / 8159, 295: 18995 / 16711 / 16451.
 __device__ __forceinline__ int wild_run(int nw)
 {
     const int per_wave = nw / (int)gridDim.x;

@@ -142,7 +142,7 @@ struct __attribute__((aligned(8))) ReadMeta {
 
 // The per-call part of a batch: device pointers of a self-contained batch
 // view, the output array and the sizes.  It lives in device memory (one
-// small copy per call), so every kernel launch of a call -- and a captured
+// small copy per call, or k_tiny_desc's argument), so every kernel launch of a call -- and a captured
 // graph of them -- is independent of the batch.
 struct BatchDesc {
     const uint8_t* read_data;
@@ -416,17 +416,19 @@ struct SpecialSet {
     int32_t* error_flag = nullptr;
 };
 hipError_t launch_fwd_special(const FwdParams& p, const SpecialSet& ss, int grid, hipStream_t st);
-// The whole FP32 pass of a small call; ss: items and range unused.  What the scaling refuses
-// goes to the rescue lists or, past the FP64 tiles' 512 rows, the final list.
-hipError_t launch_rescue_tiny(const FwdParams& p, const TinyLists& tl, int grid, int64_t* totals,
-                              hipStream_t st);
+// The whole FP32 pass of a small call; ss: items and range unused.  What the
+// scaling refuses goes to the rescue lists or, past the FP64 tiles' 512 rows,
+// the final list.
 hipError_t launch_fwd_tiny(const FwdParams& p, const SpecialSet& ss, const TinyLists& tl, int grid,
                            hipStream_t st);
+// The FP64 recompute of its rescue lists; totals: as for launch_fwd_wave_f64.
+hipError_t launch_rescue_tiny(const FwdParams& p, const TinyLists& tl, int grid, int64_t* totals,
+                              hipStream_t st);
 hipError_t launch_fwd_wave_f32(const FwdParams& p, const BinSet& bs, const int32_t* hmax_ptr,
                                float* spill, int64_t spill_elems, int32_t* error_flag, int blocks,
                                hipStream_t st);
-// pack: reads that fit share waves.  totals (may be null): {rescued, of them in FP64}, to which the launch adds
-// the items of its first bin.
+// pack: reads that fit share waves.  totals (may be null): {rescued, of them in
+// FP64}, to which the launch adds the items of its first bin.
 hipError_t launch_fwd_wave_f64(const FwdParams& p, const BinSet& bs, const int32_t* hmax_ptr,
                                double* spill, int64_t spill_elems, int32_t* error_flag, int blocks,
                                hipStream_t st, bool pack, int64_t* totals = nullptr);
