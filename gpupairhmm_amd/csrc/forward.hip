@@ -387,8 +387,9 @@ __device__ __forceinline__ void tile_setup(const FwdParams& p, typename TileTrai
 // and so are its coefficients (c1, c0) and (c3, c2): with chain in M's old
 // register every FMA mixes parities.  150-base reads against 150-350-base
 // haps: 2.69 -> 2.58 cycles per VALU instruction over the 19-row kernel, 1-2%
-// of the call (the clock gives some of it back).  The last row's pair is only
-// read by the lane transfer, and pinning it cost a move.
+// of the call (the clock gives some of it back); over the 16-row kernel, 250-base
+// reads against 2-5 kb haps, no gain (0.1% fewer cycles).  The last row's pair is
+// only read by the lane transfer, and pinning it cost a move.
 template <typename T, int NR, bool FAST, bool ROWEPS>
 __device__ __forceinline__ void tile_cell(const TileRead<T, NR, ROWEPS>& R, int j, T lam, T eps,
                                           typename TileTraits<T>::P& md,

@@ -116,7 +116,13 @@ typedef struct phmm_options {
                                   recomputed in FP64.  Tiles of 12, 13, 16,
                                   19 and 20 rows per lane only (with 1,
                                   reads of several tiles are in FP64 from
-                                  the start); not under PHMM_SEM_GCP. */
+                                  the start); not under PHMM_SEM_GCP.
+                                  Limit of 1 and 2: where the likeliest path
+                                  of a read in tiles deletes about 75 bases
+                                  or more (at gap quality 10) between two
+                                  long flanks, its scores below -75 may be
+                                  those of the next likeliest path, lower by
+                                  up to half the read; 0 has no such limit. */
     int32_t reserved[2];
 } phmm_options;
 
